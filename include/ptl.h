@@ -223,8 +223,9 @@ int ptl_debug_stop_after(ptl_ctx *ctx, int stage);
  * a compile's node count (0: < 64Ki nodes, 1: < 1Mi, 2: < 8Mi, 3: larger), the
  * block size of each stage's per-node and per-word kernels ("block.preprocess",
  * "block.isn_cnt", "block.isn_gen", "block.optimize", "block.emit",
- * "block.fix_jumps": 64, 128 or 256) and the register-allocation walks' ring
- * ("walk_ring": 4 or 8 entries).  Output never depends on them.  No counterpart
+ * "block.fix_jumps": 64, 128 or 256).  "walk_ring" (4 or 8) is accepted and has no
+ * effect: the allocation walks keep their states in LDS.  Output never depends on
+ * the knobs.  No counterpart
  * in the reference.  PTL_ERR_ARG for unknown knobs, buckets or values. */
 /* With ctx NULL, ptl_tune_set / ptl_tune_get address the process-wide defaults
  * that each context (the serving workers' included) copies at creation. */

@@ -21,12 +21,13 @@
 //                iteration of the same monotone operator; it reaches the same
 //                greatest fixpoint as the reference's two-copy iteration.
 //   regalloc     k_ra_walk (functions not in lane 0 of an 8-function group:
-//                independent), k_ra_lane0 (lane-0 functions in step lockstep:
-//                they share the first 64-entry region of the reference's
-//                register_state snapshot, :1290-1354), k_ra_serial (exact
-//                in-order walk for programs where two functions name one
-//                register), then counts, scan, emit (:1422-1697), function
-//                table fix and frame words (:1714-1811).
+//                independent), k_ra_lane0_wave / k_ra_lane0 (lane-0 functions in
+//                step lockstep: they share the first 64-entry region of the
+//                reference's register_state snapshot, :1290-1354), k_ra_group
+//                (programs of one group), k_ra_serial (exact in-order walk for
+//                programs where a function names another's register), then
+//                counts, scan, emit (:1422-1697), function table fix and frame
+//                words (:1714-1811).
 //   fix_jumps    size + scan + fused move/encode/postprocess (:1853-1993, 1995-2011).
 //
 // Batches: P programs concatenated node-wise run through the same kernels.
@@ -64,10 +65,10 @@ DEV uint32_t spec_i(uint32_t ty, uint32_t o, uint32_t rt) { return ((uint32_t)c_
 DEV uint32_t size_of(uint32_t ty, uint32_t rt) { return (c_bits[spec_i(ty, 0, rt)] >> 19) & 7u; }
 
 // error flags raised by kernels (bit set in ctx->d_flags)
-// EF_XNAMED: some function names a virtual register of a word outside itself;
-// EF_XCONFLICT: such a register is also named by another function (see xref_note).
+// EF_XCONFLICT: some program has a word in none of the forms the allocation
+// walks take (ra_op); those programs are allocated by k_ra_serial.
 // EF_WAIT: the allocation lockstep gave up waiting for the concurrent walk's rows.
-enum : uint32_t { EF_OOB = 1, EF_CALLPATH = 4, EF_XNAMED = 16, EF_XCONFLICT = 32, EF_WAIT = 64 };
+enum : uint32_t { EF_OOB = 1, EF_CALLPATH = 4, EF_XCONFLICT = 32, EF_WAIT = 64 };
 
 // ------------------------------------------------------------------ helpers
 // Workgroup barrier that orders LDS only: global loads and stores stay in
@@ -358,9 +359,10 @@ struct Dev {
     uint8_t *used, *sstore, *usedi;
     // regalloc
     uint4 *w0_f4;            // per word: rd, rs1, rs2, instruction (one 16-byte load)
-    uint16_t *sym;           // per virtual register: assigned register | swapped << 8
-    uint32_t *xref;          // per virtual register named from outside its word's function: namer + 1
-    uint32_t *cflag;         // per program: a register is named by two of its functions
+    uint32_t *ops;           // per word: what the allocation walks need of it (ra_op)
+    uint16_t *sym;           // per virtual register: assigned register | swapped << 8 | (lane-0 walks) the
+                             // register it was defined in << 9
+    uint32_t *cflag;         // per program: it is allocated by k_ra_serial
     uint32_t *ra_off;
     uint32_t W1;
     uint32_t *w1_instr, *w1_rd, *w1_rs1, *w1_rs2, *w1_jt;
@@ -1476,12 +1478,86 @@ __global__ __launch_bounds__(256) void k_opt_iter(Dev d, uint32_t *changed) {
     if (cross || (!settled && threadIdx.x == 0)) *changed = 1;
 }
 
+// ---- the allocation walks' view of a word -------------------------------
+// A walk step of a function is a chain of dependent instructions, and the
+// longest function's chain bounds the stage, so everything about a word that
+// does not depend on the allocation is worked out here, for all words at once:
+// where its operands' states are (the word that defines the register, as a
+// distance back in the function), whether it takes a free register, the
+// constant register it writes otherwise.  A step then reads one 4-byte op in
+// place of the 16-byte word and its comparisons.
+//   bits 0-7, 8-15  distance of the word defining rs1 / rs2 (0: no operand
+//                   state, the register read is x0; a word that names its own
+//                   register reads the cleared state, which is the same)
+//   bits 16-21      register written when none is allocated (0: none)
+//   OP_ALLOC        rd is the word's own register, a free integer register
+//   OP_SELF         rd is the word's own register (float: always f5, see ffz_gcc)
+//   OP_FP           an OP-FP word (its swapped operands go to f5 / f6)
+//   OP_FAR1/2       rs1 / rs2 is defined more than OP_WINDOW words back: its
+//                   state is read from HBM
+//   OP_ZERO         an operand names the word's own register: its entry ends up 0
+constexpr uint32_t OP_WINDOW = 255;   // words back an operand's state is kept in LDS
+constexpr uint32_t OP_ROWS = 256;     // rows of the walks' LDS rings (a power of two above OP_WINDOW)
+constexpr uint32_t OP_CONST = 16;     // shift of the constant register
+constexpr uint32_t OP_ALLOC = 1u << 22, OP_SELF = 1u << 23, OP_FP = 1u << 24, OP_FAR1 = 1u << 25, OP_FAR2 = 1u << 26,
+                   OP_ZERO = 1u << 27;
+
+// The op of word i of the function [s, s + size).  `odd` turns true for a word
+// of another form: an operand or destination naming a word of another function
+// (isn_gen ORs a word's own virtual register into physical argument registers,
+// rv_generator_avx.cpp:676-697, :842, which for calls with many arguments can
+// name one), a later word, or a destination other than the word's own
+// register.  The walks keep a register's state with the one thread that walks
+// its function, in the order of that function's words; a program with an odd
+// word is allocated by k_ra_serial in the reference's step and group order.
+DEV uint32_t ra_op(const Dev &d, uint32_t i, uint32_t s, uint32_t rd, uint32_t rs1, uint32_t rs2, uint32_t ins,
+                   bool &odd) {
+    const bool fp = (ins & 0x7Fu) == 0x53u;
+    uint32_t op = fp ? OP_FP : 0u;
+    const uint32_t rs[2] = {rs1, rs2};
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        if ((int32_t)rs[k] <= 63) continue;
+        const uint32_t v = rs[k] - 64u;
+        if (v >= d.W0) { atomicOr(d.flags, EF_OOB); odd = true; continue; }
+        if (v < s || v > i) { odd = true; continue; }
+        const uint32_t dist = i - v;
+        if (dist == 0) op |= OP_ZERO;
+        else if (dist <= OP_WINDOW) op |= dist << (8 * k);
+        else op |= k ? OP_FAR2 : OP_FAR1;
+    }
+    if ((int32_t)rd > 63) {
+        if (rd - 64u >= d.W0) atomicOr(d.flags, EF_OOB);
+        if (rd - 64u != i) odd = true;
+        op |= fp ? OP_SELF | (37u << OP_CONST) : OP_SELF | OP_ALLOC;
+    } else if ((int32_t)rd < 0) {
+        odd = true;
+    } else {
+        op |= rd << OP_CONST;
+    }
+    return op;
+}
+
+// The used words, regalloc's view of them, and the walks' ops (one pass: the
+// word's fields are at hand).  Streaming: 17 B read, 21 B written per word.
 __global__ __launch_bounds__(256) void k_opt_final(Dev d) {
-    uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
+    const uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
+    // the function of the wave's first word, then each lane steps to its own
+    const uint64_t i0 = blockIdx.x * (uint64_t)blockDim.x + (threadIdx.x & ~63u);
+    if (i0 >= d.W0) return;
+    uint32_t f = prog_of(d.fstarts, d.F, (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)i0));
     if (i >= d.W0) return;
-    const uint32_t rd = d.w0_rd[i];
+    while (f + 1 < d.F && d.fstarts[f + 1] <= (uint32_t)i) ++f;
+    const uint32_t rd = d.w0_rd[i], rs1 = d.w0_rs1[i], rs2 = d.w0_rs2[i], ins = d.w0_instr[i];
     d.usedi[i] = (!((int32_t)rd > 63) || d.used[i]) ? 1 : 0;
-    d.w0_f4[i] = make_uint4(rd, d.w0_rs1[i], d.w0_rs2[i], d.w0_instr[i]);  // regalloc's view of the word
+    d.w0_f4[i] = make_uint4(rd, rs1, rs2, ins);  // regalloc's view of the word
+    bool odd = false;
+    const uint32_t s = d.fstarts[f];
+    // (a word outside every function is walked by none)
+    const bool in = (uint32_t)i - s < d.fsizes[f];
+    const uint32_t op = in ? ra_op(d, (uint32_t)i, s, rd, rs1, rs2, ins, odd) : 0u;
+    d.ops[i] = op;
+    if (odd) { atomicOr(d.flags, EF_XCONFLICT); d.cflag[prog_of(d.pf, d.P, f)] = 1; }
 }
 
 // ================================================================= regalloc
@@ -1519,6 +1595,7 @@ DEV RaStep ra_eval_raw(uint32_t ins, uint32_t ord, uint32_t rs1, uint32_t rs2, u
     return r;
 }
 
+// Whether v is a virtual register inside the words (one past them is flagged).
 DEV bool virt_ok(const Dev &d, uint32_t v) {
     if ((int32_t)v <= 63) return false;
     if (v - 64u >= d.W0) { atomicOr(d.flags, EF_OOB); return false; }
@@ -1532,31 +1609,8 @@ DEV RaStep ra_eval(const Dev &d, uint32_t off, uint64_t life, bool s1, bool s2) 
     return ra_eval_raw(w.w, w.x, w.y, w.z, raw1, raw2, s1, s2, life);
 }
 
-DEV bool sym_swapped(const Dev &d, uint32_t v) { return (d.sym[v] >> 8) != 0; }
+DEV bool sym_swapped(const Dev &d, uint32_t v) { return (d.sym[v] & 0x100u) != 0; }
 
-// Register allocation keeps each virtual register's state with the one thread
-// that walks the function naming it, which is exact when no register is named
-// by two functions.  isn_gen ORs a word's own virtual register into physical
-// argument registers (rv_generator_avx.cpp:676-697 for rd; operands, which
-// read such a result from a parent slot, :842), and for calls with many
-// arguments the result can name a word of another function.  Such
-// names are noted here; the host then checks that no other function names the
-// same register (k_xref_check), and reallocates every program where one does
-// in the reference's exact step and group order (k_ra_serial).
-DEV void xref_note(const Dev &d, uint32_t v, uint32_t f) {
-    const uint32_t e = v - 64u;
-    if (e >= d.W0) return;  // out of range: flagged by the caller's bounds checks
-    const uint32_t prev = atomicCAS(&d.xref[e], 0u, f + 1u);
-    if (prev != 0u && prev != f + 1u) { atomicOr(d.flags, EF_XCONFLICT); d.cflag[prog_of(d.pf, d.P, f)] = 1; }
-    atomicOr(d.flags, EF_XNAMED);
-}
-
-DEV void xref_check_fields(const Dev &d, uint32_t f, uint32_t start, uint32_t size, uint32_t ord, uint32_t rs1,
-                           uint32_t rs2) {
-    if ((int32_t)ord > 63 && ord - 64u - start >= size) xref_note(d, ord, f);
-    if ((int32_t)rs1 > 63 && rs1 - 64u - start >= size) xref_note(d, rs1, f);
-    if ((int32_t)rs2 > 63 && rs2 - 64u - start >= size) xref_note(d, rs2, f);
-}
 DEV void sym_mark(const Dev &d, uint32_t v) { reinterpret_cast<uint8_t *>(d.sym)[2u * v + 1u] = 1; }
 
 // register_state updates of one step (rv_generator_avx.cpp:1356-1397): each
@@ -1573,27 +1627,20 @@ DEV void ra_commit_syms(const Dev &d, const RaStep &r) {
 }
 
 // Functions outside lane 0 of their group: their swapped flags are never set
-// (only lane-0 registers are ever looked up), so each walks alone.  Per step,
-// the registers each group looks up are recorded as min/max group per register.
-// permw lists these functions by size, largest first, so that the 64 walks of
-// a workgroup take about the same number of steps.  A function's virtual
-// registers are named by that function alone (k_xref_check), so each walk keeps
-// them in an LDS cache of WALK_CACHE entries (slot = word offset in the
-// function mod WALK_CACHE; entry = offset << 10 | valid << 9 | state), reads
-// HBM only on a miss, and writes every change through to HBM (stores that are
-// never waited for).  The words themselves are staged
-// into LDS WALK_CHUNK steps at a time, loaded cooperatively (consecutive
-// threads, consecutive words of one function).
-constexpr uint32_t WALK_CACHE = 64;
-// The walks' register ring of the newest definitions holds RING + 1 entries
-// (RING is the index mask: 3 or 7, chosen by the autotuner per size bucket;
-// 2 and 16 entries measured slower on every workload).
-constexpr uint32_t WALK_CHUNK = 32;
+// (only lane-0 registers are ever looked up), so each walks alone.  What the
+// lane-0 functions need of them is which registers each group looks up at each
+// step.  permw lists these functions by size, largest first, so that the 64
+// walks of a workgroup take about the same number of steps.
+//
 // Workgroups spread their per-step lookup records over up to WALK_COPIES
 // copies of the (step, register) tables (copy = workgroup mod copies), which
 // k_walk_merge folds: one table shared by every workgroup serializes its
-// atomics on the same few addresses.
+// atomics on the same few addresses.  Programs of at most RA0_WAVE_GROUPS
+// groups have (step, group) tables of 64-bit register masks instead, in up to
+// MASK_COPIES copies.
 constexpr uint32_t WALK_COPIES = 16;
+constexpr uint32_t MASK_COPIES = 2;
+constexpr uint32_t RA0_WAVE_GROUPS = 64;
 // Walk and lockstep may run at the same time: for each program whose lockstep
 // does, each walk workgroup holding functions of it publishes the program's
 // table rows in chunks of WALK_PUB rows, adding 1 to done[cbase + chunk]
@@ -1613,14 +1660,15 @@ constexpr uint64_t RA0_WAIT_TICKS = 25000000ull;  // 0.25 s
 
 // One program's allocation: functions from fbase (nf of them) in groups of 8
 // (L groups), maxsize = its longest function; its slices of the lane-0 group
-// order (perm + poff) and of the (step, register) lookup tables (+ gbase).  The
+// order (perm + poff) and of the lookup tables (+ gbase: (step, register)
+// tables, or (step, group) masks when L is at most RA0_WAVE_GROUPS).  The
 // tables hold `rows` steps: every step while a lane-0 function is running, then
 // (when some other function runs longer) one last row that gathers all later
 // steps.  Past its lane-0 functions the snapshot no longer changes and no owner
 // reads, so a later lookup only marks, whatever its step.
 // cbase: its first row chunk in the walk's publish counters (RA0_NOPUB when its
-// lockstep does not run at the same time as the walk).
-struct Ra0Prog { uint32_t fbase, L, maxsize, poff; uint64_t gbase; uint32_t nf, rows, cbase, pad; };
+// lockstep does not run at the same time as the walk).  prg: its index.
+struct Ra0Prog { uint32_t fbase, L, maxsize, poff; uint64_t gbase; uint32_t nf, rows, cbase, prg; };
 constexpr uint32_t RA0_NOPUB = 0xFFFFFFFFu;
 
 // OR of v over the 8 lanes of each group of a wave, every lane active (DPP:
@@ -1633,115 +1681,63 @@ DEV uint32_t sm_or8(uint32_t v) {
 }
 DEV uint64_t sm_or8_64(uint64_t v) { return (uint64_t)sm_or8((uint32_t)v) | ((uint64_t)sm_or8((uint32_t)(v >> 32)) << 32); }
 
-// The walk's cache of a function's states, kept by one thread: ring slot
-// x & WALK_RING holds the newest definitions (tag x << 10 | valid << 9 |
-// state); the LDS cache c[x % WALK_CACHE][lane] holds older ones; HBM (sym)
-// all of them (written through).  The ring is named registers selected by
-// index bits (an array would be indexed through scratch memory); the walks use
-// four of its eight.
-struct WcRing { uint32_t r0, r1, r2, r3, r4, r5, r6, r7; };
-
-DEV uint32_t wc_ring_at(const WcRing &g, uint32_t k) {
-    const uint32_t a = (k & 1u) ? g.r1 : g.r0, b = (k & 1u) ? g.r3 : g.r2;
-    const uint32_t c = (k & 1u) ? g.r5 : g.r4, e = (k & 1u) ? g.r7 : g.r6;
-    const uint32_t lo = (k & 2u) ? b : a, hi = (k & 2u) ? e : c;
-    return (k & 4u) ? hi : lo;
+// One step of a walk (rv_generator_avx.cpp:1062-1397) from the word's op, the
+// registers its operands are read in and the function's lifetime mask: the
+// registers freed (m; never x0), the one written (rdr, dm), the live registers
+// looked up, the new lifetime.
+struct OpStep { uint32_t rdr; uint64_t m, dm, look, life; };
+DEV OpStep op_eval(uint32_t op, uint32_t r1, uint32_t r2, uint64_t life) {
+    OpStep s;
+    s.m = ((1ull << r1) | (1ull << r2)) & ~1ull;
+    const uint64_t cl = life & ~s.m;
+    const uint32_t fr = ~(uint32_t)cl;  // free integer registers (ffz_gcc); none: t0
+    const uint32_t al = fr ? (uint32_t)__builtin_ctz(fr) : 5u;
+    s.rdr = (op & OP_ALLOC) ? al : (op >> OP_CONST) & 63u;
+    s.dm = 1ull << s.rdr;
+    s.look = ((s.m & life) | (s.dm & cl)) & ~1ull;
+    s.life = cl | s.dm;
+    return s;
 }
 
-DEV void wc_ring_set(WcRing &g, uint32_t k, uint32_t v) {
-    g.r0 = k == 0 ? v : g.r0; g.r1 = k == 1 ? v : g.r1; g.r2 = k == 2 ? v : g.r2; g.r3 = k == 3 ? v : g.r3;
-    g.r4 = k == 4 ? v : g.r4; g.r5 = k == 5 ? v : g.r5; g.r6 = k == 6 ? v : g.r6; g.r7 = k == 7 ? v : g.r7;
-}
+// The ops of four consecutive words (any 4-byte alignment).
+struct __attribute__((packed, aligned(4))) Op4 { uint32_t o[4]; };
+// Four consecutive states of a function's registers (any 2-byte alignment).
+struct __attribute__((packed, aligned(2))) Sym4 { uint64_t v; };
 
-// Write-through variants: every state change is stored to HBM as it is made,
-// so HBM always holds each register's current state and a cache slot may be
-// overwritten without a look at what it held.  Invariant: a register held in
-// the ring is current there; one held in its LDS slot and not in the ring is
-// current there; a register leaving the ring overwrites its LDS slot.
-//
-// A step reads its two operands' states without branching on where they are:
-// both ring slots and both cache slots are read for every lane, and the lanes
-// whose operand is in neither (or is another function's register) load it from
-// HBM inside one wave-uniform branch that waits for its own loads.  raw1 / raw2
-// are 0 for an operand that is not a virtual register (one past the register
-// space is flagged, as virt_ok does).
-template <uint32_t WALK_RING>
-DEV void walk_gets(const Dev &d, uint32_t (*c)[64], const WcRing &ring, uint32_t lane, uint32_t start,
-                   uint32_t size, bool con, bool on, uint32_t y, uint32_t z, uint32_t &raw1, uint32_t &raw2) {
-    const bool n1 = on && (int32_t)y > 63, n2 = on && (int32_t)z > 63;
-    if ((n1 && y - 64u >= d.W0) || (n2 && z - 64u >= d.W0)) atomicOr(d.flags, EF_OOB);
-    const bool v1 = n1 && y - 64u < d.W0, v2 = n2 && z - 64u < d.W0;
-    const uint32_t x1 = y - 64u - start, x2 = z - 64u - start;
-    const bool l1 = v1 && con && x1 < size, l2 = v2 && con && x2 < size;
-    const uint32_t e1 = wc_ring_at(ring, x1 & WALK_RING), e2 = wc_ring_at(ring, x2 & WALK_RING);
-    const uint32_t c1 = c[x1 % WALK_CACHE][lane], c2 = c[x2 % WALK_CACHE][lane];
-    const bool r1 = e1 != 0u && (e1 >> 10) == x1, r2 = e2 != 0u && (e2 >> 10) == x2;
-    const bool m1 = v1 && !(l1 && (r1 || (c1 != 0u && (c1 >> 10) == x1)));
-    const bool m2 = v2 && !(l2 && (r2 || (c2 != 0u && (c2 >> 10) == x2)));
-    raw1 = v1 ? ((r1 ? e1 : c1) & 0x1FFu) : 0u;
-    raw2 = v2 ? ((r2 ? e2 : c2) & 0x1FFu) : 0u;
-    if (__ballot(m1 || m2)) {
-        // every lane loads (entry 0 where it hit), so that both loads issue
-        // back to back under one wait
-        const uint32_t g1 = d.sym[m1 ? y - 64u : 0u];
-        const uint32_t g2 = d.sym[m2 ? z - 64u : 0u];
-        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): no load is outstanding past this branch
-        if (m1) { raw1 = g1; if (l1) c[x1 % WALK_CACHE][lane] = (x1 << 10) | 0x200u | g1; }
-        if (m2) { raw2 = g2; if (l2) c[x2 % WALK_CACHE][lane] = (x2 << 10) | 0x200u | g2; }
-    }
-}
-
-// Stages the words of steps i .. i+WALK_CHUNK-1 of the 64 walked functions in
-// LDS: thread t loads word i + t % 32 of functions t / 32, t / 32 + 2, ... (two
-// batches of 16 loads, consecutive threads on consecutive words of one
-// function).  Each load's function start and size come from the lanes that hold
-// them (readlane), and past a function's end the load reads word 0 and stages
-// zeros, so that the loads issue back to back.
-DEV void walk_stage(const Dev &d, uint4 (*words)[64], uint32_t i, uint32_t lane, uint32_t start, uint32_t size) {
-    const uint32_t kk = lane % WALK_CHUNK;
-    const bool odd = lane >= WALK_CHUNK;
-#pragma unroll
-    for (uint32_t h = 0; h < 2; ++h) {
-        uint4 tmp[16];
-#pragma unroll
-        for (uint32_t r = 0; r < 16; ++r) {
-            const uint32_t g = 2u * (16u * h + r);
-            const uint32_t st0 = (uint32_t)__builtin_amdgcn_readlane((int)start, (int)g);
-            const uint32_t st1 = (uint32_t)__builtin_amdgcn_readlane((int)start, (int)g + 1);
-            const uint32_t sz0 = (uint32_t)__builtin_amdgcn_readlane((int)size, (int)g);
-            const uint32_t sz1 = (uint32_t)__builtin_amdgcn_readlane((int)size, (int)g + 1);
-            const uint32_t st = odd ? st1 : st0, sz = odd ? sz1 : sz0;
-            const bool in = i + kk < sz;
-            const uint4 wv = d.w0_f4[in ? st + i + kk : 0u];
-            tmp[r] = in ? wv : make_uint4(0, 0, 0, 0);
-        }
-#pragma unroll
-        for (uint32_t r = 0; r < 16; ++r) words[kk][(odd ? 1u : 0u) + 2u * (16u * h + r)] = tmp[r];
-    }
-}
-
-
-template <uint32_t WALK_RING>
+// One function per lane.  The states of a function's last OP_ROWS words are in
+// an LDS ring of bytes, row = word mod OP_ROWS (a state here is just the
+// register the word's rd was given; it never changes); operands further back
+// are read from HBM.  Bound by the step's chain of instructions (latency; one
+// wave per SIMD): steps run four at a time, on one 16-byte load of ops issued
+// four steps ahead and one 8-byte store of states.  A 62-function program's
+// 4115 steps: 4.7 -> 1.7 ms against words compared and states looked up in a
+// tagged cache at each step.
 __global__ __launch_bounds__(64) void k_ra_walk(Dev d, uint32_t *gmin_all, uint32_t *gmax_all, uint64_t stride,
-                                                uint32_t copies, const Ra0Prog *progs, const uint32_t *permw,
+                                                uint32_t copies, unsigned long long *mask_all, uint64_t mstride,
+                                                uint32_t mcopies, const Ra0Prog *progs, const uint32_t *permw,
                                                 uint32_t nw, uint32_t *done) {
     __shared__ uint32_t smin[64], smax[64];
-    __shared__ uint32_t cache[WALK_CACHE][64];
-    __shared__ uint4 words[WALK_CHUNK][64];
+    __shared__ uint8_t ring[OP_ROWS * 64];
     const uint32_t lane = threadIdx.x;
     const uint32_t t = blockIdx.x * 64u + lane;
     const uint32_t f = t < nw ? permw[t] : d.F;
     const bool act = f < d.F;
-    const uint32_t start = act ? d.fstarts[f] : 0u;
-    const uint32_t size = act ? d.fsizes[f] : 0u;
     // group = function index within its program / 8; lookup table of the program
     const uint32_t prg = act ? prog_of(d.pf, d.P, f) : 0xFFFFFFFFu;
     const uint32_t grp = act ? (f - d.pf[prg]) >> 3 : 0u;
+    const bool skip = act && d.cflag[prg] != 0;  // k_ra_serial's
+    const uint32_t start = act ? d.fstarts[f] : 0u;
+    const uint32_t size = act && !skip ? d.fsizes[f] : 0u;
+    const uint32_t L = act ? progs[prg].L : 0u;
+    const bool masks = L <= RA0_WAVE_GROUPS;
     uint32_t pmin = prg, pmax = act ? prg : 0u;
     for (int s = 32; s > 0; s >>= 1) { pmin = min(pmin, (uint32_t)__shfl_xor((int)pmin, s, 64)); pmax = max(pmax, (uint32_t)__shfl_xor((int)pmax, s, 64)); }
-    const bool one = pmin == pmax;  // the workgroup's functions all belong to one program
+    // the workgroup's functions all belong to one program with (step, register) tables
+    const bool one = pmin == pmax && __ballot(act && !masks) != 0;
+    const bool any_reg = __ballot(act && !masks) != 0;
     uint32_t *gmin = gmin_all + (blockIdx.x % copies) * stride;
     uint32_t *gmax = gmax_all + (blockIdx.x % copies) * stride;
+    unsigned long long *mtab = mask_all + (blockIdx.x % mcopies) * mstride;
     const uint64_t tb = one ? progs[pmin].gbase : 0u;  // table base of that program
     const uint32_t tlast = one ? progs[pmin].rows - 1u : 0u;
     const uint64_t mbase = act ? progs[prg].gbase : 0u;  // own program's table and its last row
@@ -1764,229 +1760,378 @@ __global__ __launch_bounds__(64) void k_ra_walk(Dev d, uint32_t *gmin_all, uint3
         }
     }
     const uint32_t cbase = act ? progs[prg].cbase : RA0_NOPUB;
-    const bool publishes = done && lead && cbase != RA0_NOPUB;
-    const bool con = size < (1u << 22);  // cache on (tags hold 22 bits of word offset)
-    WcRing ring{0, 0, 0, 0, 0, 0, 0, 0};
-    // update of virtual register v (inside [64, 64 + W0))
-    auto put = [&](uint32_t v, uint32_t val, bool own) {  // own: v is defined by the word being committed
-        const uint32_t x = v - 64u - start;
-        d.sym[v - 64u] = (uint16_t)val;  // write-through
-        if (!con || x >= size) return;
-        const uint32_t e = wc_ring_at(ring, x & WALK_RING);
-        if (e && (e >> 10) == x) { wc_ring_set(ring, x & WALK_RING, (x << 10) | 0x200u | val); return; }
-        if (!own) { cache[x % WALK_CACHE][lane] = (x << 10) | 0x200u | val; return; }
-        if (e) cache[(e >> 10) % WALK_CACHE][lane] = e;
-        wc_ring_set(ring, x & WALK_RING, (x << 10) | 0x200u | val);
-    };
-    for (uint32_t k = 0; k < WALK_CACHE; ++k) cache[k][lane] = 0;
+    const bool publishes = done && lead && cbase != RA0_NOPUB && pw != 0;
+    const uint32_t nch = mlast / WALK_PUB + 1u;
+    const uint32_t npub = publishes ? min(nch, (pw + WALK_PUB - 1u) / WALK_PUB) : 0u;  // chunks it takes part in
+    uint32_t pubd = 0;
     smin[lane] = 0xFFFFFFFFu; smax[lane] = 0;
     uint32_t wmax = size;
     for (int s = 32; s > 0; s >>= 1) { uint32_t o = __shfl_xor(wmax, s, 64); wmax = wmax > o ? wmax : o; }
     uint64_t life = 0x1Full;
-    uint4 wn = make_uint4(0, 0, 0, 0);  // the word of the next step
+    const uint32_t *ops = d.ops + start;
+    Op4 on = *reinterpret_cast<const Op4 *>(ops);
     __syncthreads();
-    for (uint32_t i = 0; i < wmax; ++i) {
-        if (i % WALK_CHUNK == 0) {
-            walk_stage(d, words, i, lane, start, size);
-            __syncthreads();
-            wn = words[0][lane];
-        }
-        const uint4 w = wn;
-        if ((i + 1) % WALK_CHUNK != 0) wn = words[(i + 1) % WALK_CHUNK][lane];  // a step ahead
-        const bool on = (int32_t)i < (int32_t)size;
-        uint32_t raw1, raw2;
-        walk_gets<WALK_RING>(d, cache, ring, lane, start, size, con, on, w.y, w.z, raw1, raw2);
-        if (on) {
-            raw1 &= 0xFFu; raw2 &= 0xFFu;
-            const RaStep r = ra_eval_raw(w.w, w.x, w.y, w.z, raw1, raw2, false, false, life);
-            xref_check_fields(d, f, start, size, r.ord, r.rs1, r.rs2);
-            if (one) {
-                if (r.swd) { atomicMin(&smin[r.rdr], grp); atomicMax(&smax[r.rdr], grp + 1u); }
-                if (r.sw1) { atomicMin(&smin[r.r1r], grp); atomicMax(&smax[r.r1r], grp + 1u); }
-                if (r.sw2) { atomicMin(&smin[r.r2r], grp); atomicMax(&smax[r.r2r], grp + 1u); }
-            } else {  // functions of several programs: post straight to each program's table
-                const uint64_t row = mbase + (uint64_t)min(i, mlast) * 64u;
-                if (r.swd) { atomicMin(&gmin[row + r.rdr], grp); atomicMax(&gmax[row + r.rdr], grp + 1u); }
-                if (r.sw1) { atomicMin(&gmin[row + r.r1r], grp); atomicMax(&gmax[row + r.r1r], grp + 1u); }
-                if (r.sw2) { atomicMin(&gmin[row + r.r2r], grp); atomicMax(&gmax[row + r.r2r], grp + 1u); }
+    for (uint32_t i0 = 0; i0 < wmax; i0 += 4) {
+        const Op4 ow = on;
+        on = *reinterpret_cast<const Op4 *>(ops + min(i0 + 4u, size));  // (past the end: never used)
+        uint32_t st[4];
+#pragma unroll
+        for (uint32_t q = 0; q < 4; ++q) {
+            const uint32_t i = i0 + q;
+            const bool run = (int32_t)i < (int32_t)size;
+            const uint32_t op = run ? ow.o[q] : 0u;
+            const uint32_t d1 = op & 0xFFu, d2 = (op >> 8) & 0xFFu;
+            uint32_t r1 = ring[((i - d1) & (OP_ROWS - 1u)) * 64u + lane];
+            uint32_t r2 = ring[((i - d2) & (OP_ROWS - 1u)) * 64u + lane];
+            r1 = d1 ? r1 : 0u; r2 = d2 ? r2 : 0u;
+            if (__ballot((op & (OP_FAR1 | OP_FAR2)) != 0)) {
+                if (op & (OP_FAR1 | OP_FAR2)) {
+                    const uint4 w = d.w0_f4[start + i];
+                    if (op & OP_FAR1) r1 = d.sym[w.y - 64u] & 0xFFu;
+                    if (op & OP_FAR2) r2 = d.sym[w.z - 64u] & 0xFFu;
+                }
             }
-            life = r.newlife;
-            // register_state updates (ra_commit_syms): destination, then rs1, then rs2
-            if (((int32_t)r.ord > 63 && r.ord - 64u >= d.W0) || ((int32_t)r.rs1 > 63 && r.rs1 - 64u >= d.W0) ||
-                ((int32_t)r.rs2 > 63 && r.rs2 - 64u >= d.W0)) {
-                atomicOr(d.flags, EF_OOB);
-            } else {
-                // only entries whose value changes are stored; a destination is
-                // skipped when an operand names it (the operand's store is later)
-                const uint32_t self = 64u + start + i;
-                const bool vo = (int32_t)r.ord > 63, v1 = (int32_t)r.rs1 > 63, v2 = (int32_t)r.rs2 > 63;
-                if (vo && !(v1 && r.rs1 == r.ord) && !(v2 && r.rs2 == r.ord)) put(r.ord, r.rdr, r.ord == self);
-                if (v1 && !(v2 && r.rs2 == r.rs1) && r.r1r != raw1) put(r.rs1, r.r1r, false);
-                if (v2 && r.r2r != raw2) put(r.rs2, r.r2r, false);
+            const OpStep s = op_eval(op, r1, r2, life);
+            life = s.life;
+            st[q] = (op & OP_SELF) && !(op & OP_ZERO) ? s.rdr : 0u;
+            ring[(i & (OP_ROWS - 1u)) * 64u + lane] = (uint8_t)st[q];
+            if (run && masks && s.look) atomicOr(&mtab[mbase + (uint64_t)min(i, mlast) * L + grp], (unsigned long long)s.look);
+            if (any_reg) {
+                uint64_t lk = run && !masks ? s.look : 0ull;
+                if (!one) {  // functions of several programs: post straight to each program's table
+                    const uint64_t row = mbase + (uint64_t)min(i, mlast) * 64u;
+                    while (lk) {
+                        const uint32_t r = (uint32_t)__builtin_ctzll(lk);
+                        lk &= lk - 1;
+                        atomicMin(&gmin[row + r], grp); atomicMax(&gmax[row + r], grp + 1u);
+                    }
+                } else {
+                    while (lk) {
+                        const uint32_t r = (uint32_t)__builtin_ctzll(lk);
+                        lk &= lk - 1;
+                        atomicMin(&smin[r], grp); atomicMax(&smax[r], grp + 1u);
+                    }
+                    lds_barrier();
+                    const uint32_t mx = smax[lane];
+                    if (mx) {
+                        atomicMin(&gmin[tb + (uint64_t)min(i, tlast) * 64u + lane], smin[lane]);
+                        atomicMax(&gmax[tb + (uint64_t)min(i, tlast) * 64u + lane], mx);
+                        smin[lane] = 0xFFFFFFFFu; smax[lane] = 0;
+                    }
+                    lds_barrier();
+                }
             }
         }
-        lds_barrier();
-        uint32_t mx = smax[lane];
-        if (mx) {
-            atomicMin(&gmin[tb + (uint64_t)min(i, tlast) * 64u + lane], smin[lane]);
-            atomicMax(&gmax[tb + (uint64_t)min(i, tlast) * 64u + lane], mx);
-            smin[lane] = 0xFFFFFFFFu; smax[lane] = 0;
+        // (sym starts cleared: only words past the last whole four need care)
+        if ((int32_t)(i0 + 3u) < (int32_t)size) {
+            reinterpret_cast<Sym4 *>(d.sym + start + i0)->v =
+                (uint64_t)(st[0] | (st[1] << 16)) | ((uint64_t)(st[2] | (st[3] << 16)) << 32);
+        } else {
+#pragma unroll
+            for (uint32_t q = 0; q < 4; ++q)
+                if ((int32_t)(i0 + q) < (int32_t)size) d.sym[start + i0 + q] = (uint16_t)st[q];
         }
-        lds_barrier();
         if (done) {
-            // a program's functions here leave a chunk of its rows (steps past
-            // its last row all post to that row): publish it after every
-            // lane's posts are visible
-            bool pub = false;
-            uint32_t chunk = 0;
-            if (publishes && i < pw) {
-                const uint32_t r = min(i, mlast), rn = min(i + 1u, mlast);
-                pub = i + 1u == pw || r / WALK_PUB != rn / WALK_PUB;
-                chunk = cbase + r / WALK_PUB;
-            }
+            // chunks of the program's rows that its functions here are past
+            // (steps past its last row all post to that row): published after
+            // every lane's posts are visible; at most one chunk per four steps
+            const uint32_t e = i0 + 4u;
+            const uint32_t past = e >= pw ? npub : min(e / WALK_PUB, nch - 1u);
+            const bool pub = publishes && past > pubd;
             if (__ballot(pub)) {
                 __threadfence();
                 __syncthreads();
-                if (pub) __hip_atomic_fetch_add(&done[chunk], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (pub) {
+                    __hip_atomic_fetch_add(&done[cbase + pubd], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    ++pubd;
+                }
             }
         }
     }
 }
 
-// gmin/gmax[e] = min/max over the copies (copy c at c * stride).
-__global__ void k_walk_merge(uint32_t *gmin, uint32_t *gmax, uint64_t stride, uint32_t copies) {
+// gmin/gmax[e] = min/max over the copies (copy c at c * stride); mask[e] = OR
+// over its copies.
+__global__ void k_walk_merge(uint32_t *gmin, uint32_t *gmax, uint64_t stride, uint32_t copies,
+                             unsigned long long *mask, uint64_t mstride, uint32_t mcopies) {
     const uint64_t e = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
-    if (e >= stride) return;
-    uint32_t mn = gmin[e], mx = gmax[e];
-    for (uint32_t c = 1; c < copies; ++c) {
-        mn = min(mn, gmin[c * stride + e]);
-        mx = max(mx, gmax[c * stride + e]);
+    if (copies > 1 && e < stride) {
+        uint32_t mn = gmin[e], mx = gmax[e];
+        for (uint32_t c = 1; c < copies; ++c) {
+            mn = min(mn, gmin[c * stride + e]);
+            mx = max(mx, gmax[c * stride + e]);
+        }
+        gmin[e] = mn; gmax[e] = mx;
     }
-    gmin[e] = mn; gmax[e] = mx;
+    if (mcopies > 1 && e < mstride) {
+        unsigned long long m = mask[e];
+        for (uint32_t c = 1; c < mcopies; ++c) m |= mask[c * mstride + e];
+        mask[e] = m;
+    }
 }
 
-// Programs of at most 8 functions (one group): the reference's vector loop
-// runs them as one 8-lane vector, and only its lane 0 writes region 0 of
-// register_state.  One wave holds 8 such programs, lane 8s + k walking function
-// k of program slot s (the walk's register ring, LDS cache and word staging).
-// Per step the 8 lanes' swap lookups are ORed across the group; lane 0 then
-// marks the snapshot entries looked up (not one its own current word names:
-// its reset lands after a same-group mark) and updates region 0 with its own
-// write and resets.  Every lookup and mark of the step comes after every
-// operand read of the step, as in the vector loop.  A mark on a register outside
-// lane 0's own function cannot be kept in its cache: the program then takes the
-// exact serial path.  The first `solo` programs of the list (the longest) have
-// a wave each, in slot 0, so that no other program's rarer paths (a cache
-// miss, a mark) hold up their steps.
-template <uint32_t WALK_RING>
+// Waits (every lane of the wave) until the walk has published row chunk c;
+// `ok` turns false, for good, when a wait sees no progress for RA0_WAIT_TICKS.
+DEV void ra0_wait(const Dev &d, const uint32_t *done, const uint32_t *need, uint32_t c, bool &ok) {
+    if (!ok) return;
+    const uint32_t want = need[c];
+    const uint64_t t0 = wall_clock64();
+    while (__hip_atomic_load(&done[c], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT) < want) {
+        if (wall_clock64() - t0 > RA0_WAIT_TICKS) { ok = false; atomicOr(d.flags, EF_WAIT); return; }
+        __builtin_amdgcn_s_sleep(2);
+    }
+}
+
+// ---------------------------------------------- lane-0 functions in one wave
+// Region 0 of the reference's register_state holds the last lane-0 write per
+// physical register; every lookup of any function at step i reads its
+// step-start snapshot and marks the virtual register found there as swapped.
+// A lane steps one function; the snapshot is kept apart by owner: `own` has
+// the entries that hold one of this function's virtual registers, hold[r] the
+// word that defines it, `mk` the owned entries whose register is marked
+// already.  A register can only be held by the entry of the register it was
+// defined in, its home, so a state is
+//     register | swapped << 8 | home << 9
+// and the entry an operand is held by is found from its state alone.  States of
+// the last OP_ROWS words are in an LDS ring; HBM (sym) has all of them, written
+// through.
+struct RaL0 { uint32_t start, size; uint64_t life, own, mk; };
+
+template <int CTRL, int RMASK = 0xF>
+DEV uint32_t dpp_or(uint32_t v) {
+    return v | (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, RMASK, 0xF, RMASK == 0xF);
+}
+// Inclusive OR over the lanes up to this one, in the wave's first row of 16
+// lanes (ROWS 1) or the whole wave; every lane active.
+template <int ROWS>
+DEV uint32_t scan_or(uint32_t v) {
+    v = dpp_or<0x111>(v); v = dpp_or<0x112>(v); v = dpp_or<0x114>(v); v = dpp_or<0x118>(v);  // row_shr 1, 2, 4, 8
+    if (ROWS > 1) { v = dpp_or<0x142, 0xA>(v); v = dpp_or<0x143, 0xC>(v); }                  // row_bcast 15, 31
+    return v;
+}
+// The lane below's value (0 in lane 0).
+template <int ROWS>
+DEV uint32_t from_below(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, ROWS > 1 ? 0x138 : 0x111, 0xF, 0xF, true);  // wave_shr / row_shr 1
+}
+// OR over the lanes above this one; `all` the OR over every lane.
+template <int ROWS>
+DEV uint32_t suffix_or(uint32_t v, uint32_t lane, uint32_t &all) {
+    v = dpp_or<0x101>(v); v = dpp_or<0x102>(v); v = dpp_or<0x104>(v); v = dpp_or<0x108>(v);  // row_shl 1, 2, 4, 8
+    uint32_t x = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x101, 0xF, 0xF, true);
+    const uint32_t t0 = (uint32_t)__builtin_amdgcn_readlane((int)v, 0);
+    if (ROWS == 1) { all = t0; return x; }
+    const uint32_t t1 = (uint32_t)__builtin_amdgcn_readlane((int)v, 16), t2 = (uint32_t)__builtin_amdgcn_readlane((int)v, 32),
+                   t3 = (uint32_t)__builtin_amdgcn_readlane((int)v, 48);
+    x |= lane < 48u ? t3 : 0u;
+    x |= lane < 32u ? t2 : 0u;
+    x |= lane < 16u ? t1 : 0u;
+    all = t0 | t1 | t2 | t3;
+    return x;
+}
+
+// One step i of this lane's function on its word's op.  ROWS 0: programs of one
+// group, 8 to a wave, lane 8s + k walking function k of program slot s (l0: k is
+// 0); the group's lookups of the step mark, except an entry whose register the
+// word names (its reset lands after a same-group mark).  ROWS 1, 4: lane j
+// walks the lane-0 function of group j of one program (of at most 16 or 64
+// groups), W being the registers looked up by the group's other functions.
+// There a lookup by a lower group is seen by the owner's operand read of the
+// same step (a flip), settled by re-evaluation until the flips are stable:
+// lane j's depend on the lanes below it alone, so this reaches the in-order
+// result; one by a higher group lands after the owner's own reset; and the last
+// group to write or free a register decides its entry.
+// The ring has a column per lane (RC of them), hold one per lane or, ROWS 0,
+// per program slot (HC).
+template <int ROWS, int RC, int HC>
+DEV void ra_l0_step(const Dev &d, RaL0 &f, uint16_t *ring, uint32_t *hold, uint32_t rc, uint32_t hc, uint32_t lane,
+                    bool l0, uint32_t i, uint32_t opw, uint64_t W) {
+    const bool run = (int32_t)i < (int32_t)f.size;
+    const uint32_t op = run ? opw : 0u;
+    const uint32_t d1 = op & 0xFFu, d2 = (op >> 8) & 0xFFu;
+    uint32_t p1 = i - d1, p2 = i - d2;
+    uint32_t e1 = ring[(p1 & (OP_ROWS - 1u)) * RC + rc], e2 = ring[(p2 & (OP_ROWS - 1u)) * RC + rc];
+    e1 = d1 ? e1 : 0u; e2 = d2 ? e2 : 0u;
+    if (__ballot((op & (OP_FAR1 | OP_FAR2)) != 0)) {
+        if (op & (OP_FAR1 | OP_FAR2)) {
+            const uint4 w = d.w0_f4[f.start + i];
+            if (op & OP_FAR1) { p1 = w.y - 64u - f.start; e1 = d.sym[w.y - 64u]; }
+            if (op & OP_FAR2) { p2 = w.z - 64u - f.start; e2 = d.sym[w.z - 64u]; }
+        }
+    }
+    const uint32_t h1 = e1 >> 9, h2 = e2 >> 9;
+    const uint32_t q1 = hold[h1 * HC + hc], q2 = hold[h2 * HC + hc];
+    const uint32_t sr1 = (op & OP_FP) ? 37u : 5u, sr2 = (op & OP_FP) ? 38u : 6u;
+    bool s1 = (e1 & 0x100u) != 0, s2 = (e2 & 0x100u) != 0;
+    uint32_t r1 = s1 ? sr1 : e1 & 0x3Fu, r2 = s2 ? sr2 : e2 & 0x3Fu;
+    OpStep s = op_eval(op, r1, r2, f.life);
+    // the entries holding the operands (no operand: home x0, which is never held)
+    const uint64_t nb1 = q1 == p1 ? f.own & (1ull << h1) : 0ull, nb2 = q2 == p2 ? f.own & (1ull << h2) : 0ull;
+    const uint64_t nb = nb1 | nb2;
+    const bool self = (op & OP_SELF) != 0;
+    uint64_t mset, lost, won;
+    if (ROWS == 0) {
+        const uint64_t T = sm_or8_64(s.look);
+        lost = s.m | ((op & (OP_SELF | (63u << OP_CONST))) ? s.dm : 0ull);
+        won = self && l0 ? s.dm : 0ull;
+        mset = f.own & T & ~nb;
+    } else {
+        uint32_t tl = (uint32_t)(s.look | W), th = (uint32_t)((s.look | W) >> 32);
+        uint32_t il = scan_or<ROWS>(tl), ih = scan_or<ROWS>(th);  // inclusive over the lanes below
+        uint64_t high = 0;
+        if (__ballot(nb != 0)) {
+            bool f1 = false, f2 = false;
+            const bool w1 = s1, w2 = s2;  // swapped already
+            for (;;) {
+                const uint64_t low = (uint64_t)from_below<ROWS>(il) | ((uint64_t)from_below<ROWS>(ih) << 32);
+                const bool n1 = (nb1 & low) != 0, n2 = (nb2 & low) != 0;
+                const bool ch = (n1 != f1 && !w1) || (n2 != f2 && !w2);
+                if (!__ballot(ch)) break;
+                f1 = n1; f2 = n2;
+                s1 = w1 || f1; s2 = w2 || f2;
+                r1 = s1 ? sr1 : e1 & 0x3Fu; r2 = s2 ? sr2 : e2 & 0x3Fu;
+                s = op_eval(op, r1, r2, f.life);
+                tl = (uint32_t)(s.look | W); th = (uint32_t)((s.look | W) >> 32);
+                il = scan_or<ROWS>(tl); ih = scan_or<ROWS>(th);
+            }
+            uint32_t x;
+            high = (uint64_t)suffix_or<ROWS>(tl, lane, x);
+            high |= (uint64_t)suffix_or<ROWS>(th, lane, x) << 32;
+        }
+        constexpr int LAST = ROWS == 1 ? 15 : 63;
+        const uint64_t T = (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)il, LAST) |
+                           ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)ih, LAST) << 32);
+        const uint64_t touch = s.m | ((op & (OP_SELF | (63u << OP_CONST))) ? s.dm : 0ull);
+        uint32_t al, ah;
+        uint64_t above = (uint64_t)suffix_or<ROWS>((uint32_t)touch, lane, al);
+        above |= (uint64_t)suffix_or<ROWS>((uint32_t)(touch >> 32), lane, ah) << 32;
+        lost = (uint64_t)al | ((uint64_t)ah << 32);
+        won = self ? s.dm & ~above : 0ull;
+        mset = f.own & ((T & ~nb) | (high & nb));
+    }
+    // the step's commit: swapped operands take the register they were read
+    // through, and their flags are cleared
+    uint8_t *symb = reinterpret_cast<uint8_t *>(d.sym + f.start);
+    if (s1) {
+        const uint16_t st = (uint16_t)(r1 | (h1 << 9));
+        if (i - p1 <= OP_WINDOW) ring[(p1 & (OP_ROWS - 1u)) * RC + rc] = st;
+        d.sym[f.start + p1] = st;
+    }
+    if (s2) {
+        const uint16_t st = (uint16_t)(r2 | (h2 << 9));
+        if (i - p2 <= OP_WINDOW) ring[(p2 & (OP_ROWS - 1u)) * RC + rc] = st;
+        d.sym[f.start + p2] = st;
+    }
+    f.mk &= ~nb;
+    uint64_t nm = mset & ~f.mk;
+    f.mk |= mset;
+    // marks not standing yet: the flag byte of the states in the ring and in HBM
+    while (nm) {
+        const uint32_t r = (uint32_t)__builtin_ctzll(nm);
+        nm &= nm - 1;
+        const uint32_t p = hold[r * HC + hc];
+        const uint8_t fl = (uint8_t)(1u | (r << 1));
+        if (i - p <= OP_WINDOW) reinterpret_cast<uint8_t *>(ring)[2u * ((p & (OP_ROWS - 1u)) * RC + rc) + 1u] = fl;
+        symb[2u * p + 1u] = fl;
+    }
+    if (run) {
+        const uint32_t st = self ? ((op & OP_ZERO) ? 0u : s.rdr) | (s.rdr << 9) : 0u;
+        ring[(i & (OP_ROWS - 1u)) * RC + rc] = (uint16_t)st;
+        if (self) {
+            d.sym[f.start + i] = (uint16_t)st;
+            if (ROWS || l0) hold[s.rdr * HC + hc] = i;
+        }
+    }
+    f.life = s.life;
+    f.own = (f.own & ~lost) | won;
+    f.mk &= ~lost;
+}
+
+// Programs of at most 8 functions (one group): the reference's vector loop runs
+// them as one 8-lane vector, and only its lane 0 writes region 0 of
+// register_state.  One wave holds 8 such programs.  The first `solo` programs
+// of the list (the longest) have a wave each, in slot 0, so that no other
+// program's rarer paths (a mark, a state read from HBM) hold up their steps.
+// Latency bound: 1.5 -> 0.58 us a step alone in a wave (a function of 35k words,
+// 52 -> 22 ms).
 __global__ __launch_bounds__(64) void k_ra_group(Dev d, const uint32_t *plist, uint32_t np, uint32_t solo) {
-    __shared__ uint32_t cache[WALK_CACHE][64];
-    __shared__ uint4 words[WALK_CHUNK][64];
-    __shared__ int32_t Sv[8][64];
+    __shared__ uint16_t ring[OP_ROWS * 64];
+    __shared__ uint32_t hold[64 * 8];
     const uint32_t lane = threadIdx.x, slot = lane >> 3, k = lane & 7u;
     const uint32_t pi = blockIdx.x < solo ? (slot == 0 ? blockIdx.x : np) : solo + (blockIdx.x - solo) * 8u + slot;
     const uint32_t prg = pi < np ? plist[pi] : 0xFFFFFFFFu;
     const uint32_t fb = prg != 0xFFFFFFFFu ? d.pf[prg] : 0u;
     const uint32_t nf = prg != 0xFFFFFFFFu ? d.pf[prg + 1] - fb : 0u;
-    const bool act = k < nf && nf <= 8u;
-    if (prg != 0xFFFFFFFFu && nf > 8u) atomicOr(d.flags, EF_OOB);
-    const uint32_t f = fb + k;
-    const uint32_t start = act ? d.fstarts[f] : 0u;
-    const uint32_t size = act ? d.fsizes[f] : 0u;
-    const bool con = size < (1u << 22);
-    WcRing ring{0, 0, 0, 0, 0, 0, 0, 0};
-    auto put = [&](uint32_t v, uint32_t val, bool own) {  // own: v is defined by the word being committed
-        const uint32_t x = v - 64u - start;
-        d.sym[v - 64u] = (uint16_t)val;  // write-through
-        if (!con || x >= size) return;
-        const uint32_t e = wc_ring_at(ring, x & WALK_RING);
-        if (e && (e >> 10) == x) { wc_ring_set(ring, x & WALK_RING, (x << 10) | 0x200u | val); return; }
-        if (!own) { cache[x % WALK_CACHE][lane] = (x << 10) | 0x200u | val; return; }
-        if (e) cache[(e >> 10) % WALK_CACHE][lane] = e;
-        wc_ring_set(ring, x & WALK_RING, (x << 10) | 0x200u | val);
-    };
-    for (uint32_t q = 0; q < WALK_CACHE; ++q) cache[q][lane] = 0;
-    Sv[slot][k] = -1; Sv[slot][k + 8] = -1; Sv[slot][k + 16] = -1; Sv[slot][k + 24] = -1;
-    Sv[slot][k + 32] = -1; Sv[slot][k + 40] = -1; Sv[slot][k + 48] = -1; Sv[slot][k + 56] = -1;
-    uint32_t wmax = size;
+    if (nf > 8u) atomicOr(d.flags, EF_OOB);
+    const bool act = k < nf && nf <= 8u && d.cflag[prg] == 0;  // (flagged programs: k_ra_serial's)
+    RaL0 f{act ? d.fstarts[fb + k] : 0u, act ? d.fsizes[fb + k] : 0u, 0x1Full, 0, 0};
+    uint32_t wmax = f.size;
     for (int s = 32; s > 0; s >>= 1) { uint32_t o = __shfl_xor(wmax, s, 64); wmax = wmax > o ? wmax : o; }
-    // a mark sets the swapped flag in place: in the ring, in the LDS cache, or
-    // as a byte store to HBM (the register bits stay)
-    auto mark = [&](uint32_t v) {
-        const uint32_t x = v - 64u - start;
-        sym_mark(d, v - 64u);  // write-through
-        const uint32_t e = wc_ring_at(ring, x & WALK_RING);
-        if (e && (e >> 10) == x) { wc_ring_set(ring, x & WALK_RING, e | 0x100u); return; }
-        const uint32_t ce = cache[x % WALK_CACHE][lane];
-        if (ce && (ce >> 10) == x) cache[x % WALK_CACHE][lane] = ce | 0x100u;
-    };
-    uint64_t life = 0x1Full;
-    uint64_t valid = 0;  // lane 0 of a slot: region-0 entries holding a virtual register
-    uint64_t mkd = 0;    // lane 0: entries whose register is known to be marked already
-    uint4 wn = make_uint4(0, 0, 0, 0);  // the word of the next step
+    const uint32_t *ops = d.ops + f.start;
+    Op4 on = *reinterpret_cast<const Op4 *>(ops);
     __syncthreads();
-    for (uint32_t i = 0; i < wmax; ++i) {
-        if (i % WALK_CHUNK == 0) {
-            walk_stage(d, words, i, lane, start, size);
-            __syncthreads();
-            wn = words[0][lane];
+    for (uint32_t i = 0; i < wmax; i += 4) {
+        const Op4 ow = on;
+        on = *reinterpret_cast<const Op4 *>(ops + min(i + 4u, f.size));  // (past the end: never used)
+#pragma unroll
+        for (uint32_t q = 0; q < 4; ++q)
+            ra_l0_step<0, 64, 8>(d, f, ring, hold, lane, slot, lane, k == 0, i + q, ow.o[q], 0ull);
+    }
+}
+
+// The lane-0 functions of a program of 2 to 16 (ROWS 1) or 64 (ROWS 4) groups,
+// in step lockstep on one wave: what the groups exchange in a step goes through
+// DPP scans of 64-bit register masks, so a step has no barrier.  The walk's
+// lookups of a step are one mask per group, loaded two blocks of four steps
+// ahead.  Bound by the chain of a step's instructions (latency): 5.4 -> 0.8 us a
+// step for 8 groups, against a workgroup exchanging lookups through LDS atomics
+// and barriers with its states in HBM.
+template <int ROWS>
+__global__ __launch_bounds__(64) void k_ra_lane0_wave(Dev d, const Ra0Prog *progs, const unsigned long long *mask_all,
+                                                      uint64_t mstride, uint32_t mcopies, const uint32_t *done,
+                                                      const uint32_t *need) {
+    constexpr int NL = ROWS == 1 ? 16 : 64;
+    __shared__ uint16_t ring[OP_ROWS * NL];
+    __shared__ uint32_t hold[64 * NL];
+    const uint32_t lane = threadIdx.x, col = lane % NL;
+    const Ra0Prog pg = progs[blockIdx.x];
+    if (d.cflag[pg.prg]) return;  // k_ra_serial's
+    if (pg.L > (uint32_t)NL) { if (lane == 0) atomicOr(d.flags, EF_OOB); return; }
+    const bool act = lane < pg.L;
+    RaL0 f{act ? d.fstarts[pg.fbase + 8u * lane] : 0u, act ? d.fsizes[pg.fbase + 8u * lane] : 0u, 0x1Full, 0, 0};
+    const uint32_t rows = pg.rows;
+    const uint32_t *pdone = done && pg.cbase != RA0_NOPUB ? done + pg.cbase : nullptr;
+    const uint32_t *pneed = pdone ? need + pg.cbase : nullptr;
+    const unsigned long long *mtab = mask_all + pg.gbase + (act ? lane : 0u);
+    const uint64_t m1 = mcopies > 1 ? mstride : 0u;
+    bool wok = true;  // the walk's rows still arrive
+    // rows i .. i + 3 of the walk's masks (both copies), once published
+    struct Rows { unsigned long long a[4], b[4]; };
+    auto load_rows = [&](uint32_t i) {
+        Rows r;
+        if (pdone && i < rows && i % WALK_PUB == 0) ra0_wait(d, pdone, pneed, i / WALK_PUB, wok);
+#pragma unroll
+        for (uint32_t q = 0; q < 4; ++q) {
+            const uint64_t e = (uint64_t)min(i + q, rows - 1u) * pg.L;
+            r.a[q] = mtab[e];
+            r.b[q] = mtab[m1 + e];
         }
-        const bool on = (int32_t)i < (int32_t)size;
-        const uint4 w = wn;
-        if ((i + 1) % WALK_CHUNK != 0) wn = words[(i + 1) % WALK_CHUNK][lane];  // a step ahead
-        RaStep r{};
-        uint64_t look = 0;
-        uint32_t raw1, raw2;
-        walk_gets<WALK_RING>(d, cache, ring, lane, start, size, con, on, w.y, w.z, raw1, raw2);
-        if (on) {
-            // this step's commit may clear a set swapped flag (an operand's, or a
-            // destination that is not the word's own new register): forget what
-            // is marked
-            if (((raw1 | raw2) & 0x100u) || ((int32_t)w.x > 63 && w.x != 64u + start + i)) mkd = 0;
-            r = ra_eval_raw(w.w, w.x, w.y, w.z, raw1 & 0xFFu, raw2 & 0xFFu, (raw1 >> 8) & 1u, (raw2 >> 8) & 1u, life);
-            xref_check_fields(d, f, start, size, r.ord, r.rs1, r.rs2);
-            if (r.swd) look |= 1ull << r.rdr;
-            if (r.sw1) look |= 1ull << r.r1r;
-            if (r.sw2) look |= 1ull << r.r2r;
-            life = r.newlife;
-        }
-        // the group's lookups of this step, at every lane of the group
-        const uint64_t glook = sm_or8_64(look);
-        if (k == 0) {
-            // marks on the step-start snapshot, before any commit of the step
-            uint64_t m = glook & valid & ~mkd;
-            while (m) {
-                const uint32_t reg = (uint32_t)__builtin_ctzll(m);
-                m &= m - 1;
-                const uint32_t v = (uint32_t)Sv[slot][reg];
-                if (on && (v == r.ord || v == r.rs1 || v == r.rs2)) continue;
-                if (v - 64u - start < size && con) { mark(v); mkd |= 1ull << reg; }
-                else { atomicOr(d.flags, EF_XCONFLICT); d.cflag[prg] = 1; }
-            }
-        }
-        if (on) {
-            // register_state updates (ra_commit_syms): destination, then rs1, then rs2
-            if (((int32_t)r.ord > 63 && r.ord - 64u >= d.W0) || ((int32_t)r.rs1 > 63 && r.rs1 - 64u >= d.W0) ||
-                ((int32_t)r.rs2 > 63 && r.rs2 - 64u >= d.W0)) {
-                atomicOr(d.flags, EF_OOB);
-            } else {
-                // only entries whose value changes are stored; a destination is
-                // skipped when an operand names it (the operand's store is later)
-                const uint32_t self = 64u + start + i;
-                const bool vo = (int32_t)r.ord > 63, v1 = (int32_t)r.rs1 > 63, v2 = (int32_t)r.rs2 > 63;
-                if (vo && !(v1 && r.rs1 == r.ord) && !(v2 && r.rs2 == r.ord)) put(r.ord, r.rdr, r.ord == self);
-                if (v1 && !(v2 && r.rs2 == r.rs1) && r.r1r != raw1) put(r.rs1, r.r1r, false);
-                if (v2 && r.r2r != raw2) put(r.rs2, r.r2r, false);
-            }
-            if (k == 0) {  // region 0: the write, then the resets (a reset of the written register is skipped)
-                if (r.ord) {
-                    Sv[slot][r.rdr] = (int32_t)r.ord;
-                    valid = (int32_t)r.ord >= 64 ? valid | (1ull << r.rdr) : valid & ~(1ull << r.rdr);
-                    mkd &= ~(1ull << r.rdr);
-                }
-                if (r.r1r != r.rdr) { Sv[slot][r.r1r] = -1; valid &= ~(1ull << r.r1r); }
-                if (r.r2r != r.rdr) { Sv[slot][r.r2r] = -1; valid &= ~(1ull << r.r2r); }
-            }
+        return r;
+    };
+    auto load_ops = [&](uint32_t i) { return *reinterpret_cast<const Op4 *>(d.ops + f.start + min(i, f.size)); };
+    Rows wa = load_rows(0), wb = load_rows(4);
+    Op4 oa = load_ops(0), ob = load_ops(4);
+    __syncthreads();
+    for (uint32_t i = 0; i < rows; i += 4) {
+        const Rows w = wa;
+        const Op4 o = oa;
+        wa = wb; oa = ob;
+        wb = load_rows(i + 8u);
+        ob = load_ops(i + 8u);
+#pragma unroll
+        for (uint32_t q = 0; q < 4; ++q) {
+            const uint64_t W = act && i + q < rows ? w.a[q] | w.b[q] : 0ull;
+            ra_l0_step<ROWS, NL, NL>(d, f, ring, hold, col, col, lane, true, i + q, o.o[q], W);
         }
     }
 }
@@ -2016,9 +2161,8 @@ __global__ __launch_bounds__(64) void k_ra_group(Dev d, const uint32_t *plist, u
 // nf - 1, seg[k] a multiple of 8).  Lanes exchange values with DPP inside a
 // group's 8 lanes and with readlane across groups; region 0 of each program
 // is an LDS table read by lane = register, double-buffered by step parity.
-// A register named outside its own function is noted for k_xref_check as in
-// the other kernels; a mark on one, which the owner's bytes cannot hold,
-// sends the program to the exact serial path.
+// (Programs naming registers outside their own function are reallocated by
+// k_ra_serial, whatever this kernel makes of them.)
 constexpr uint32_t SM_CHUNK = 32;        // steps per staged chunk of words
 constexpr uint32_t SM_PROGS = 8;         // programs per wave at most
 constexpr uint32_t SM_STATE_OFF = 40960; // LDS bytes before the register states
@@ -2115,8 +2259,7 @@ __global__ __launch_bounds__(64) void k_ra_small(Dev d, const SmWave *waves) {
                 for (uint32_t r = 0; r < 16; ++r) words[kk][g0 + 2u * (16u * h + r)] = tmp[r];
             }
             __syncthreads();
-            // this function's words of the chunk: registers past the words, and
-            // names outside the function (noted for k_xref_check)
+            // this function's words of the chunk: registers past the words
             for (uint32_t k = 0; k < SM_CHUNK && i + k < size; ++k) {
                 const uint4 wk = words[k][lane];
                 if (((int32_t)wk.x > 63 && wk.x - 64u >= d.W0) || ((int32_t)wk.y > 63 && wk.y - 64u >= d.W0) ||
@@ -2124,7 +2267,6 @@ __global__ __launch_bounds__(64) void k_ra_small(Dev d, const SmWave *waves) {
                     atomicOr(d.flags, EF_OOB);
                     bad = true;
                 }
-                xref_check_fields(d, f, start, size, wk.x, wk.y, wk.z);
             }
         }
         const uint32_t c = i & 1u, nx = c ^ 1u;
@@ -2479,18 +2621,6 @@ DEV void ra0_row(const uint32_t *gmin, const uint32_t *gmax, uint64_t stride, ui
     for (uint32_t c = 1; c < RA0_MAXCOPIES; ++c) { mn = min(mn, a[c]); mx = max(mx, b[c]); }
 }
 
-// Waits (every lane of the wave) until the walk has published row chunk c;
-// `ok` turns false, for good, when a wait sees no progress for RA0_WAIT_TICKS.
-DEV void ra0_wait(const Dev &d, const uint32_t *done, const uint32_t *need, uint32_t c, bool &ok) {
-    if (!ok) return;
-    const uint32_t want = need[c];
-    const uint64_t t0 = wall_clock64();
-    while (__hip_atomic_load(&done[c], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT) < want) {
-        if (wall_clock64() - t0 > RA0_WAIT_TICKS) { ok = false; atomicOr(d.flags, EF_WAIT); return; }
-        __builtin_amdgcn_s_sleep(2);
-    }
-}
-
 // Folds row r of the walk's tables into the lockstep's lookup row of its step
 // (mn / mx, cleared beforehand; min / max over the copies by LDS atomics):
 // copy k is loaded by wave nwv-1-(k mod nwv), the last waves holding the
@@ -2538,6 +2668,7 @@ __global__ __launch_bounds__(1024) void k_ra_lane0(Dev d, const Ra0Prog *progs, 
     uint32_t rmn = 0xFFFFFFFFu, rmx = 0;
     // this workgroup's program: groups of 8 functions from fbase, L of them
     const Ra0Prog pg = progs[blockIdx.x];
+    if (d.cflag[pg.prg]) return;  // k_ra_serial's
     const uint32_t L = pg.L, maxsize = pg.rows, fbase = pg.fbase;  // steps: the table's rows
     const uint32_t *perm = perm_all + pg.poff;
     const uint32_t *gmin = gmin_all + pg.gbase, *gmax = gmax_all + pg.gbase;
@@ -2601,7 +2732,6 @@ __global__ __launch_bounds__(1024) void k_ra_lane0(Dev d, const Ra0Prog *progs, 
             const uint32_t j = f.j;
             if ((int32_t)i < (int32_t)f.size) {
                 ra0_cur<KEEP>(f, cur_rd, cur_rs1, cur_rs2, j);
-                xref_check_fields(d, fbase + 8u * j, f.start, f.size, f.ord, f.rs1, f.rs2);
                 const RaStep r = ra0_step(f);
                 if (f.own) {
                     ra0_lookups(Omin[c], Omax[c], r, j);
@@ -2813,7 +2943,7 @@ __global__ __launch_bounds__(1024) void k_ra_lane0(Dev d, const Ra0Prog *progs, 
 }
 
 // Exact fallback for programs in which two functions name the same virtual
-// register (see xref_note): the reference's allocation walk as written
+// register (ra_op): the reference's allocation walk as written
 // (rv_generator_avx.cpp:1041-1418 at one thread), one wave: steps in order,
 // groups of 8 functions in order within a step, the 8 functions of a group on
 // lanes 0-7.  Each group body reads its operands' states before any of its
@@ -2867,25 +2997,6 @@ __global__ __launch_bounds__(64) void k_ra_serial(Dev d, const Ra0Prog *progs, c
             for (uint32_t k = 0; k < 8; ++k) { if (ok && lane == k && (int32_t)r.rs1 > 63) d.sym[r.rs1 - 64u] = (uint16_t)r.r1r; __syncthreads(); }
             for (uint32_t k = 0; k < 8; ++k) { if (ok && lane == k && (int32_t)r.rs2 > 63) d.sym[r.rs2 - 64u] = (uint16_t)r.r2r; __syncthreads(); }
         }
-    }
-}
-
-// Every word naming a register that a function outside the register's own
-// function also names must belong to that same function (see xref_note).
-__global__ __launch_bounds__(256) void k_xref_check(Dev d) {
-    uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
-    if (i >= d.W0) return;
-    const uint4 w = d.w0_f4[i];
-    const uint32_t vs[3] = {w.x, w.y, w.z};
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        const uint32_t v = vs[k];
-        if (!((int32_t)v > 63) || v - 64u >= d.W0) continue;
-        const uint32_t t = d.xref[v - 64u];
-        if (!t) continue;
-        uint32_t lo = 0, hi = d.F;  // function of word i: last start <= i
-        while (hi - lo > 1) { uint32_t m = (lo + hi) / 2; if (d.fstarts[m] <= i) lo = m; else hi = m; }
-        if (lo + 1u != t) { atomicOr(d.flags, EF_XCONFLICT); d.cflag[prog_of(d.pf, d.P, lo)] = 1; }
     }
 }
 
@@ -2956,14 +3067,14 @@ __global__ __launch_bounds__(256) void k_ra_emit(Dev d) {
         ((int32_t)rdv > 63 && rdv - 64u >= d.W0)) { atomicOr(d.flags, EF_OOB); return; }
     if ((int32_t)r1 > 63) {
         const uint32_t e = d.sym[r1 - 64u];
-        const bool sw = (e >> 8) != 0;
+        const bool sw = (e & 0x100u) != 0;
         l1 = sw ? base : -1;
         st1 = spill(r1 - 64u);
         a1 = sw ? (((ins == 0xC0007053u) || (ins & 0x7Fu) == 0x53u) ? 37u : 5u) : (e & 0xFFu);
     }
     if ((int32_t)r2 > 63) {
         const uint32_t e = d.sym[r2 - 64u];
-        const bool sw = (e >> 8) != 0;
+        const bool sw = (e & 0x100u) != 0;
         l2 = sw ? base : -1;  // the reference tests its own, still -1, offset (D6)
         st2 = spill(r2 - 64u);
         a2 = sw ? (((ins & 0x7Fu) == 0x53u) ? 38u : 6u) : (e & 0xFFu);
@@ -2971,7 +3082,7 @@ __global__ __launch_bounds__(256) void k_ra_emit(Dev d) {
     const int32_t mo = base + (l1 > 0 ? 1 : 0) + (l2 > 0 ? 1 : 0);
     if ((int32_t)rdv > 63) {
         const uint32_t e = d.sym[rdv - 64u];
-        const bool sw = (e >> 8) != 0;
+        const bool sw = (e & 0x100u) != 0;
         rdo = sw ? mo + 1 : -1;
         std_ = spill(rdv - 64u);
         ad = e & 0xFFu;

@@ -3,8 +3,8 @@
     python -m ptilopsis_amd.tune [--out PATH]   (on the GPU; default ptilopsis_amd/tuning.json)
 
 Knobs (include/ptl.h, ptl_tune_set): the block size of each stage's per-node
-and per-word kernels (64, 128 or 256 threads) and the register-allocation
-walks' ring (4 or 8 entries).  Buckets: a compile's node count below 64Ki, 1Mi,
+and per-word kernels (64, 128 or 256 threads), the walk_ring knob (without
+effect) and small_programs.  Buckets: a compile's node count below 64Ki, 1Mi,
 8Mi, or larger.  For each bucket a representative workload is compiled with
 each value of each knob in turn (the others at their current choice), and the
 value with the smallest device time of the stage the knob affects is kept
@@ -34,7 +34,7 @@ KNOBS = {
     "block.optimize": ((64, 128, 256), 256, 3),
     "block.emit": ((64, 128, 256), 256, 4),
     "block.fix_jumps": ((64, 128, 256), 256, 5),
-    "walk_ring": ((4, 8), 4, 4),
+    "walk_ring": ((4, 8), 4, 4),  # without effect: the allocation walks keep their states in LDS
     # programs of at most 64 functions allocated by one wave each (1) or by the
     # walk and the lockstep (0)
     "small_programs": ((0, 1), 0, 4),

@@ -1,0 +1,69 @@
+"""Register allocation's walks at the sizes where their launch changes: programs
+around one group of 8 functions (k_ra_group), around 16 and 64 groups (the
+lockstep in one wave, one row of lanes or four; then a workgroup), alone with
+walk and lockstep overlapped and not, and together in one batch; and operands
+defined more words back than the walks' LDS rings hold.  Every output equals
+the oracle's."""
+import sys
+
+import numpy as np
+import pytest
+
+import oracle
+from ptilopsis_amd import parse_source, workloads as W
+
+pytestmark = pytest.mark.gpu
+OUT = ("words", "func_ids", "func_starts", "func_ends", "func_sizes")
+COUNTS = (1, 7, 8, 9, 16, 17, 127, 128, 129, 136, 137, 511, 512, 513, 520)
+
+
+def say(*a):
+    print(*a, file=sys.stderr, flush=True)
+
+
+def assert_same(gpu, ref, what):
+    for k in OUT:
+        assert np.array_equal(np.asarray(gpu[k]), np.asarray(ref[k])), (what, k)
+
+
+def program(nf):
+    return parse_source(W.program_source(0xA110 + nf, nf, min_stmts=1, max_stmts=9)[0])
+
+
+@pytest.mark.parametrize("nf", COUNTS)
+def test_gpu_alloc_function_counts(gpu_ctx, nf):
+    t = program(nf)
+    want = oracle.compile_tree(t)
+    try:
+        for on in (1, 0):
+            say("allocation,", nf, "functions, overlap", on)
+            gpu_ctx.set_overlap(on)
+            assert_same(gpu_ctx.compile(t), want, (nf, on))
+    finally:
+        gpu_ctx.set_overlap(1)
+
+
+def test_gpu_alloc_function_counts_batch(gpu_ctx):
+    trees = [program(nf) for nf in COUNTS]
+    say("allocation, one batch of", len(trees), "programs")
+    for nf, t, r in zip(COUNTS, trees, gpu_ctx.compile_batch(trees)):
+        assert_same(r, oracle.compile_tree(t), nf)
+
+
+@pytest.mark.parametrize("nf", [0, 9, 70])
+def test_gpu_alloc_far_operands(gpu_ctx, nf):
+    # wide balanced expressions: an operand's word is thousands of words back
+    base = dict(W.STRESS, min_args=2, max_args=4)
+    t = W.stress_program(0xFA4, 16000) if nf == 0 else parse_source(
+        W.program_source(0xFA4 + nf, nf, base=base, min_stmts=1, max_stmts=2, max_nest=1)[0])
+    o = oracle.Oracle(t)
+    o.run(4)
+    far = 0
+    for name in ("rs1", "rs2"):
+        a = o.get(name).astype(np.int64)
+        d = np.arange(a.shape[0]) - (a - 64)
+        far += int(((a > 63) & (a < 1 << 31) & (d > 255)).sum())
+    o.close()
+    assert far > 0
+    say("allocation, far operands", far, "in", t.n, "nodes")
+    assert_same(gpu_ctx.compile(t), oracle.compile_tree(t), nf)
