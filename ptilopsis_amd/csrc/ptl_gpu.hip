@@ -1496,8 +1496,8 @@ __global__ __launch_bounds__(256) void k_opt_iter(Dev d, uint32_t *changed) {
 //   OP_FAR1/2       rs1 / rs2 is defined more than OP_WINDOW words back: its
 //                   state is read from HBM
 //   OP_ZERO         an operand names the word's own register: its entry ends up 0
-constexpr uint32_t OP_WINDOW = 255;   // words back an operand's state is kept in LDS
-constexpr uint32_t OP_ROWS = 256;     // rows of the walks' LDS rings (a power of two above OP_WINDOW)
+constexpr uint32_t OP_ROWS = 256;     // rows of the walks' LDS rings (a power of two)
+constexpr uint32_t OP_WINDOW = 248;   // words back an operand's state is in LDS for sure (ring_low)
 constexpr uint32_t OP_CONST = 16;     // shift of the constant register
 constexpr uint32_t OP_ALLOC = 1u << 22, OP_SELF = 1u << 23, OP_FP = 1u << 24, OP_FAR1 = 1u << 25, OP_FAR2 = 1u << 26,
                    OP_ZERO = 1u << 27;
@@ -1681,6 +1681,11 @@ DEV uint32_t sm_or8(uint32_t v) {
 }
 DEV uint64_t sm_or8_64(uint64_t v) { return (uint64_t)sm_or8((uint32_t)v) | ((uint64_t)sm_or8((uint32_t)(v >> 32)) << 32); }
 
+// Ends a rarely taken branch that loads: without a wait of its own the compiler
+// waits where the branch joins, on every step, and since loads and stores share
+// the counter that wait is for every store and atomic before it too.
+DEV void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0F70); }  // vmcnt(0)
+
 // One step of a walk (rv_generator_avx.cpp:1062-1397) from the word's op, the
 // registers its operands are read in and the function's lifetime mask: the
 // registers freed (m; never x0), the one written (rdr, dm), the live registers
@@ -1704,13 +1709,34 @@ struct __attribute__((packed, aligned(4))) Op4 { uint32_t o[4]; };
 // Four consecutive states of a function's registers (any 2-byte alignment).
 struct __attribute__((packed, aligned(2))) Sym4 { uint64_t v; };
 
+// A function's ops in registers, 16 steps at a time: the load of the next 16 is
+// waited for once in 16 steps (its wait also waits for every store before it),
+// and `cur` moves down by four every four steps, so that it is indexed by
+// constants alone.
+struct OpBlock {
+    Op4 cur[4], nxt[4];
+    DEV void load(const uint32_t *ops, uint32_t i, uint32_t size) {
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) nxt[k] = *reinterpret_cast<const Op4 *>(ops + min(i + 4u * k, size));
+    }
+    DEV void step4(const uint32_t *ops, uint32_t i, uint32_t size) {  // before steps i .. i + 3 (i % 4 == 0)
+        if (i % 16u == 0) {
+#pragma unroll
+            for (uint32_t k = 0; k < 4; ++k) cur[k] = nxt[k];
+            load(ops, i + 16u, size);
+        } else {
+            cur[0] = cur[1]; cur[1] = cur[2]; cur[2] = cur[3];
+        }
+    }
+};
+
 // One function per lane.  The states of a function's last OP_ROWS words are in
 // an LDS ring of bytes, row = word mod OP_ROWS (a state here is just the
 // register the word's rd was given; it never changes); operands further back
 // are read from HBM.  Bound by the step's chain of instructions (latency; one
-// wave per SIMD): steps run four at a time, on one 16-byte load of ops issued
-// four steps ahead and one 8-byte store of states.  A 62-function program's
-// 4115 steps: 4.7 -> 1.7 ms against words compared and states looked up in a
+// wave per SIMD): steps run four at a time, on ops loaded 16 steps ahead and with
+// one 8-byte store of states.  A 62-function program's
+// 4115 steps: 4.7 -> 1.2 ms against words compared and states looked up in a
 // tagged cache at each step.
 __global__ __launch_bounds__(64) void k_ra_walk(Dev d, uint32_t *gmin_all, uint32_t *gmax_all, uint64_t stride,
                                                 uint32_t copies, unsigned long long *mask_all, uint64_t mstride,
@@ -1769,17 +1795,17 @@ __global__ __launch_bounds__(64) void k_ra_walk(Dev d, uint32_t *gmin_all, uint3
     for (int s = 32; s > 0; s >>= 1) { uint32_t o = __shfl_xor(wmax, s, 64); wmax = wmax > o ? wmax : o; }
     uint64_t life = 0x1Full;
     const uint32_t *ops = d.ops + start;
-    Op4 on = *reinterpret_cast<const Op4 *>(ops);
+    OpBlock ob;
+    ob.load(ops, 0, size);
     __syncthreads();
     for (uint32_t i0 = 0; i0 < wmax; i0 += 4) {
-        const Op4 ow = on;
-        on = *reinterpret_cast<const Op4 *>(ops + min(i0 + 4u, size));  // (past the end: never used)
+        ob.step4(ops, i0, size);
         uint32_t st[4];
 #pragma unroll
         for (uint32_t q = 0; q < 4; ++q) {
             const uint32_t i = i0 + q;
             const bool run = (int32_t)i < (int32_t)size;
-            const uint32_t op = run ? ow.o[q] : 0u;
+            const uint32_t op = run ? ob.cur[0].o[q] : 0u;
             const uint32_t d1 = op & 0xFFu, d2 = (op >> 8) & 0xFFu;
             uint32_t r1 = ring[((i - d1) & (OP_ROWS - 1u)) * 64u + lane];
             uint32_t r2 = ring[((i - d2) & (OP_ROWS - 1u)) * 64u + lane];
@@ -1789,6 +1815,7 @@ __global__ __launch_bounds__(64) void k_ra_walk(Dev d, uint32_t *gmin_all, uint3
                     const uint4 w = d.w0_f4[start + i];
                     if (op & OP_FAR1) r1 = d.sym[w.y - 64u] & 0xFFu;
                     if (op & OP_FAR2) r2 = d.sym[w.z - 64u] & 0xFFu;
+                    wait_loads();
                 }
             }
             const OpStep s = op_eval(op, r1, r2, life);
@@ -1930,118 +1957,172 @@ DEV uint32_t suffix_or(uint32_t v, uint32_t lane, uint32_t &all) {
     return x;
 }
 
-// One step i of this lane's function on its word's op.  ROWS 0: programs of one
-// group, 8 to a wave, lane 8s + k walking function k of program slot s (l0: k is
-// 0); the group's lookups of the step mark, except an entry whose register the
-// word names (its reset lands after a same-group mark).  ROWS 1, 4: lane j
-// walks the lane-0 function of group j of one program (of at most 16 or 64
-// groups), W being the registers looked up by the group's other functions.
-// There a lookup by a lower group is seen by the owner's operand read of the
-// same step (a flip), settled by re-evaluation until the flips are stable:
-// lane j's depend on the lanes below it alone, so this reaches the in-order
-// result; one by a higher group lands after the owner's own reset; and the last
-// group to write or free a register decides its entry.
-// The ring has a column per lane (RC of them), hold one per lane or, ROWS 0,
-// per program slot (HC).
-template <int ROWS, int RC, int HC>
+// Lookups of the step by the walked functions, as a lane-0 step takes them: per
+// lane a mask of the registers its group's other functions look up (W), or per
+// register the least and greatest group + 1 (mn, mx) with the mask of those
+// looked up at all (any).
+struct RaLooks { uint64_t W; const uint32_t *mn, *mx; uint64_t any; };
+
+// Register states of a lane's last words: an LDS ring of OP_ROWS rows, row = word
+// mod OP_ROWS, and one row more that takes the writes of lanes whose function has
+// ended (RC columns).  Rows leave it four at a time, before the steps of a block
+// of four from b overwrite them, so that HBM gets one 8-byte store per four steps
+// and no store for a change within the ring: words from ring_low(b) on are in
+// the ring, older ones in HBM.
+DEV uint32_t ring_low(uint32_t b, uint32_t size) {  // (the last block's for a function that has ended)
+    const uint32_t e = min(b, (size - 1u) & ~3u);
+    return e > OP_ROWS - 4u ? e - (OP_ROWS - 4u) : 0u;
+}
+template <int RC>
+DEV void ra_evict(const Dev &d, const RaL0 &f, const uint16_t *ring, uint32_t rc, uint32_t b) {
+    if (b >= OP_ROWS && (int32_t)b < (int32_t)f.size) {
+        uint32_t e[4];
+#pragma unroll
+        for (uint32_t q = 0; q < 4; ++q) e[q] = ring[((b + q) & (OP_ROWS - 1u)) * RC + rc];
+        reinterpret_cast<Sym4 *>(d.sym + f.start + (b - OP_ROWS))->v =
+            (uint64_t)(e[0] | (e[1] << 16)) | ((uint64_t)(e[2] | (e[3] << 16)) << 32);
+    }
+}
+// The states still in the ring, after the last step.
+template <int RC>
+DEV void ra_flush(const Dev &d, const RaL0 &f, const uint16_t *ring, uint32_t rc) {
+    if (f.size == 0) return;
+    for (uint32_t p = ring_low(f.size, f.size); p < f.size; ++p)
+        d.sym[f.start + p] = ring[(p & (OP_ROWS - 1u)) * RC + rc];
+}
+
+// One step i (of the block of four from b) of this lane's function on its word's
+// op (0 where it has ended).  MODE 0: programs of one group, 8 to a wave, lane
+// 8s + k walking function k of program slot s (l0: k is 0); the group's lookups
+// of the step mark, except an entry whose register the word names (its reset
+// lands after a same-group mark).  MODE 1, 4, 5: the wave's lanes walk the lane-0
+// functions of one program, the highest group in lane 0 (j: the lane's group), in
+// the first row of 16 lanes (1) or all four, the walk's lookups given by lane (1,
+// 4) or by register (5).
+// There a lookup by a lower group is seen by the owner's operand read of the same
+// step (a flip), settled by re-evaluation until the flips are stable: a group's
+// depend on the groups below it alone, so this reaches the in-order result.  A
+// lookup by a higher group lands after the owner's own reset, and the last group
+// to write or free a register decides its entry.
+// A wave runs alone on its SIMD, so a branch costs what ten instructions do
+// whether it is taken or not: everything but the rare cases (a state read from
+// HBM, a second mark, a flip) is straight-line, its writes going to a spare row or
+// entry where there is nothing to write.
+// hold has an entry per register (and one spare) and, MODE 0, program slot (HC).
+template <int MODE, int RC, int HC>
 DEV void ra_l0_step(const Dev &d, RaL0 &f, uint16_t *ring, uint32_t *hold, uint32_t rc, uint32_t hc, uint32_t lane,
-                    bool l0, uint32_t i, uint32_t opw, uint64_t W) {
-    const bool run = (int32_t)i < (int32_t)f.size;
-    const uint32_t op = run ? opw : 0u;
+                    bool l0, uint32_t j, uint32_t b, uint32_t i, uint32_t op, const RaLooks &lk) {
+    constexpr int ROWS = MODE > 1 ? 4 : 1;
+    constexpr int LAST = ROWS == 1 ? 15 : 63;
     const uint32_t d1 = op & 0xFFu, d2 = (op >> 8) & 0xFFu;
+    const uint32_t ws = (int32_t)i < (int32_t)f.size ? i & (OP_ROWS - 1u) : OP_ROWS;  // this word's row
     uint32_t p1 = i - d1, p2 = i - d2;
-    uint32_t e1 = ring[(p1 & (OP_ROWS - 1u)) * RC + rc], e2 = ring[(p2 & (OP_ROWS - 1u)) * RC + rc];
+    uint32_t w1 = d1 ? p1 & (OP_ROWS - 1u) : ws, w2 = d2 ? p2 & (OP_ROWS - 1u) : ws;
+    uint32_t e1 = ring[w1 * RC + rc], e2 = ring[w2 * RC + rc];
     e1 = d1 ? e1 : 0u; e2 = d2 ? e2 : 0u;
-    if (__ballot((op & (OP_FAR1 | OP_FAR2)) != 0)) {
+    const uint32_t rl = ring_low(b, f.size);
+    const bool far = __builtin_expect(__ballot((op & (OP_FAR1 | OP_FAR2)) != 0) != 0, 0);
+    if (far) {
         if (op & (OP_FAR1 | OP_FAR2)) {
             const uint4 w = d.w0_f4[f.start + i];
-            if (op & OP_FAR1) { p1 = w.y - 64u - f.start; e1 = d.sym[w.y - 64u]; }
-            if (op & OP_FAR2) { p2 = w.z - 64u - f.start; e2 = d.sym[w.z - 64u]; }
+            if (op & OP_FAR1) {
+                p1 = w.y - 64u - f.start;
+                if (p1 >= rl) { w1 = p1 & (OP_ROWS - 1u); e1 = ring[w1 * RC + rc]; } else e1 = d.sym[f.start + p1];
+            }
+            if (op & OP_FAR2) {
+                p2 = w.z - 64u - f.start;
+                if (p2 >= rl) { w2 = p2 & (OP_ROWS - 1u); e2 = ring[w2 * RC + rc]; } else e2 = d.sym[f.start + p2];
+            }
+            wait_loads();
         }
     }
+    // whether the entry of an operand's home holds it (no operand: home x0, which
+    // is never held)
     const uint32_t h1 = e1 >> 9, h2 = e2 >> 9;
     const uint32_t q1 = hold[h1 * HC + hc], q2 = hold[h2 * HC + hc];
+    uint32_t mn1 = 0, mn2 = 0, mx1 = 0, mx2 = 0;
+    if (MODE == 5) { mn1 = lk.mn[h1]; mn2 = lk.mn[h2]; mx1 = lk.mx[h1]; mx2 = lk.mx[h2]; }
     const uint32_t sr1 = (op & OP_FP) ? 37u : 5u, sr2 = (op & OP_FP) ? 38u : 6u;
     bool s1 = (e1 & 0x100u) != 0, s2 = (e2 & 0x100u) != 0;
     uint32_t r1 = s1 ? sr1 : e1 & 0x3Fu, r2 = s2 ? sr2 : e2 & 0x3Fu;
     OpStep s = op_eval(op, r1, r2, f.life);
-    // the entries holding the operands (no operand: home x0, which is never held)
     const uint64_t nb1 = q1 == p1 ? f.own & (1ull << h1) : 0ull, nb2 = q2 == p2 ? f.own & (1ull << h2) : 0ull;
     const uint64_t nb = nb1 | nb2;
     const bool self = (op & OP_SELF) != 0;
-    uint64_t mset, lost, won;
-    if (ROWS == 0) {
-        const uint64_t T = sm_or8_64(s.look);
-        lost = s.m | ((op & (OP_SELF | (63u << OP_CONST))) ? s.dm : 0ull);
-        won = self && l0 ? s.dm : 0ull;
-        mset = f.own & T & ~nb;
+    uint64_t T, high = 0;
+    if (MODE == 0) {
+        T = sm_or8_64(s.look);
     } else {
-        uint32_t tl = (uint32_t)(s.look | W), th = (uint32_t)((s.look | W) >> 32);
-        uint32_t il = scan_or<ROWS>(tl), ih = scan_or<ROWS>(th);  // inclusive over the lanes below
-        uint64_t high = 0;
-        if (__ballot(nb != 0)) {
-            bool f1 = false, f2 = false;
-            const bool w1 = s1, w2 = s2;  // swapped already
-            for (;;) {
-                const uint64_t low = (uint64_t)from_below<ROWS>(il) | ((uint64_t)from_below<ROWS>(ih) << 32);
-                const bool n1 = (nb1 & low) != 0, n2 = (nb2 & low) != 0;
-                const bool ch = (n1 != f1 && !w1) || (n2 != f2 && !w2);
-                if (!__ballot(ch)) break;
-                f1 = n1; f2 = n2;
-                s1 = w1 || f1; s2 = w2 || f2;
+        uint32_t tl = (uint32_t)s.look | (uint32_t)lk.W, th = (uint32_t)(s.look >> 32) | (uint32_t)(lk.W >> 32);
+        // looked up by a lower group (the lanes above); the walk's by register
+        const uint64_t wl = MODE == 5 ? (mn1 < j ? nb1 : 0ull) | (mn2 < j ? nb2 : 0ull) : 0ull;
+        uint32_t x;
+        uint64_t low = wl | (uint64_t)suffix_or<ROWS>(tl, lane, x) | ((uint64_t)suffix_or<ROWS>(th, lane, x) << 32);
+        bool n1 = (nb1 & low) != 0, n2 = (nb2 & low) != 0;
+        const bool z1 = s1, z2 = s2;  // swapped already
+        if (__ballot((n1 && !z1) || (n2 && !z2))) {
+            bool ch;
+            do {
+                const bool f1 = n1, f2 = n2;
+                s1 = z1 || f1; s2 = z2 || f2;
                 r1 = s1 ? sr1 : e1 & 0x3Fu; r2 = s2 ? sr2 : e2 & 0x3Fu;
                 s = op_eval(op, r1, r2, f.life);
-                tl = (uint32_t)(s.look | W); th = (uint32_t)((s.look | W) >> 32);
-                il = scan_or<ROWS>(tl); ih = scan_or<ROWS>(th);
-            }
-            uint32_t x;
-            high = (uint64_t)suffix_or<ROWS>(tl, lane, x);
-            high |= (uint64_t)suffix_or<ROWS>(th, lane, x) << 32;
+                tl = (uint32_t)s.look | (uint32_t)lk.W; th = (uint32_t)(s.look >> 32) | (uint32_t)(lk.W >> 32);
+                low = wl | (uint64_t)suffix_or<ROWS>(tl, lane, x) | ((uint64_t)suffix_or<ROWS>(th, lane, x) << 32);
+                n1 = (nb1 & low) != 0; n2 = (nb2 & low) != 0;
+                ch = (n1 != f1 && !z1) || (n2 != f2 && !z2);
+            } while (__ballot(ch));
         }
-        constexpr int LAST = ROWS == 1 ? 15 : 63;
-        const uint64_t T = (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)il, LAST) |
-                           ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)ih, LAST) << 32);
-        const uint64_t touch = s.m | ((op & (OP_SELF | (63u << OP_CONST))) ? s.dm : 0ull);
-        uint32_t al, ah;
-        uint64_t above = (uint64_t)suffix_or<ROWS>((uint32_t)touch, lane, al);
-        above |= (uint64_t)suffix_or<ROWS>((uint32_t)(touch >> 32), lane, ah) << 32;
-        lost = (uint64_t)al | ((uint64_t)ah << 32);
+        const uint32_t il = scan_or<ROWS>(tl), ih = scan_or<ROWS>(th);
+        high = (uint64_t)from_below<ROWS>(il) | ((uint64_t)from_below<ROWS>(ih) << 32);
+        if (MODE == 5) high |= (mx1 > j + 1u ? nb1 : 0ull) | (mx2 > j + 1u ? nb2 : 0ull);
+        T = (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)il, LAST) |
+            ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)ih, LAST) << 32);
+        if (MODE == 5) T |= lk.any;
+    }
+    // new marks: owned entries looked up whose mark does not stand yet
+    f.mk &= ~nb;
+    const uint64_t nm = f.own & ~f.mk & ((T & ~nb) | (high & nb));
+    f.mk |= nm;
+    const uint32_t mr = (uint32_t)__builtin_ctzll(nm | (1ull << 63));
+    const uint32_t mp = hold[mr * HC + hc];
+    // the registers written or freed: by any lane, by a higher group
+    const uint64_t touch = s.m | ((op & (OP_SELF | (63u << OP_CONST))) ? s.dm : 0ull);
+    uint64_t lost, won;
+    if (MODE == 0) {
+        lost = touch;
+        won = self && l0 ? s.dm : 0ull;
+    } else {
+        const uint32_t il = scan_or<ROWS>((uint32_t)touch), ih = scan_or<ROWS>((uint32_t)(touch >> 32));
+        const uint64_t above = (uint64_t)from_below<ROWS>(il) | ((uint64_t)from_below<ROWS>(ih) << 32);
+        lost = (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)il, LAST) |
+               ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)ih, LAST) << 32);
         won = self ? s.dm & ~above : 0ull;
-        mset = f.own & ((T & ~nb) | (high & nb));
     }
     // the step's commit: swapped operands take the register they were read
-    // through, and their flags are cleared
-    uint8_t *symb = reinterpret_cast<uint8_t *>(d.sym + f.start);
-    if (s1) {
-        const uint16_t st = (uint16_t)(r1 | (h1 << 9));
-        if (i - p1 <= OP_WINDOW) ring[(p1 & (OP_ROWS - 1u)) * RC + rc] = st;
-        d.sym[f.start + p1] = st;
+    // through, and their flags are cleared (an operand not swapped keeps its
+    // entry; without one, this word's row takes the write and its own after it)
+    const uint32_t st1 = s1 ? r1 | (h1 << 9) : e1, st2 = s2 ? r2 | (h2 << 9) : e2;
+    ring[w1 * RC + rc] = (uint16_t)st1;
+    ring[w2 * RC + rc] = (uint16_t)st2;
+    if (far) {
+        if ((op & OP_FAR1) && s1 && p1 < rl) d.sym[f.start + p1] = (uint16_t)st1;
+        if ((op & OP_FAR2) && s2 && p2 < rl) d.sym[f.start + p2] = (uint16_t)st2;
     }
-    if (s2) {
-        const uint16_t st = (uint16_t)(r2 | (h2 << 9));
-        if (i - p2 <= OP_WINDOW) ring[(p2 & (OP_ROWS - 1u)) * RC + rc] = st;
-        d.sym[f.start + p2] = st;
-    }
-    f.mk &= ~nb;
-    uint64_t nm = mset & ~f.mk;
-    f.mk |= mset;
-    // marks not standing yet: the flag byte of the states in the ring and in HBM
-    while (nm) {
-        const uint32_t r = (uint32_t)__builtin_ctzll(nm);
-        nm &= nm - 1;
-        const uint32_t p = hold[r * HC + hc];
-        const uint8_t fl = (uint8_t)(1u | (r << 1));
-        if (i - p <= OP_WINDOW) reinterpret_cast<uint8_t *>(ring)[2u * ((p & (OP_ROWS - 1u)) * RC + rc) + 1u] = fl;
-        symb[2u * p + 1u] = fl;
-    }
-    if (run) {
-        const uint32_t st = self ? ((op & OP_ZERO) ? 0u : s.rdr) | (s.rdr << 9) : 0u;
-        ring[(i & (OP_ROWS - 1u)) * RC + rc] = (uint16_t)st;
-        if (self) {
-            d.sym[f.start + i] = (uint16_t)st;
-            if (ROWS || l0) hold[s.rdr * HC + hc] = i;
+    // the mark of the first marked entry; the flag byte of its state
+    uint8_t *rb = reinterpret_cast<uint8_t *>(ring);
+    const bool inr = nm != 0 && mp >= rl;
+    rb[2u * ((inr ? mp & (OP_ROWS - 1u) : OP_ROWS) * RC + rc) + 1u] = (uint8_t)(1u | (mr << 1));
+    if (__builtin_expect(__ballot((nm & (nm - 1)) != 0 || (nm != 0 && !inr)) != 0, 0)) {
+        for (uint64_t m = nm; m; m &= m - 1) {
+            const uint32_t r = (uint32_t)__builtin_ctzll(m), p = hold[r * HC + hc];
+            const uint8_t fl = (uint8_t)(1u | (r << 1));
+            if (p >= rl) rb[2u * ((p & (OP_ROWS - 1u)) * RC + rc) + 1u] = fl;
+            else reinterpret_cast<uint8_t *>(d.sym + f.start)[2u * p + 1u] = fl;
         }
     }
+    ring[ws * RC + rc] = (uint16_t)(self ? ((op & OP_ZERO) ? 0u : s.rdr) | (s.rdr << 9) : 0u);
+    hold[(won ? s.rdr : 64u) * HC + hc] = i;
     f.life = s.life;
     f.own = (f.own & ~lost) | won;
     f.mk &= ~lost;
@@ -2052,11 +2133,11 @@ DEV void ra_l0_step(const Dev &d, RaL0 &f, uint16_t *ring, uint32_t *hold, uint3
 // register_state.  One wave holds 8 such programs.  The first `solo` programs
 // of the list (the longest) have a wave each, in slot 0, so that no other
 // program's rarer paths (a mark, a state read from HBM) hold up their steps.
-// Latency bound: 1.5 -> 0.58 us a step alone in a wave (a function of 35k words,
-// 52 -> 22 ms).
+// Latency bound: 1.5 -> 0.59 us a step alone in a wave (a function of 35k words,
+// 52 -> 21 ms).
 __global__ __launch_bounds__(64) void k_ra_group(Dev d, const uint32_t *plist, uint32_t np, uint32_t solo) {
-    __shared__ uint16_t ring[OP_ROWS * 64];
-    __shared__ uint32_t hold[64 * 8];
+    __shared__ uint16_t ring[(OP_ROWS + 1) * 64];
+    __shared__ uint32_t hold[65 * 8];
     const uint32_t lane = threadIdx.x, slot = lane >> 3, k = lane & 7u;
     const uint32_t pi = blockIdx.x < solo ? (slot == 0 ? blockIdx.x : np) : solo + (blockIdx.x - solo) * 8u + slot;
     const uint32_t prg = pi < np ? plist[pi] : 0xFFFFFFFFu;
@@ -2068,72 +2149,106 @@ __global__ __launch_bounds__(64) void k_ra_group(Dev d, const uint32_t *plist, u
     uint32_t wmax = f.size;
     for (int s = 32; s > 0; s >>= 1) { uint32_t o = __shfl_xor(wmax, s, 64); wmax = wmax > o ? wmax : o; }
     const uint32_t *ops = d.ops + f.start;
-    Op4 on = *reinterpret_cast<const Op4 *>(ops);
+    const RaLooks none{0, nullptr, nullptr, 0};
+    OpBlock ob;
+    ob.load(ops, 0, f.size);
     __syncthreads();
     for (uint32_t i = 0; i < wmax; i += 4) {
-        const Op4 ow = on;
-        on = *reinterpret_cast<const Op4 *>(ops + min(i + 4u, f.size));  // (past the end: never used)
+        ob.step4(ops, i, f.size);
+        ra_evict<64>(d, f, ring, lane, i);
 #pragma unroll
-        for (uint32_t q = 0; q < 4; ++q)
-            ra_l0_step<0, 64, 8>(d, f, ring, hold, lane, slot, lane, k == 0, i + q, ow.o[q], 0ull);
+        for (uint32_t q = 0; q < 4; ++q) {
+            const uint32_t op = (int32_t)(i + q) < (int32_t)f.size ? ob.cur[0].o[q] : 0u;
+            ra_l0_step<0, 64, 8>(d, f, ring, hold, lane, slot, lane, k == 0, 0u, i, i + q, op, none);
+        }
     }
+    ra_flush<64>(d, f, ring, lane);
 }
 
 // The lane-0 functions of a program of 2 to 16 (ROWS 1) or 64 (ROWS 4) groups,
 // in step lockstep on one wave: what the groups exchange in a step goes through
-// DPP scans of 64-bit register masks, so a step has no barrier.  The walk's
-// lookups of a step are one mask per group, loaded two blocks of four steps
-// ahead.  Bound by the chain of a step's instructions (latency): 5.4 -> 0.8 us a
-// step for 8 groups, against a workgroup exchanging lookups through LDS atomics
-// and barriers with its states in HBM.
+// ballots and DPP scans of 64-bit register masks, so a step has no barrier.  A
+// second wave fetches the ops and the walk's lookups (one mask per group and
+// step) into LDS, RA0_FETCH steps ahead: the stepping wave then waits for no
+// load, and so for none of its own stores either (they share a counter).
+// Bound by the chain of a step's instructions (latency): 5.4 -> 0.53 us a step
+// for 8 groups, against a workgroup exchanging lookups through LDS atomics and
+// barriers with its states in HBM; 0.8 us with the loads in the stepping wave.
+constexpr uint32_t RA0_FETCH = 16;
 template <int ROWS>
-__global__ __launch_bounds__(64) void k_ra_lane0_wave(Dev d, const Ra0Prog *progs, const unsigned long long *mask_all,
-                                                      uint64_t mstride, uint32_t mcopies, const uint32_t *done,
-                                                      const uint32_t *need) {
+__global__ __launch_bounds__(128) void k_ra_lane0_wave(Dev d, const Ra0Prog *progs, const unsigned long long *mask_all,
+                                                       uint64_t mstride, uint32_t mcopies, const uint32_t *done,
+                                                       const uint32_t *need) {
     constexpr int NL = ROWS == 1 ? 16 : 64;
-    __shared__ uint16_t ring[OP_ROWS * NL];
-    __shared__ uint32_t hold[64 * NL];
-    const uint32_t lane = threadIdx.x, col = lane % NL;
+    __shared__ uint16_t ring[(OP_ROWS + 1) * NL];
+    __shared__ uint32_t hold[65];
+    __shared__ uint32_t fop[2][RA0_FETCH][NL];
+    __shared__ unsigned long long fw[2][RA0_FETCH][NL];
+    const uint32_t lane = threadIdx.x & 63u, col = lane % NL;
+    const bool fetch = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) != 0;
     const Ra0Prog pg = progs[blockIdx.x];
     if (d.cflag[pg.prg]) return;  // k_ra_serial's
-    if (pg.L > (uint32_t)NL) { if (lane == 0) atomicOr(d.flags, EF_OOB); return; }
+    if (pg.L > (uint32_t)NL) { if (threadIdx.x == 0) atomicOr(d.flags, EF_OOB); return; }
     const bool act = lane < pg.L;
-    RaL0 f{act ? d.fstarts[pg.fbase + 8u * lane] : 0u, act ? d.fsizes[pg.fbase + 8u * lane] : 0u, 0x1Full, 0, 0};
+    const uint32_t j = act ? pg.L - 1u - lane : 0u;  // the lane's group
+    RaL0 f{act ? d.fstarts[pg.fbase + 8u * j] : 0u, act ? d.fsizes[pg.fbase + 8u * j] : 0u, 0x1Full, 0, 0};
     const uint32_t rows = pg.rows;
-    const uint32_t *pdone = done && pg.cbase != RA0_NOPUB ? done + pg.cbase : nullptr;
-    const uint32_t *pneed = pdone ? need + pg.cbase : nullptr;
-    const unsigned long long *mtab = mask_all + pg.gbase + (act ? lane : 0u);
-    const uint64_t m1 = mcopies > 1 ? mstride : 0u;
-    bool wok = true;  // the walk's rows still arrive
-    // rows i .. i + 3 of the walk's masks (both copies), once published
-    struct Rows { unsigned long long a[4], b[4]; };
-    auto load_rows = [&](uint32_t i) {
-        Rows r;
-        if (pdone && i < rows && i % WALK_PUB == 0) ra0_wait(d, pdone, pneed, i / WALK_PUB, wok);
+    if (fetch) {
+        const uint32_t *pdone = done && pg.cbase != RA0_NOPUB ? done + pg.cbase : nullptr;
+        const uint32_t *pneed = pdone ? need + pg.cbase : nullptr;
+        const unsigned long long *mtab = mask_all + pg.gbase + j;
+        const uint64_t m1 = mcopies > 1 ? mstride : 0u;
+        bool wok = true;  // the walk's rows still arrive
+        for (uint32_t i = 0;; i += RA0_FETCH) {  // steps i .. i + RA0_FETCH - 1, zeros past the last row
+            if (i < rows) {
+                const uint32_t b = (i / RA0_FETCH) & 1u;
+                if (pdone && i % WALK_PUB == 0) ra0_wait(d, pdone, pneed, i / WALK_PUB, wok);
+                Op4 o[RA0_FETCH / 4];
+                unsigned long long w0[RA0_FETCH], w1[RA0_FETCH];
 #pragma unroll
-        for (uint32_t q = 0; q < 4; ++q) {
-            const uint64_t e = (uint64_t)min(i + q, rows - 1u) * pg.L;
-            r.a[q] = mtab[e];
-            r.b[q] = mtab[m1 + e];
-        }
-        return r;
-    };
-    auto load_ops = [&](uint32_t i) { return *reinterpret_cast<const Op4 *>(d.ops + f.start + min(i, f.size)); };
-    Rows wa = load_rows(0), wb = load_rows(4);
-    Op4 oa = load_ops(0), ob = load_ops(4);
-    __syncthreads();
-    for (uint32_t i = 0; i < rows; i += 4) {
-        const Rows w = wa;
-        const Op4 o = oa;
-        wa = wb; oa = ob;
-        wb = load_rows(i + 8u);
-        ob = load_ops(i + 8u);
+                for (uint32_t k = 0; k < RA0_FETCH / 4; ++k)
+                    o[k] = *reinterpret_cast<const Op4 *>(d.ops + f.start + min(i + 4u * k, f.size));
 #pragma unroll
-        for (uint32_t q = 0; q < 4; ++q) {
-            const uint64_t W = act && i + q < rows ? w.a[q] | w.b[q] : 0ull;
-            ra_l0_step<ROWS, NL, NL>(d, f, ring, hold, col, col, lane, true, i + q, o.o[q], W);
+                for (uint32_t k = 0; k < RA0_FETCH; ++k) {
+                    const uint64_t e = (uint64_t)min(i + k, rows - 1u) * pg.L;
+                    w0[k] = mtab[e];
+                    w1[k] = mtab[m1 + e];
+                }
+                if (lane < (uint32_t)NL) {
+#pragma unroll
+                    for (uint32_t k = 0; k < RA0_FETCH; ++k) {
+                        fop[b][k][col] = (int32_t)(i + k) < (int32_t)f.size ? o[k / 4].o[k % 4] : 0u;
+                        fw[b][k][col] = act && i + k < rows ? w0[k] | w1[k] : 0ull;
+                    }
+                }
+            }
+            lds_barrier();
+            if (i >= rows) break;
         }
+        return;
     }
+    lds_barrier();  // the first steps are in
+    for (uint32_t i0 = 0; i0 < rows; i0 += RA0_FETCH) {
+        const uint32_t b = (i0 / RA0_FETCH) & 1u;
+        uint32_t op = fop[b][0][col];
+        unsigned long long W = fw[b][0][col];
+        for (uint32_t k = 0; k < RA0_FETCH; k += 4) {
+            ra_evict<NL>(d, f, ring, col, i0 + k);
+#pragma unroll
+            for (uint32_t q = 0; q < 4; ++q) {
+                // the next step's op and lookups, read a step ahead
+                const uint32_t kn = (k + q + 1u) % RA0_FETCH;
+                const uint32_t opn = fop[b][kn][col];
+                const unsigned long long Wn = fw[b][kn][col];
+                ra_l0_step<ROWS, NL, 1>(d, f, ring, hold, col, 0u, lane, true, j, i0 + k, i0 + k + q,
+                                        lane < (uint32_t)NL ? op : 0u,
+                                        RaLooks{lane < (uint32_t)NL ? W : 0ull, nullptr, nullptr, 0});
+                op = opn; W = Wn;
+            }
+        }
+        lds_barrier();  // the next steps are in
+    }
+    ra_flush<NL>(d, f, ring, col);
 }
 
 // ============================================================ small programs
@@ -2940,6 +3055,443 @@ __global__ __launch_bounds__(1024) void k_ra_lane0(Dev d, const Ra0Prog *progs, 
         for (int q = 0; q < PER; ++q)
             if ((int32_t)(i + 1) < (int32_t)fn[q].size) fn[q].nw = ra0_word(d, fn[q], i + 2);
     }
+}
+
+// The lane-0 functions of a program of more than RA0_WAVE_GROUPS groups, in step
+// lockstep on one workgroup.  Lanes hold functions in group order, 64 to a
+// wave slot (slot k on wave k mod the computing waves, PER slots a wave at
+// most), so what a step exchanges between groups is an OR over the lanes below
+// or above within a slot (DPP) and one pair of 64-bit masks per slot through
+// LDS: the registers looked up and the ones written or freed.  A step takes one
+// barrier, and one more for each round in which flips are settled across
+// slots; a single slot settles without.  Every RA0_PACK steps the functions
+// still running (or still holding a snapshot entry) are packed into as few
+// slots as they fit, through memory, and waves left without one end; the LDS
+// ring of states gets as many rows as the slots leave room for, reloaded from
+// HBM.  The last wave only fetches the walk's table rows (the fold of their
+// copies), four to eight steps ahead of use.
+//
+// Once one slot is left it steps as k_ra_lane0_wave does.
+// Bound by the chain of a step's instructions and barriers (latency), and while
+// more than about 500 functions run by instruction issue on the one compute unit.
+// 157 groups, 5267 steps: 19.0 -> 5.7 ms; 2500 groups, 5658 steps: 24.1 -> 21.5 ms,
+// against lookups exchanged by LDS atomics with the states in HBM.
+//
+// States in the ring are bytes: register | swapped << 6 | 0x80 when the register
+// is not the home any more (the home is then read from HBM).
+constexpr uint32_t RA0_PACK = 64;
+constexpr uint32_t RA0_WROWS = 16;         // walk rows in LDS
+constexpr uint32_t RA0_RING_MAX = 131072;  // bytes of ring at most (160 KB of LDS per compute unit)
+struct Ra0Tot { unsigned long long look, touch; };  // look bit 0 (x0 is never looked up): the slot's flag
+struct Ra0Move { uint32_t j, start, size, pad; uint64_t life, own, mk; };
+
+template <int PER>
+__global__ __launch_bounds__(1024) void k_ra_lane0_wg(Dev d, const Ra0Prog *progs, const uint32_t *gmin_all,
+                                                      const uint32_t *gmax_all, const uint32_t *done,
+                                                      const uint32_t *need, uint32_t copies, uint64_t stride,
+                                                      Ra0Move *move_all, uint32_t ring_bytes) {
+    extern __shared__ __align__(16) uint8_t wg_ring[];
+    __shared__ Ra0Tot tot[2][64], settle[2][64];
+    __shared__ uint32_t Wmn[RA0_WROWS][64], Wmx[RA0_WROWS][64];
+    __shared__ unsigned long long Wany[RA0_WROWS];
+    __shared__ uint32_t hold[65], cnt[64];
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const uint32_t CW = (blockDim.x >> 6) - 1u;  // computing waves
+    const bool helper = wave == CW;
+    const Ra0Prog pg = progs[blockIdx.x];
+    if (d.cflag[pg.prg]) return;  // k_ra_serial's
+    const uint32_t steps = pg.rows;
+    uint32_t NW = (pg.L + 63u) / 64u;
+    if (NW > 64u || NW > CW * PER) { if (threadIdx.x == 0) atomicOr(d.flags, EF_OOB); return; }
+    if (!helper && wave >= NW) return;  // (ended waves count as arrived at every barrier)
+    const uint32_t *gmin = gmin_all + pg.gbase, *gmax = gmax_all + pg.gbase;
+    const uint32_t *pdone = done && pg.cbase != RA0_NOPUB ? done + pg.cbase : nullptr;
+    const uint32_t *pneed = pdone ? need + pg.cbase : nullptr;
+    Ra0Move *mv = move_all + pg.poff;
+    uint32_t slots = NW * 64u, rm;  // ring: rows rm + 1 of `slots` bytes
+    auto ring_rows = [&]() {
+        uint32_t r = OP_ROWS;
+        while (r > 1u && r * slots > ring_bytes) r >>= 1;
+        return r;
+    };
+    rm = ring_rows() - 1u;
+    struct Fn { uint32_t j, start, size, pr; uint64_t life, own, mk; Op4 cur, nxt; };
+    // packing at step i: the slots left, and where a slot's functions go
+    auto pack_count = [&](uint32_t &before) {
+        before = lane < NW ? cnt[lane] : 0u;  // inclusive over the slots
+        for (uint32_t o = 1; o < 64; o <<= 1) {
+            const uint32_t u = (uint32_t)__shfl_up((int)before, o, 64);
+            if (lane >= o) before += u;
+        }
+        return (uint32_t)__builtin_amdgcn_readlane((int)before, 63);
+    };
+    // the totals of every slot, one per lane
+    auto totals = [&](const Ra0Tot *t) {
+        Ra0Tot r{0, 0};
+        if (lane < NW) r = t[lane];
+        return r;
+    };
+    if (helper) {
+        // four rows at a time, their loads issued four steps before they are
+        // folded and eight before the first is used; the barriers are the
+        // computing waves'
+        bool wok = true;  // the walk's rows still arrive
+        uint32_t a[4][RA0_MAXCOPIES], b[4][RA0_MAXCOPIES];
+        auto load4 = [&](uint32_t r) {
+            if (pdone && r < steps && r % WALK_PUB == 0) ra0_wait(d, pdone, pneed, r / WALK_PUB, wok);
+#pragma unroll
+            for (uint32_t y = 0; y < 4; ++y) {
+                const uint64_t e = (uint64_t)min(r + y, steps - 1u) * 64u + lane;
+#pragma unroll
+                for (uint32_t k = 0; k < RA0_MAXCOPIES; ++k) {
+                    const uint64_t o = (k < copies ? k : 0u) * stride + e;
+                    a[y][k] = gmin[o]; b[y][k] = gmax[o];
+                }
+            }
+        };
+        auto put4 = [&](uint32_t r) {
+#pragma unroll
+            for (uint32_t y = 0; y < 4; ++y) {
+                uint32_t mn = a[y][0], mx = b[y][0];
+#pragma unroll
+                for (uint32_t k = 1; k < RA0_MAXCOPIES; ++k) { mn = min(mn, a[y][k]); mx = max(mx, b[y][k]); }
+                const uint32_t w = (r + y) % RA0_WROWS;
+                Wmn[w][lane] = mn; Wmx[w][lane] = mx;
+                const uint64_t any = __ballot(mx != 0);
+                if (lane == 0) Wany[w] = any;
+            }
+        };
+        load4(0); put4(0); load4(4);
+        __syncthreads();
+        uint32_t i = 0;
+        for (; i < steps; ++i) {
+            if (i % RA0_PACK == 0 && i) {
+                __syncthreads();
+                __syncthreads();
+                uint32_t before;
+                const uint32_t nn = max(1u, (pack_count(before) + 63u) / 64u);
+                if (nn < NW) {
+                    __syncthreads();
+                    NW = nn;
+                    __syncthreads();
+                    if (NW == 1u) break;
+                }
+            }
+            lds_barrier();
+            // rows i + 4 .. i + 7, over rows no wave reads any more
+            if (i % 4u == 0) { put4(i + 4u); load4(i + 8u); }
+            if (__ballot(totals(tot[i & 1u]).look & 1ull)) {
+                uint32_t r = 0;
+                do { lds_barrier(); } while (__ballot(totals(settle[r++ & 1u]).look & 1ull));
+            }
+        }
+        for (; i < steps; i += 4) {  // one slot left: a barrier per four steps
+            lds_barrier();
+            put4(i + 4u);
+            load4(i + 8u);
+        }
+        return;
+    }
+    Fn fn[PER];
+    auto ops_at = [&](const Fn &f, uint32_t i) { return *reinterpret_cast<const Op4 *>(d.ops + f.start + min(i, f.size)); };
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+        Fn &f = fn[q];
+        const uint32_t j = (wave + q * CW) * 64u + lane;
+        const bool act = j < pg.L;
+        f.j = j; f.pr = 0; f.life = 0x1Full; f.own = 0; f.mk = 0;
+        f.start = act ? d.fstarts[pg.fbase + 8u * j] : 0u;
+        f.size = act ? d.fsizes[pg.fbase + 8u * j] : 0u;
+        f.cur = ops_at(f, 0); f.nxt = ops_at(f, 4);
+    }
+    __syncthreads();
+    uint32_t i = 0;
+    for (; i < steps; ++i) {
+        if (i % RA0_PACK == 0 && i) {
+            // pack: functions still running or holding an entry keep their order
+            __syncthreads();  // every store of the steps before is done
+#pragma unroll
+            for (int q = 0; q < PER; ++q) {
+                const uint32_t ws = wave + q * CW;
+                if (ws >= NW) continue;
+                if (fn[q].pr) { hold[fn[q].pr] = i - 1u; fn[q].pr = 0; }
+                const uint64_t m = __ballot((int32_t)i < (int32_t)fn[q].size || fn[q].own != 0);
+                if (lane == 0) cnt[ws] = (uint32_t)__popcll(m);
+            }
+            __syncthreads();
+            uint32_t before;
+            const uint32_t all = pack_count(before);
+            const uint32_t nn = max(1u, (all + 63u) / 64u);
+            if (nn < NW) {
+#pragma unroll
+                for (int q = 0; q < PER; ++q) {
+                    const uint32_t ws = wave + q * CW;
+                    if (ws >= NW) continue;
+                    const Fn &f = fn[q];
+                    const bool keep = (int32_t)i < (int32_t)f.size || f.own != 0;
+                    const uint64_t m = __ballot(keep);
+                    const uint32_t b = ws ? (uint32_t)__builtin_amdgcn_readlane((int)before, (int)ws - 1) : 0u;
+                    const uint32_t k = b + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+                    if (keep) mv[k] = Ra0Move{f.j, f.start, f.size, 0u, f.life, f.own, f.mk};
+                }
+                __syncthreads();
+                NW = nn;
+                if (wave >= NW) return;
+                if (NW == 1u) {
+                    // one slot: its functions in reverse, the highest group in
+                    // lane 0, and the ring as ra_l0_step has it
+                    const Ra0Move r = lane < all ? mv[all - 1u - lane] : Ra0Move{0, 0, 0, 0, 0x1Full, 0, 0};
+                    Fn &f = fn[0];
+                    f.j = r.j; f.start = r.start; f.size = r.size; f.life = r.life; f.own = r.own; f.mk = r.mk;
+                    uint16_t *ring = reinterpret_cast<uint16_t *>(wg_ring);
+                    const uint32_t last = min(i, f.size);
+                    for (uint32_t p = last > OP_ROWS ? (last - OP_ROWS) & ~3u : 0u; p < last; p += 4) {
+                        const uint64_t v = reinterpret_cast<const Sym4 *>(d.sym + f.start + p)->v;
+#pragma unroll
+                        for (uint32_t y = 0; y < 4; ++y)
+                            if (p + y < last) ring[((p + y) & (OP_ROWS - 1u)) * 64u + lane] = (uint16_t)(v >> (16u * y));
+                    }
+                    __syncthreads();
+                    break;
+                }
+                slots = NW * 64u;
+                const uint32_t rows = ring_rows();
+                rm = rows - 1u;
+#pragma unroll
+                for (int q = 0; q < PER; ++q) {
+                    const uint32_t ws = wave + q * CW;
+                    if (ws >= NW) continue;
+                    Fn &f = fn[q];
+                    const uint32_t k = ws * 64u + lane;
+                    const Ra0Move r = k < all ? mv[k] : Ra0Move{0, 0, 0, 0, 0x1Full, 0, 0};
+                    f.j = r.j; f.start = r.start; f.size = r.size; f.life = r.life; f.own = r.own; f.mk = r.mk;
+                    f.cur = ops_at(f, i); f.nxt = ops_at(f, i + 4u);
+                    if ((int32_t)i < (int32_t)f.size)
+                        for (uint32_t p = i > rows ? i - rows : 0u; p < i; p += 4) {  // (all multiples of 4 but the rows below 4)
+                            const uint64_t v = reinterpret_cast<const Sym4 *>(d.sym + f.start + p)->v;
+#pragma unroll
+                            for (uint32_t y = 0; y < 4; ++y) {
+                                const uint32_t e = (uint32_t)(v >> (16u * y)) & 0xFFFFu, reg = e & 0x3Fu;
+                                wg_ring[((p + y) & rm) * slots + k] =
+                                    (uint8_t)(reg | (((e >> 8) & 1u) << 6) | (reg != (e >> 9) ? 0x80u : 0u));
+                            }
+                        }
+                }
+                __syncthreads();
+            }
+        }
+        const uint32_t c = i & 1u;
+        // a function's step fields between the barriers: its op, and packed the
+        // operand states e (7 bits each), homes h, flips f and whether the
+        // entry of its home holds the operand (b); the words defining them
+        struct Mid { uint32_t op, x, p1, p2; };
+        Mid md[PER];
+        bool has_nb[PER];
+        auto regs = [&](const Mid &m, uint32_t fl, uint32_t &r1, uint32_t &r2) {
+            const bool s1 = ((m.x >> 6) & 1u) || (fl & 1u), s2 = ((m.x >> 13) & 1u) || (fl & 2u);
+            r1 = s1 ? ((m.op & OP_FP) ? 37u : 5u) : m.x & 0x3Fu;
+            r2 = s2 ? ((m.op & OP_FP) ? 38u : 6u) : (m.x >> 7) & 0x3Fu;
+        };
+        auto touched = [&](const Mid &m, const OpStep &s) {
+            return s.m | ((m.op & (OP_SELF | (63u << OP_CONST))) ? s.dm : 0ull);
+        };
+        auto or64 = [&](uint64_t v) {  // OR over the wave, uniform
+            const uint32_t l = scan_or<4>((uint32_t)v), h = scan_or<4>((uint32_t)(v >> 32));
+            return (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)l, 63) |
+                   ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)h, 63) << 32);
+        };
+        {
+#pragma unroll
+            for (int q = 0; q < PER; ++q) {
+                const uint32_t ws = wave + q * CW;
+                has_nb[q] = false;
+                if (ws >= NW) continue;
+                Fn &f = fn[q];
+                Mid &m = md[q];
+                const uint32_t k = ws * 64u + lane;
+                m.op = (int32_t)i < (int32_t)f.size ? f.cur.o[0] : 0u;
+                f.cur.o[0] = f.cur.o[1]; f.cur.o[1] = f.cur.o[2]; f.cur.o[2] = f.cur.o[3];
+                const uint32_t d1 = m.op & 0xFFu, d2 = (m.op >> 8) & 0xFFu;
+                m.p1 = i - d1; m.p2 = i - d2;
+                uint32_t e1 = wg_ring[(m.p1 & rm) * slots + k], e2 = wg_ring[(m.p2 & rm) * slots + k];
+                e1 = d1 ? e1 : 0u; e2 = d2 ? e2 : 0u;
+                uint32_t h1 = e1 & 0x3Fu, h2 = e2 & 0x3Fu;
+                // operands older than the ring, or no longer in their home: from HBM
+                const bool o1 = (m.op & OP_FAR1) || d1 > rm || (e1 & 0x80u), o2 = (m.op & OP_FAR2) || d2 > rm || (e2 & 0x80u);
+                if (__ballot(o1 || o2)) {
+                    if (o1 || o2) {
+                        if (m.op & (OP_FAR1 | OP_FAR2)) {
+                            const uint4 w = d.w0_f4[f.start + i];
+                            if (m.op & OP_FAR1) m.p1 = w.y - 64u - f.start;
+                            if (m.op & OP_FAR2) m.p2 = w.z - 64u - f.start;
+                        }
+                        const uint32_t g1 = d.sym[f.start + (o1 ? m.p1 : 0u)], g2 = d.sym[f.start + (o2 ? m.p2 : 0u)];
+                        wait_loads();
+                        if (o1) { e1 = (g1 & 0x3Fu) | (((g1 >> 8) & 1u) << 6); h1 = g1 >> 9; }
+                        if (o2) { e2 = (g2 & 0x3Fu) | (((g2 >> 8) & 1u) << 6); h2 = g2 >> 9; }
+                    }
+                }
+                // (an entry won in the step before is not in hold yet)
+                const uint32_t q1 = h1 == f.pr ? i - 1u : hold[h1], q2 = h2 == f.pr ? i - 1u : hold[h2];
+                const uint32_t b1 = q1 == m.p1 && ((f.own >> h1) & 1u), b2 = q2 == m.p2 && ((f.own >> h2) & 1u);
+                m.x = (e1 & 0x7Fu) | ((e2 & 0x7Fu) << 7) | (h1 << 14) | (h2 << 20) | (b1 << 28) | (b2 << 29);
+                uint32_t r1, r2;
+                regs(m, 0u, r1, r2);
+                const OpStep s = op_eval(m.op, r1, r2, f.life);
+                has_nb[q] = __ballot(b1 | b2) != 0;
+                const uint64_t tl = or64(s.look), tt = or64(touched(m, s));
+                if (lane == 0) tot[c][ws] = Ra0Tot{tl | (has_nb[q] ? 1ull : 0ull), tt};
+            }
+        }
+        lds_barrier();
+#pragma unroll
+        for (int q = 0; q < PER; ++q)
+            if (fn[q].pr) { hold[fn[q].pr] = i - 1u; fn[q].pr = 0; }
+        Ra0Tot t = totals(tot[c]);
+        if (__ballot(t.look & 1ull)) {
+            // settle the flips: a slot's lanes against the slots below as last
+            // published, until no slot's totals change
+            for (uint32_t r = 0;; ++r) {
+                const uint32_t cl = scan_or<4>((uint32_t)t.look), ch = scan_or<4>((uint32_t)(t.look >> 32));
+                {
+#pragma unroll
+                    for (int q = 0; q < PER; ++q) {
+                        const uint32_t ws = wave + q * CW;
+                        if (ws >= NW) continue;
+                        Fn &f = fn[q];
+                        Mid &m = md[q];
+                        Ra0Tot nt{((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)t.look, (int)ws) |
+                                   ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(t.look >> 32), (int)ws) << 32)) & ~1ull,
+                                  (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)t.touch, (int)ws) |
+                                      ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(t.touch >> 32), (int)ws) << 32)};
+                        bool changed = false;
+                        if (has_nb[q]) {
+                            uint64_t below = 0;
+                            if (ws) below = (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)cl, (int)ws - 1) |
+                                            ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)ch, (int)ws - 1) << 32);
+                            const uint32_t h1 = (m.x >> 14) & 0x3Fu, h2 = (m.x >> 20) & 0x3Fu;
+                            const bool b1 = (m.x >> 28) & 1u, b2 = (m.x >> 29) & 1u;
+                            const bool wl1 = Wmn[i % RA0_WROWS][h1] < f.j, wl2 = Wmn[i % RA0_WROWS][h2] < f.j;
+                            uint32_t fl = (m.x >> 26) & 3u, r1, r2;
+                            OpStep s;
+                            for (;;) {
+                                regs(m, fl, r1, r2);
+                                s = op_eval(m.op, r1, r2, f.life);
+                                const uint64_t low = below |
+                                    (uint64_t)from_below<4>(scan_or<4>((uint32_t)s.look)) |
+                                    ((uint64_t)from_below<4>(scan_or<4>((uint32_t)(s.look >> 32))) << 32);
+                                const uint32_t nf = ((b1 && (wl1 || ((low >> h1) & 1u))) ? 1u : 0u) |
+                                                    ((b2 && (wl2 || ((low >> h2) & 1u))) ? 2u : 0u);
+                                const bool ch2 = nf != fl;
+                                fl = nf;
+                                if (!__ballot(ch2)) break;
+                            }
+                            m.x = (m.x & ~(3u << 26)) | (fl << 26);
+                            const uint64_t tl = or64(s.look), tt = or64(touched(m, s));
+                            changed = tl != nt.look || tt != nt.touch;
+                            nt.look = tl; nt.touch = tt;
+                        }
+                        if (lane == 0) settle[r & 1u][ws] = Ra0Tot{nt.look | (changed ? 1ull : 0ull), nt.touch};
+                    }
+                }
+                lds_barrier();
+                t = totals(settle[r & 1u]);
+                if (!__ballot(t.look & 1ull)) break;
+            }
+        }
+        // the step's end: every slot's totals are final
+        uint64_t T = or64(t.look) | Wany[i % RA0_WROWS];
+        T &= ~1ull;
+        uint32_t al, ah, ul, uh;
+        ul = suffix_or<4>((uint32_t)t.touch, lane, al);
+        uh = suffix_or<4>((uint32_t)(t.touch >> 32), lane, ah);
+        const uint64_t lost = (uint64_t)al | ((uint64_t)ah << 32);
+#pragma unroll
+        for (int q = 0; q < PER; ++q) {
+            const uint32_t ws = wave + q * CW;
+            if (ws >= NW) continue;
+            Fn &f = fn[q];
+            const Mid &m = md[q];
+            const uint32_t k = ws * 64u + lane;
+            const uint32_t fl = (m.x >> 26) & 3u;
+            uint32_t r1, r2, x;
+            regs(m, fl, r1, r2);
+            const OpStep s = op_eval(m.op, r1, r2, f.life);
+            const uint64_t touch = touched(m, s);
+            uint64_t above = (uint64_t)suffix_or<4>((uint32_t)touch, lane, x) |
+                             ((uint64_t)suffix_or<4>((uint32_t)(touch >> 32), lane, x) << 32);
+            above |= (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)ul, (int)ws) |
+                     ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)uh, (int)ws) << 32);
+            const bool run = (int32_t)i < (int32_t)f.size, self = (m.op & OP_SELF) != 0;
+            const uint32_t h1 = (m.x >> 14) & 0x3Fu, h2 = (m.x >> 20) & 0x3Fu;
+            uint64_t mset = f.own & T;
+            if (has_nb[q]) {
+                uint32_t yl, yh;
+                uint64_t high = (uint64_t)suffix_or<4>((uint32_t)s.look, lane, x) |
+                                ((uint64_t)suffix_or<4>((uint32_t)(s.look >> 32), lane, x) << 32);
+                yl = suffix_or<4>((uint32_t)t.look, lane, x);
+                yh = suffix_or<4>((uint32_t)(t.look >> 32), lane, x);
+                high |= (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)yl, (int)ws) |
+                        ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)yh, (int)ws) << 32);
+                const uint64_t nb1 = ((m.x >> 28) & 1u) ? 1ull << h1 : 0ull, nb2 = ((m.x >> 29) & 1u) ? 1ull << h2 : 0ull;
+                if (Wmx[i % RA0_WROWS][h1] > f.j + 1u) high |= nb1;
+                if (Wmx[i % RA0_WROWS][h2] > f.j + 1u) high |= nb2;
+                const uint64_t nb = nb1 | nb2;
+                mset = f.own & ((T & ~nb) | (high & nb));
+                f.mk &= ~nb;
+            }
+            const bool s1 = ((m.x >> 6) & 1u) || (fl & 1u), s2 = ((m.x >> 13) & 1u) || (fl & 2u);
+            if (s1) {
+                if (i - m.p1 <= rm) wg_ring[(m.p1 & rm) * slots + k] = (uint8_t)(r1 | 0x80u);
+                d.sym[f.start + m.p1] = (uint16_t)(r1 | (h1 << 9));
+            }
+            if (s2) {
+                if (i - m.p2 <= rm) wg_ring[(m.p2 & rm) * slots + k] = (uint8_t)(r2 | 0x80u);
+                d.sym[f.start + m.p2] = (uint16_t)(r2 | (h2 << 9));
+            }
+            uint64_t nm = mset & ~f.mk;
+            f.mk |= mset;
+            while (nm) {
+                const uint32_t r = (uint32_t)__builtin_ctzll(nm);
+                nm &= nm - 1;
+                const uint32_t p = hold[r];
+                if (i - p <= rm) wg_ring[(p & rm) * slots + k] |= 0x40u;
+                reinterpret_cast<uint8_t *>(d.sym + f.start)[2u * p + 1u] = (uint8_t)(1u | (r << 1));
+            }
+            const uint64_t won = self ? s.dm & ~above : 0ull;
+            if (run) {
+                const uint32_t reg = self && !(m.op & OP_ZERO) ? s.rdr : 0u;
+                wg_ring[(i & rm) * slots + k] = (uint8_t)(reg | (self && reg != s.rdr ? 0x80u : 0u));
+                if (self) d.sym[f.start + i] = (uint16_t)(reg | (s.rdr << 9));
+            }
+            f.life = s.life;
+            f.own = (f.own & ~lost) | won;
+            f.mk &= ~lost;
+            f.pr = won ? s.rdr : 0u;
+            if ((i & 3u) == 3u) { f.cur = f.nxt; f.nxt = ops_at(f, i + 5u); }
+        }
+    }
+    if (i >= steps) return;
+    // one slot left: its steps need no exchange with other waves
+    RaL0 f{fn[0].start, fn[0].size, fn[0].life, fn[0].own, fn[0].mk};
+    uint16_t *ring = reinterpret_cast<uint16_t *>(wg_ring);
+    const uint32_t *ops = d.ops + f.start;
+    OpBlock ob;
+    ob.load(ops, i, f.size);  // (i is a multiple of RA0_PACK)
+    for (; i < steps; i += 4) {
+        lds_barrier();  // the walk's rows of the four steps are in
+        ob.step4(ops, i, f.size);
+        ra_evict<64>(d, f, ring, lane, i);
+#pragma unroll
+        for (uint32_t q = 0; q < 4; ++q) {
+            const uint32_t r = (i + q) % RA0_WROWS;
+            const uint32_t op = (int32_t)(i + q) < (int32_t)f.size ? ob.cur[0].o[q] : 0u;
+            ra_l0_step<5, 64, 1>(d, f, ring, hold, lane, 0u, lane, true, fn[0].j, i, i + q, op,
+                                 RaLooks{0ull, Wmn[r], Wmx[r], i + q < steps ? Wany[r] : 0ull});
+        }
+    }
+    ra_flush<64>(d, f, ring, lane);
 }
 
 // Exact fallback for programs in which two functions name the same virtual

@@ -1,8 +1,9 @@
 """Register allocation's walks at the sizes where their launch changes: programs
 around one group of 8 functions (k_ra_group), around 16 and 64 groups (the
-lockstep in one wave, one row of lanes or four; then a workgroup), alone with
-walk and lockstep overlapped and not, and together in one batch; and operands
-defined more words back than the walks' LDS rings hold.  Every output equals
+lockstep in one wave, one row of lanes or four) and 256, 960 and 2880 groups (a
+workgroup of one slot of 64 groups a wave or three), alone with walk and lockstep
+overlapped and not, and together in one batch; and operands defined more words
+back than the walks' LDS rings hold.  Every output equals
 the oracle's."""
 import sys
 
@@ -37,6 +38,23 @@ def test_gpu_alloc_function_counts(gpu_ctx, nf):
     try:
         for on in (1, 0):
             say("allocation,", nf, "functions, overlap", on)
+            gpu_ctx.set_overlap(on)
+            assert_same(gpu_ctx.compile(t), want, (nf, on))
+    finally:
+        gpu_ctx.set_overlap(1)
+
+
+@pytest.mark.parametrize("nf", [2048, 2049, 7680, 7681, 23040, 23041])
+def test_gpu_alloc_group_classes(gpu_ctx, nf):
+    # a few long functions among short ones, so that slots empty and are packed
+    rng = np.random.default_rng(nf)
+    targets = np.where(rng.random(nf) < 0.02, 1500, 60).astype(np.uint32)
+    targets[[0, 8 * (nf // 16)]] = 4000
+    t = parse_source(W.program_source(0xA110 + nf, nf, targets)[0])
+    want = oracle.compile_tree(t)
+    try:
+        for on in (1, 0):
+            say("allocation,", nf, "functions,", t.n, "nodes, overlap", on)
             gpu_ctx.set_overlap(on)
             assert_same(gpu_ctx.compile(t), want, (nf, on))
     finally:
