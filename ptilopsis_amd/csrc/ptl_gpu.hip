@@ -1730,6 +1730,30 @@ struct OpBlock {
     }
 };
 
+// The same a step at a time: N loads of four ops ahead.
+template <int N>
+struct OpQueue {
+    Op4 cur[N], nxt[N];
+    DEV void load(const uint32_t *ops, uint32_t i, uint32_t size) {
+#pragma unroll
+        for (int k = 0; k < N; ++k) nxt[k] = *reinterpret_cast<const Op4 *>(ops + min(i + 4u * k, size));
+    }
+    DEV uint32_t next(const uint32_t *ops, uint32_t i, uint32_t size) {  // step i's op, from i % (4 * N) == 0 on
+        if (i % (4u * N) == 0) {
+#pragma unroll
+            for (int k = 0; k < N; ++k) cur[k] = nxt[k];
+            load(ops, i + 4u * N, size);
+        } else if (N > 1 && i % 4u == 0) {
+#pragma unroll
+            for (int k = 0; k + 1 < N; ++k) cur[k] = cur[k + 1];
+        }
+        const uint32_t op = cur[0].o[0];
+        cur[0].o[0] = cur[0].o[1]; cur[0].o[1] = cur[0].o[2]; cur[0].o[2] = cur[0].o[3];
+        return op;
+    }
+};
+
+
 // One function per lane.  The states of a function's last OP_ROWS words are in
 // an LDS ring of bytes, row = word mod OP_ROWS (a state here is just the
 // register the word's rd was given; it never changes); operands further back
@@ -3058,32 +3082,61 @@ __global__ __launch_bounds__(1024) void k_ra_lane0(Dev d, const Ra0Prog *progs, 
 }
 
 // The lane-0 functions of a program of more than RA0_WAVE_GROUPS groups, in step
-// lockstep on one workgroup.  Lanes hold functions in group order, 64 to a
-// wave slot (slot k on wave k mod the computing waves, PER slots a wave at
-// most), so what a step exchanges between groups is an OR over the lanes below
-// or above within a slot (DPP) and one pair of 64-bit masks per slot through
-// LDS: the registers looked up and the ones written or freed.  A step takes one
-// barrier, and one more for each round in which flips are settled across
-// slots; a single slot settles without.  Every RA0_PACK steps the functions
-// still running (or still holding a snapshot entry) are packed into as few
-// slots as they fit, through memory, and waves left without one end; the LDS
-// ring of states gets as many rows as the slots leave room for, reloaded from
-// HBM.  The last wave only fetches the walk's table rows (the fold of their
+// lockstep on one workgroup.  Lanes hold functions in group order, the highest
+// first, 64 to a wave slot (slot k on wave k mod the computing waves, PER slots
+// a wave at most), so what a step exchanges between groups is an OR over the
+// lanes below or above within a slot (DPP) and one pair of 64-bit masks per slot
+// through LDS: the registers looked up and the ones written or freed.
+//
+// A step takes one barrier.  Flips (ra_l0_step) are settled within the slot
+// before it, against the walk's lookups and the slot's own; a lane whose operand
+// none of them looks up says so (chk), and only where a lower slot turns out to
+// look it up do the slots settle together, at a barrier a round: the walk has
+// seven functions to each of these, so mostly it has looked the register up.
+//
+// Every RA0_PACK steps the functions still running (or still holding a snapshot
+// entry) are packed into as few slots as they fit, through memory, and waves
+// left without one end; the LDS ring of states gets as many rows as the slots
+// leave room for, reloaded from HBM.  One slot left steps as k_ra_lane0_wave
+// does.  The last wave only fetches the walk's table rows (the fold of their
 // copies), four to eight steps ahead of use.
 //
-// Once one slot is left it steps as k_ra_lane0_wave does.
-// Bound by the chain of a step's instructions and barriers (latency), and while
-// more than about 500 functions run by instruction issue on the one compute unit.
-// 157 groups, 5267 steps: 19.0 -> 5.7 ms; 2500 groups, 5658 steps: 24.1 -> 21.5 ms,
-// against lookups exchanged by LDS atomics with the states in HBM.
+// Bound by the chain of a step's instructions, LDS reads and the barrier
+// (latency), and with more than a slot per SIMD by instruction issue on the one
+// compute unit: 157 groups, 5267 steps: 19.0 -> 5.1 ms; 2500 groups, 5658 steps:
+// 24.1 -> 14.2 ms, against lookups exchanged by LDS atomics with the states in
+// HBM; 5.7 and 21.5 ms with a barrier more on nearly every step to settle flips.
 //
 // States in the ring are bytes: register | swapped << 6 | 0x80 when the register
-// is not the home any more (the home is then read from HBM).
+// is not the home (which matters only while the home's entry holds it, and is
+// then found among the few entries the lane owns).
 constexpr uint32_t RA0_PACK = 64;
 constexpr uint32_t RA0_WROWS = 16;         // walk rows in LDS
-constexpr uint32_t RA0_RING_MAX = 131072;  // bytes of ring at most (160 KB of LDS per compute unit)
-struct Ra0Tot { unsigned long long look, touch; };  // look bit 0 (x0 is never looked up): the slot's flag
+constexpr uint32_t RA0_RING_MAX = 147456;  // bytes of ring at most (160 KB of LDS per compute unit)
+struct Ra0Tot { unsigned long long look, touch; };  // look bit 0 (x0 is never looked up): changed in this round
 struct Ra0Move { uint32_t j, start, size, pad; uint64_t life, own, mk; };
+
+DEV uint64_t lane64(uint32_t lo, uint32_t hi, uint32_t l) {
+    return (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)lo, (int)l) |
+           ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)hi, (int)l) << 32);
+}
+
+// A function of k_ra_lane0_wg; pr: the entry it won in the step before (0: none),
+// not in hold yet.
+template <int N> struct WgFn { uint32_t j, start, size, pr; uint64_t life, own, mk; OpQueue<N> ops; };
+// Its step between the barriers: the op; packed, the operands' state bytes (8
+// bits each), homes (6 bits each, at 16 and 22), flips taken (28, 29) and whether
+// the homes' entries hold them (30, 31); the words defining them.
+struct WgMid { uint32_t op, x, p1, p2; };
+
+DEV void wg_regs(const WgMid &m, uint32_t fl, uint32_t &r1, uint32_t &r2) {
+    const bool s1 = ((m.x >> 6) & 1u) || (fl & 1u), s2 = ((m.x >> 14) & 1u) || (fl & 2u);
+    r1 = s1 ? ((m.op & OP_FP) ? 37u : 5u) : m.x & 0x3Fu;
+    r2 = s2 ? ((m.op & OP_FP) ? 38u : 6u) : (m.x >> 8) & 0x3Fu;
+}
+DEV uint64_t wg_touch(uint32_t op, const OpStep &s) {
+    return s.m | ((op & (OP_SELF | (63u << OP_CONST))) ? s.dm : 0ull);
+}
 
 template <int PER>
 __global__ __launch_bounds__(1024) void k_ra_lane0_wg(Dev d, const Ra0Prog *progs, const uint32_t *gmin_all,
@@ -3092,6 +3145,7 @@ __global__ __launch_bounds__(1024) void k_ra_lane0_wg(Dev d, const Ra0Prog *prog
                                                       Ra0Move *move_all, uint32_t ring_bytes) {
     extern __shared__ __align__(16) uint8_t wg_ring[];
     __shared__ Ra0Tot tot[2][64], settle[2][64];
+    __shared__ uint32_t chk[2][64];  // by register: step << 6 | slot of a holder that no lookup flips yet
     __shared__ uint32_t Wmn[RA0_WROWS][64], Wmx[RA0_WROWS][64];
     __shared__ unsigned long long Wany[RA0_WROWS];
     __shared__ uint32_t hold[65], cnt[64];
@@ -3108,29 +3162,33 @@ __global__ __launch_bounds__(1024) void k_ra_lane0_wg(Dev d, const Ra0Prog *prog
     const uint32_t *gmin = gmin_all + pg.gbase, *gmax = gmax_all + pg.gbase;
     const uint32_t *pdone = done && pg.cbase != RA0_NOPUB ? done + pg.cbase : nullptr;
     const uint32_t *pneed = pdone ? need + pg.cbase : nullptr;
-    Ra0Move *mv = move_all + pg.poff;
-    uint32_t slots = NW * 64u, rm;  // ring: rows rm + 1 of `slots` bytes
-    auto ring_rows = [&]() {
-        uint32_t r = OP_ROWS;
-        while (r > 1u && r * slots > ring_bytes) r >>= 1;
-        return r;
-    };
-    rm = ring_rows() - 1u;
-    struct Fn { uint32_t j, start, size, pr; uint64_t life, own, mk; Op4 cur, nxt; };
-    // packing at step i: the slots left, and where a slot's functions go
-    auto pack_count = [&](uint32_t &before) {
-        before = lane < NW ? cnt[lane] : 0u;  // inclusive over the slots
-        for (uint32_t o = 1; o < 64; o <<= 1) {
-            const uint32_t u = (uint32_t)__shfl_up((int)before, o, 64);
-            if (lane >= o) before += u;
-        }
-        return (uint32_t)__builtin_amdgcn_readlane((int)before, 63);
-    };
+    if (threadIdx.x < 128u) (&chk[0][0])[threadIdx.x] = 0xFFFFFFFFu;  // (two slots at least: those waves are there)
     // the totals of every slot, one per lane
     auto totals = [&](const Ra0Tot *t) {
         Ra0Tot r{0, 0};
         if (lane < NW) r = t[lane];
         return r;
+    };
+    // whether a holder that no lookup flips within its slot is looked up by a
+    // lower slot (a higher slot number): then the slots settle together
+    auto unsettled = [&](const Ra0Tot &t, uint32_t i) {
+        const uint32_t key = chk[i & 1u][lane];
+        bool any = false;
+        for (uint64_t z = __ballot((key >> 6) == (i & 0x3FFFFFFu)); z; z &= z - 1) {
+            const int r = __builtin_ctzll(z);
+            const uint32_t es = (uint32_t)__builtin_amdgcn_readlane((int)key, r) & 63u;
+            any = any || (__ballot((t.look >> r) & 1ull) >> es >> 1) != 0;
+        }
+        return any;
+    };
+    // packing at step i: the functions kept, inclusive over the slots
+    auto pack_count = [&](uint32_t &before) {
+        before = lane < NW ? cnt[lane] : 0u;
+        for (uint32_t o = 1; o < 64; o <<= 1) {
+            const uint32_t u = (uint32_t)__shfl_up((int)before, o, 64);
+            if (lane >= o) before += u;
+        }
+        return (uint32_t)__builtin_amdgcn_readlane((int)before, 63);
     };
     if (helper) {
         // four rows at a time, their loads issued four steps before they are
@@ -3181,7 +3239,7 @@ __global__ __launch_bounds__(1024) void k_ra_lane0_wg(Dev d, const Ra0Prog *prog
             lds_barrier();
             // rows i + 4 .. i + 7, over rows no wave reads any more
             if (i % 4u == 0) { put4(i + 4u); load4(i + 8u); }
-            if (__ballot(totals(tot[i & 1u]).look & 1ull)) {
+            if (unsettled(totals(tot[i & 1u]), i)) {
                 uint32_t r = 0;
                 do { lds_barrier(); } while (__ballot(totals(settle[r++ & 1u]).look & 1ull));
             }
@@ -3193,288 +3251,409 @@ __global__ __launch_bounds__(1024) void k_ra_lane0_wg(Dev d, const Ra0Prog *prog
         }
         return;
     }
-    Fn fn[PER];
-    auto ops_at = [&](const Fn &f, uint32_t i) { return *reinterpret_cast<const Op4 *>(d.ops + f.start + min(i, f.size)); };
-#pragma unroll
-    for (int q = 0; q < PER; ++q) {
-        Fn &f = fn[q];
-        const uint32_t j = (wave + q * CW) * 64u + lane;
-        const bool act = j < pg.L;
-        f.j = j; f.pr = 0; f.life = 0x1Full; f.own = 0; f.mk = 0;
-        f.start = act ? d.fstarts[pg.fbase + 8u * j] : 0u;
-        f.size = act ? d.fsizes[pg.fbase + 8u * j] : 0u;
-        f.cur = ops_at(f, 0); f.nxt = ops_at(f, 4);
-    }
-    __syncthreads();
-    uint32_t i = 0;
-    for (; i < steps; ++i) {
-        if (i % RA0_PACK == 0 && i) {
-            // pack: functions still running or holding an entry keep their order
-            __syncthreads();  // every store of the steps before is done
-#pragma unroll
-            for (int q = 0; q < PER; ++q) {
-                const uint32_t ws = wave + q * CW;
-                if (ws >= NW) continue;
-                if (fn[q].pr) { hold[fn[q].pr] = i - 1u; fn[q].pr = 0; }
-                const uint64_t m = __ballot((int32_t)i < (int32_t)fn[q].size || fn[q].own != 0);
-                if (lane == 0) cnt[ws] = (uint32_t)__popcll(m);
+    Ra0Move *mv = move_all + pg.poff;
+    // the ring: `rows` rows of `slots` bytes and a spare one, word i in row ri
+    uint32_t slots, rows, ri;
+    auto ring_shape = [&](uint32_t i) {
+        slots = NW * 64u;
+        rows = min(OP_ROWS, ring_bytes / slots - 1u);
+        ri = i % rows;
+    };
+    auto row_of = [&](uint32_t dist) { return ri >= dist ? ri - dist : ri + rows - dist; };  // dist <= rows
+    ring_shape(0);
+    // whether entry h of this lane holds word p (h: an operand's home), or for a
+    // state that left its home (odd) which entry does
+    auto home_of = [&](uint32_t e, uint32_t p, uint64_t own, uint32_t pr, uint32_t i) {
+        uint32_t h = 0;
+        if (e & 0x80u)
+            for (uint64_t m = own; m; m &= m - 1) {
+                const uint32_t r = (uint32_t)__builtin_ctzll(m);
+                if ((r == pr ? i - 1u : hold[r]) == p) h = r;
             }
-            __syncthreads();
-            uint32_t before;
-            const uint32_t all = pack_count(before);
-            const uint32_t nn = max(1u, (all + 63u) / 64u);
-            if (nn < NW) {
-#pragma unroll
-                for (int q = 0; q < PER; ++q) {
-                    const uint32_t ws = wave + q * CW;
-                    if (ws >= NW) continue;
-                    const Fn &f = fn[q];
-                    const bool keep = (int32_t)i < (int32_t)f.size || f.own != 0;
-                    const uint64_t m = __ballot(keep);
-                    const uint32_t b = ws ? (uint32_t)__builtin_amdgcn_readlane((int)before, (int)ws - 1) : 0u;
-                    const uint32_t k = b + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
-                    if (keep) mv[k] = Ra0Move{f.j, f.start, f.size, 0u, f.life, f.own, f.mk};
+        return (e & 0x80u) ? h : e & 0x3Fu;
+    };
+    // the first part of a function's step: its operands' states (ring column k)
+    auto operands = [&](uint32_t op, uint32_t i, uint32_t k, uint32_t start, uint64_t own, uint32_t pr, WgMid &m) {
+        m.op = op;
+        const uint32_t d1 = op & 0xFFu, d2 = (op >> 8) & 0xFFu;
+        m.p1 = i - d1; m.p2 = i - d2;
+        uint32_t e1 = wg_ring[row_of(min(d1, rows)) * slots + k], e2 = wg_ring[row_of(min(d2, rows)) * slots + k];
+        e1 = d1 ? e1 : 0u; e2 = d2 ? e2 : 0u;
+        // operands older than the ring: from HBM
+        const bool o1 = (op & OP_FAR1) || d1 >= rows, o2 = (op & OP_FAR2) || d2 >= rows;
+        if (__builtin_expect(__ballot(o1 || o2) != 0, 0)) {
+            if (o1 || o2) {
+                if (op & (OP_FAR1 | OP_FAR2)) {
+                    const uint4 w = d.w0_f4[start + i];
+                    if (op & OP_FAR1) m.p1 = w.y - 64u - start;
+                    if (op & OP_FAR2) m.p2 = w.z - 64u - start;
                 }
-                __syncthreads();
-                NW = nn;
-                if (wave >= NW) return;
-                if (NW == 1u) {
-                    // one slot: its functions in reverse, the highest group in
-                    // lane 0, and the ring as ra_l0_step has it
-                    const Ra0Move r = lane < all ? mv[all - 1u - lane] : Ra0Move{0, 0, 0, 0, 0x1Full, 0, 0};
-                    Fn &f = fn[0];
-                    f.j = r.j; f.start = r.start; f.size = r.size; f.life = r.life; f.own = r.own; f.mk = r.mk;
-                    uint16_t *ring = reinterpret_cast<uint16_t *>(wg_ring);
-                    const uint32_t last = min(i, f.size);
-                    for (uint32_t p = last > OP_ROWS ? (last - OP_ROWS) & ~3u : 0u; p < last; p += 4) {
-                        const uint64_t v = reinterpret_cast<const Sym4 *>(d.sym + f.start + p)->v;
-#pragma unroll
-                        for (uint32_t y = 0; y < 4; ++y)
-                            if (p + y < last) ring[((p + y) & (OP_ROWS - 1u)) * 64u + lane] = (uint16_t)(v >> (16u * y));
-                    }
-                    __syncthreads();
-                    break;
-                }
-                slots = NW * 64u;
-                const uint32_t rows = ring_rows();
-                rm = rows - 1u;
-#pragma unroll
-                for (int q = 0; q < PER; ++q) {
-                    const uint32_t ws = wave + q * CW;
-                    if (ws >= NW) continue;
-                    Fn &f = fn[q];
-                    const uint32_t k = ws * 64u + lane;
-                    const Ra0Move r = k < all ? mv[k] : Ra0Move{0, 0, 0, 0, 0x1Full, 0, 0};
-                    f.j = r.j; f.start = r.start; f.size = r.size; f.life = r.life; f.own = r.own; f.mk = r.mk;
-                    f.cur = ops_at(f, i); f.nxt = ops_at(f, i + 4u);
-                    if ((int32_t)i < (int32_t)f.size)
-                        for (uint32_t p = i > rows ? i - rows : 0u; p < i; p += 4) {  // (all multiples of 4 but the rows below 4)
-                            const uint64_t v = reinterpret_cast<const Sym4 *>(d.sym + f.start + p)->v;
-#pragma unroll
-                            for (uint32_t y = 0; y < 4; ++y) {
-                                const uint32_t e = (uint32_t)(v >> (16u * y)) & 0xFFFFu, reg = e & 0x3Fu;
-                                wg_ring[((p + y) & rm) * slots + k] =
-                                    (uint8_t)(reg | (((e >> 8) & 1u) << 6) | (reg != (e >> 9) ? 0x80u : 0u));
-                            }
-                        }
-                }
-                __syncthreads();
+                const uint32_t g1 = d.sym[start + (o1 ? m.p1 : 0u)], g2 = d.sym[start + (o2 ? m.p2 : 0u)];
+                wait_loads();
+                if (o1) e1 = (g1 & 0x3Fu) | (((g1 >> 8) & 1u) << 6) | ((g1 & 0x3Fu) != g1 >> 9 ? 0x80u : 0u);
+                if (o2) e2 = (g2 & 0x3Fu) | (((g2 >> 8) & 1u) << 6) | ((g2 & 0x3Fu) != g2 >> 9 ? 0x80u : 0u);
             }
         }
-        const uint32_t c = i & 1u;
-        // a function's step fields between the barriers: its op, and packed the
-        // operand states e (7 bits each), homes h, flips f and whether the
-        // entry of its home holds the operand (b); the words defining them
-        struct Mid { uint32_t op, x, p1, p2; };
-        Mid md[PER];
-        bool has_nb[PER];
-        auto regs = [&](const Mid &m, uint32_t fl, uint32_t &r1, uint32_t &r2) {
-            const bool s1 = ((m.x >> 6) & 1u) || (fl & 1u), s2 = ((m.x >> 13) & 1u) || (fl & 2u);
-            r1 = s1 ? ((m.op & OP_FP) ? 37u : 5u) : m.x & 0x3Fu;
-            r2 = s2 ? ((m.op & OP_FP) ? 38u : 6u) : (m.x >> 7) & 0x3Fu;
-        };
-        auto touched = [&](const Mid &m, const OpStep &s) {
-            return s.m | ((m.op & (OP_SELF | (63u << OP_CONST))) ? s.dm : 0ull);
-        };
-        auto or64 = [&](uint64_t v) {  // OR over the wave, uniform
-            const uint32_t l = scan_or<4>((uint32_t)v), h = scan_or<4>((uint32_t)(v >> 32));
-            return (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)l, 63) |
-                   ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)h, 63) << 32);
-        };
-        {
+        uint32_t h1 = e1 & 0x3Fu, h2 = e2 & 0x3Fu;
+        if (__builtin_expect(__ballot(((e1 | e2) & 0x80u) != 0) != 0, 0)) {
+            h1 = home_of(e1, m.p1, own, pr, i);
+            h2 = home_of(e2, m.p2, own, pr, i);
+        }
+        m.x = e1 | (e2 << 8) | (h1 << 16) | (h2 << 22);
+    };
+    // the second: commit and marks (new marks nm), and the word's own state
+    auto commit = [&](const WgMid &m, const OpStep &s, uint32_t r1, uint32_t r2, uint32_t i, uint32_t k, uint32_t start,
+                      bool run, uint64_t nm) {
+        const uint32_t fl = (m.x >> 28) & 3u, h1 = (m.x >> 16) & 0x3Fu, h2 = (m.x >> 22) & 0x3Fu;
+        const bool s1 = ((m.x >> 6) & 1u) || (fl & 1u), s2 = ((m.x >> 14) & 1u) || (fl & 2u);
+        if (__ballot(s1 || s2)) {
+            if (s1) {
+                if (i - m.p1 < rows) wg_ring[row_of(i - m.p1) * slots + k] = (uint8_t)(r1 | 0x80u);
+                d.sym[start + m.p1] = (uint16_t)(r1 | (h1 << 9));
+            }
+            if (s2) {
+                if (i - m.p2 < rows) wg_ring[row_of(i - m.p2) * slots + k] = (uint8_t)(r2 | 0x80u);
+                d.sym[start + m.p2] = (uint16_t)(r2 | (h2 << 9));
+            }
+        }
+        while (nm) {
+            const uint32_t r = (uint32_t)__builtin_ctzll(nm);
+            nm &= nm - 1;
+            const uint32_t p = hold[r];
+            if (i - p < rows) wg_ring[row_of(i - p) * slots + k] |= 0x40u;
+            reinterpret_cast<uint8_t *>(d.sym + start)[2u * p + 1u] = (uint8_t)(1u | (r << 1));
+        }
+        const bool self = (m.op & OP_SELF) != 0;
+        if (run) {
+            const uint32_t reg = self && !(m.op & OP_ZERO) ? s.rdr : 0u;
+            wg_ring[ri * slots + k] = (uint8_t)(reg | (self && reg != s.rdr ? 0x80u : 0u));
+            if (self) d.sym[start + i] = (uint16_t)(reg | (s.rdr << 9));
+        }
+    };
+    // packs the slots of fn[] (slot wave + q * CW in fn[q]) at step i; true when
+    // this wave goes on
+    auto pack = [&](auto &fn, uint32_t i) {
+        constexpr int N = (int)(sizeof(fn) / sizeof(fn[0]));
+        __syncthreads();  // every store of the steps before is done
+#pragma unroll
+        for (int q = 0; q < N; ++q) {
+            const uint32_t ws = wave + q * CW;
+            if (ws >= NW) continue;
+            if (fn[q].pr) { hold[fn[q].pr] = i - 1u; fn[q].pr = 0; }
+            const uint64_t m = __ballot((int32_t)i < (int32_t)fn[q].size || fn[q].own != 0);
+            if (lane == 0) cnt[ws] = (uint32_t)__popcll(m);
+        }
+        __syncthreads();
+        uint32_t before;
+        const uint32_t all = pack_count(before);
+        const uint32_t nn = max(1u, (all + 63u) / 64u);
+        if (nn >= NW) return true;
+#pragma unroll
+        for (int q = 0; q < N; ++q) {
+            const uint32_t ws = wave + q * CW;
+            if (ws >= NW) continue;
+            const auto &f = fn[q];
+            const bool keep = (int32_t)i < (int32_t)f.size || f.own != 0;
+            const uint64_t m = __ballot(keep);
+            const uint32_t b = ws ? (uint32_t)__builtin_amdgcn_readlane((int)before, (int)ws - 1) : 0u;
+            if (keep) mv[b + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] =
+                Ra0Move{f.j, f.start, f.size, 0u, f.life, f.own, f.mk};
+        }
+        __syncthreads();
+        NW = nn;
+        if (wave >= NW) return false;
+        ring_shape(i);
+#pragma unroll
+        for (int q = 0; q < N; ++q) {
+            const uint32_t ws = wave + q * CW;
+            if (ws >= NW) continue;
+            auto &f = fn[q];
+            const uint32_t k = ws * 64u + lane;
+            const Ra0Move r = k < all ? mv[k] : Ra0Move{0, 0, 0, 0, 0x1Full, 0, 0};
+            f.j = r.j; f.start = r.start; f.size = r.size; f.life = r.life; f.own = r.own; f.mk = r.mk;
+            f.ops.load(d.ops + f.start, i, f.size);
+            if (NW == 1u) {  // the ring as ra_l0_step has it, of functions that have ended too
+                uint16_t *ring = reinterpret_cast<uint16_t *>(wg_ring);
+                const uint32_t last = min(i, f.size);
+                for (uint32_t p = last > OP_ROWS ? (last - OP_ROWS) & ~3u : 0u; p < last; p += 4) {
+                    const uint64_t v = reinterpret_cast<const Sym4 *>(d.sym + f.start + p)->v;
+#pragma unroll
+                    for (uint32_t y = 0; y < 4; ++y)
+                        if (p + y < last) ring[((p + y) & (OP_ROWS - 1u)) * 64u + lane] = (uint16_t)(v >> (16u * y));
+                }
+            } else if ((int32_t)i < (int32_t)f.size) {
+                for (uint32_t p = (i > rows ? i - rows : 0u) & ~3u; p < i; p += 4) {
+                    const uint64_t v = reinterpret_cast<const Sym4 *>(d.sym + f.start + p)->v;
+#pragma unroll
+                    for (uint32_t y = 0; y < 4; ++y) {
+                        const uint32_t e = (uint32_t)(v >> (16u * y)) & 0xFFFFu, reg = e & 0x3Fu;
+                        if (i - (p + y) <= rows)
+                            wg_ring[((p + y) % rows) * slots + k] =
+                                (uint8_t)(reg | (((e >> 8) & 1u) << 6) | (reg != (e >> 9) ? 0x80u : 0u));
+                    }
+                }
+            }
+        }
+        __syncthreads();
+        return true;
+    };
+    auto next_row = [&]() { ri = ri + 1u == rows ? 0u : ri + 1u; };
+    uint32_t i = 0;
+    WgFn<4> f1[1];
+    if (PER > 1) {
+        // more slots than waves: each wave steps its slots one after the other,
+        // keeping of each between the barriers only a WgMid
+        WgFn<1> fn[PER];
+#pragma unroll
+        for (int q = 0; q < PER; ++q) {
+            WgFn<1> &f = fn[q];
+            const uint32_t k = (wave + q * CW) * 64u + lane;
+            const bool act = k < pg.L;
+            f.j = act ? pg.L - 1u - k : 0u; f.pr = 0; f.life = 0x1Full; f.own = 0; f.mk = 0;
+            f.start = act ? d.fstarts[pg.fbase + 8u * f.j] : 0u;
+            f.size = act ? d.fsizes[pg.fbase + 8u * f.j] : 0u;
+            f.ops.load(d.ops + f.start, 0, f.size);
+        }
+        __syncthreads();
+        for (; i < steps && NW > CW; ++i) {
+            if (i % RA0_PACK == 0 && i) {
+                if (!pack(fn, i)) return;
+                if (NW <= CW) break;
+            }
+            WgMid md[PER];
+            bool has_nb[PER];
+            // settles slot q's flips against `below` (what lower slots look up)
+            // and returns its totals
+            auto settle_slot = [&](int q, uint64_t below) {
+                const WgFn<1> &f = fn[q];
+                WgMid &m = md[q];
+                uint32_t fl = (m.x >> 28) & 3u, r1, r2, x;
+                OpStep s;
+                if (has_nb[q]) {
+                    const uint32_t h1 = (m.x >> 16) & 0x3Fu, h2 = (m.x >> 22) & 0x3Fu;
+                    const bool b1 = (m.x >> 30) & 1u, b2 = (m.x >> 31) & 1u;
+                    const uint32_t *wmn = Wmn[i % RA0_WROWS];
+                    const bool w1 = b1 && (wmn[h1] < f.j || ((below >> h1) & 1u)), w2 = b2 && (wmn[h2] < f.j || ((below >> h2) & 1u));
+                    bool ch;
+                    do {
+                        wg_regs(m, fl, r1, r2);
+                        s = op_eval(m.op, r1, r2, f.life);
+                        const uint64_t low = (uint64_t)suffix_or<4>((uint32_t)s.look, lane, x) |
+                                             ((uint64_t)suffix_or<4>((uint32_t)(s.look >> 32), lane, x) << 32);
+                        const uint32_t nf = (w1 || (b1 && ((low >> h1) & 1u)) ? 1u : 0u) |
+                                            (w2 || (b2 && ((low >> h2) & 1u)) ? 2u : 0u);
+                        ch = nf != fl;
+                        fl = nf;
+                    } while (__ballot(ch));
+                    m.x = (m.x & ~(3u << 28)) | (fl << 28);
+                }
+                wg_regs(m, fl, r1, r2);
+                s = op_eval(m.op, r1, r2, f.life);
+                const uint64_t tc = wg_touch(m.op, s);
+                const uint32_t a = scan_or<4>((uint32_t)s.look), b = scan_or<4>((uint32_t)(s.look >> 32));
+                const uint32_t e = scan_or<4>((uint32_t)tc), g = scan_or<4>((uint32_t)(tc >> 32));
+                return Ra0Tot{lane64(a, b, 63), lane64(e, g, 63)};
+            };
 #pragma unroll
             for (int q = 0; q < PER; ++q) {
                 const uint32_t ws = wave + q * CW;
                 has_nb[q] = false;
                 if (ws >= NW) continue;
-                Fn &f = fn[q];
-                Mid &m = md[q];
-                const uint32_t k = ws * 64u + lane;
-                m.op = (int32_t)i < (int32_t)f.size ? f.cur.o[0] : 0u;
-                f.cur.o[0] = f.cur.o[1]; f.cur.o[1] = f.cur.o[2]; f.cur.o[2] = f.cur.o[3];
-                const uint32_t d1 = m.op & 0xFFu, d2 = (m.op >> 8) & 0xFFu;
-                m.p1 = i - d1; m.p2 = i - d2;
-                uint32_t e1 = wg_ring[(m.p1 & rm) * slots + k], e2 = wg_ring[(m.p2 & rm) * slots + k];
-                e1 = d1 ? e1 : 0u; e2 = d2 ? e2 : 0u;
-                uint32_t h1 = e1 & 0x3Fu, h2 = e2 & 0x3Fu;
-                // operands older than the ring, or no longer in their home: from HBM
-                const bool o1 = (m.op & OP_FAR1) || d1 > rm || (e1 & 0x80u), o2 = (m.op & OP_FAR2) || d2 > rm || (e2 & 0x80u);
-                if (__ballot(o1 || o2)) {
-                    if (o1 || o2) {
-                        if (m.op & (OP_FAR1 | OP_FAR2)) {
-                            const uint4 w = d.w0_f4[f.start + i];
-                            if (m.op & OP_FAR1) m.p1 = w.y - 64u - f.start;
-                            if (m.op & OP_FAR2) m.p2 = w.z - 64u - f.start;
-                        }
-                        const uint32_t g1 = d.sym[f.start + (o1 ? m.p1 : 0u)], g2 = d.sym[f.start + (o2 ? m.p2 : 0u)];
-                        wait_loads();
-                        if (o1) { e1 = (g1 & 0x3Fu) | (((g1 >> 8) & 1u) << 6); h1 = g1 >> 9; }
-                        if (o2) { e2 = (g2 & 0x3Fu) | (((g2 >> 8) & 1u) << 6); h2 = g2 >> 9; }
-                    }
+                WgFn<1> &f = fn[q];
+                const uint32_t op = f.ops.next(d.ops + f.start, i, f.size);
+                operands((int32_t)i < (int32_t)f.size ? op : 0u, i, ws * 64u + lane, f.start, f.own, f.pr, md[q]);
+                if (__ballot(f.own != 0)) {
+                    const uint32_t h1 = (md[q].x >> 16) & 0x3Fu, h2 = (md[q].x >> 22) & 0x3Fu;
+                    const uint32_t q1 = h1 == f.pr ? i - 1u : hold[h1], q2 = h2 == f.pr ? i - 1u : hold[h2];
+                    const bool b1 = q1 == md[q].p1 && ((f.own >> h1) & 1u), b2 = q2 == md[q].p2 && ((f.own >> h2) & 1u);
+                    has_nb[q] = __ballot(b1 || b2) != 0;
+                    md[q].x |= (b1 ? 1u << 30 : 0u) | (b2 ? 1u << 31 : 0u);
                 }
-                // (an entry won in the step before is not in hold yet)
-                const uint32_t q1 = h1 == f.pr ? i - 1u : hold[h1], q2 = h2 == f.pr ? i - 1u : hold[h2];
-                const uint32_t b1 = q1 == m.p1 && ((f.own >> h1) & 1u), b2 = q2 == m.p2 && ((f.own >> h2) & 1u);
-                m.x = (e1 & 0x7Fu) | ((e2 & 0x7Fu) << 7) | (h1 << 14) | (h2 << 20) | (b1 << 28) | (b2 << 29);
-                uint32_t r1, r2;
-                regs(m, 0u, r1, r2);
-                const OpStep s = op_eval(m.op, r1, r2, f.life);
-                has_nb[q] = __ballot(b1 | b2) != 0;
-                const uint64_t tl = or64(s.look), tt = or64(touched(m, s));
-                if (lane == 0) tot[c][ws] = Ra0Tot{tl | (has_nb[q] ? 1ull : 0ull), tt};
+                const Ra0Tot r = settle_slot(q, 0ull);
+                if (has_nb[q]) {
+                    const uint32_t x = md[q].x, key = ((i & 0x3FFFFFFu) << 6) | ws;
+                    if (((x >> 30) & 1u) && !((x >> 28) & 1u) && !((x >> 6) & 1u)) chk[i & 1u][(x >> 16) & 0x3Fu] = key;
+                    if (((x >> 31) & 1u) && !((x >> 29) & 1u) && !((x >> 14) & 1u)) chk[i & 1u][(x >> 22) & 0x3Fu] = key;
+                }
+                if (lane == 0) tot[i & 1u][ws] = r;
             }
-        }
-        lds_barrier();
+            lds_barrier();
 #pragma unroll
-        for (int q = 0; q < PER; ++q)
-            if (fn[q].pr) { hold[fn[q].pr] = i - 1u; fn[q].pr = 0; }
-        Ra0Tot t = totals(tot[c]);
-        if (__ballot(t.look & 1ull)) {
-            // settle the flips: a slot's lanes against the slots below as last
-            // published, until no slot's totals change
-            for (uint32_t r = 0;; ++r) {
-                const uint32_t cl = scan_or<4>((uint32_t)t.look), ch = scan_or<4>((uint32_t)(t.look >> 32));
-                {
+            for (int q = 0; q < PER; ++q)
+                if (fn[q].pr) { hold[fn[q].pr] = i - 1u; fn[q].pr = 0; }
+            Ra0Tot t = totals(tot[i & 1u]);
+            if (unsettled(t, i)) {
+                for (uint32_t r = 0;; ++r) {
+                    uint32_t x;
+                    const uint32_t bl = suffix_or<4>((uint32_t)t.look, lane, x), bh = suffix_or<4>((uint32_t)(t.look >> 32), lane, x);
 #pragma unroll
                     for (int q = 0; q < PER; ++q) {
                         const uint32_t ws = wave + q * CW;
                         if (ws >= NW) continue;
-                        Fn &f = fn[q];
-                        Mid &m = md[q];
-                        Ra0Tot nt{((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)t.look, (int)ws) |
-                                   ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(t.look >> 32), (int)ws) << 32)) & ~1ull,
-                                  (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)t.touch, (int)ws) |
-                                      ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(t.touch >> 32), (int)ws) << 32)};
-                        bool changed = false;
+                        Ra0Tot n{lane64((uint32_t)t.look, (uint32_t)(t.look >> 32), ws) & ~1ull,
+                                 lane64((uint32_t)t.touch, (uint32_t)(t.touch >> 32), ws)};
                         if (has_nb[q]) {
-                            uint64_t below = 0;
-                            if (ws) below = (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)cl, (int)ws - 1) |
-                                            ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)ch, (int)ws - 1) << 32);
-                            const uint32_t h1 = (m.x >> 14) & 0x3Fu, h2 = (m.x >> 20) & 0x3Fu;
-                            const bool b1 = (m.x >> 28) & 1u, b2 = (m.x >> 29) & 1u;
-                            const bool wl1 = Wmn[i % RA0_WROWS][h1] < f.j, wl2 = Wmn[i % RA0_WROWS][h2] < f.j;
-                            uint32_t fl = (m.x >> 26) & 3u, r1, r2;
-                            OpStep s;
-                            for (;;) {
-                                regs(m, fl, r1, r2);
-                                s = op_eval(m.op, r1, r2, f.life);
-                                const uint64_t low = below |
-                                    (uint64_t)from_below<4>(scan_or<4>((uint32_t)s.look)) |
-                                    ((uint64_t)from_below<4>(scan_or<4>((uint32_t)(s.look >> 32))) << 32);
-                                const uint32_t nf = ((b1 && (wl1 || ((low >> h1) & 1u))) ? 1u : 0u) |
-                                                    ((b2 && (wl2 || ((low >> h2) & 1u))) ? 2u : 0u);
-                                const bool ch2 = nf != fl;
-                                fl = nf;
-                                if (!__ballot(ch2)) break;
-                            }
-                            m.x = (m.x & ~(3u << 26)) | (fl << 26);
-                            const uint64_t tl = or64(s.look), tt = or64(touched(m, s));
-                            changed = tl != nt.look || tt != nt.touch;
-                            nt.look = tl; nt.touch = tt;
+                            const Ra0Tot o = n;
+                            n = settle_slot(q, lane64(bl, bh, ws));
+                            if (n.look != o.look || n.touch != o.touch) n.look |= 1ull;
                         }
-                        if (lane == 0) settle[r & 1u][ws] = Ra0Tot{nt.look | (changed ? 1ull : 0ull), nt.touch};
+                        if (lane == 0) settle[r & 1u][ws] = n;
                     }
+                    lds_barrier();
+                    t = totals(settle[r & 1u]);
+                    if (!__ballot(t.look & 1ull)) break;
                 }
+            }
+            // every slot's totals are final: of all, of the slots above each
+            const uint32_t la = scan_or<4>((uint32_t)t.look), lb = scan_or<4>((uint32_t)(t.look >> 32));
+            const uint32_t ta = scan_or<4>((uint32_t)t.touch), tb = scan_or<4>((uint32_t)(t.touch >> 32));
+            const uint64_t T = (lane64(la, lb, 63) | Wany[i % RA0_WROWS]) & ~1ull, lost = lane64(ta, tb, 63);
+#pragma unroll
+            for (int q = 0; q < PER; ++q) {
+                const uint32_t ws = wave + q * CW;
+                if (ws >= NW) continue;
+                WgFn<1> &f = fn[q];
+                const WgMid &m = md[q];
+                uint32_t r1, r2;
+                wg_regs(m, (m.x >> 28) & 3u, r1, r2);
+                const OpStep s = op_eval(m.op, r1, r2, f.life);
+                const uint64_t tc = wg_touch(m.op, s);
+                uint64_t won = (m.op & OP_SELF) ? s.dm & ~(ws ? lane64(ta, tb, ws - 1u) : 0ull) : 0ull;
+                if (__ballot(won != 0))
+                    won &= ~((uint64_t)from_below<4>(scan_or<4>((uint32_t)tc)) |
+                             ((uint64_t)from_below<4>(scan_or<4>((uint32_t)(tc >> 32))) << 32));
+                uint64_t nm = 0;
+                if (__ballot(f.own != 0)) {
+                    uint64_t mset = f.own & T;
+                    if (has_nb[q]) {
+                        const uint32_t h1 = (m.x >> 16) & 0x3Fu, h2 = (m.x >> 22) & 0x3Fu;
+                        uint64_t high = (uint64_t)from_below<4>(scan_or<4>((uint32_t)s.look)) |
+                                        ((uint64_t)from_below<4>(scan_or<4>((uint32_t)(s.look >> 32))) << 32);
+                        if (ws) high |= lane64(la, lb, ws - 1u);
+                        const uint64_t nb1 = (m.x >> 30) & 1u ? 1ull << h1 : 0ull, nb2 = (m.x >> 31) & 1u ? 1ull << h2 : 0ull;
+                        if (Wmx[i % RA0_WROWS][h1] > f.j + 1u) high |= nb1;
+                        if (Wmx[i % RA0_WROWS][h2] > f.j + 1u) high |= nb2;
+                        const uint64_t nb = nb1 | nb2;
+                        mset = f.own & ((T & ~nb) | (high & nb));
+                        f.mk &= ~nb;
+                    }
+                    nm = mset & ~f.mk;
+                    f.mk |= mset;
+                }
+                commit(m, s, r1, r2, i, ws * 64u + lane, f.start, (int32_t)i < (int32_t)f.size, nm);
+                f.life = s.life;
+                f.own = (f.own & ~lost) | won;
+                f.mk &= ~lost;
+                f.pr = won ? s.rdr : 0u;
+            }
+            next_row();
+        }
+        if (i >= steps) return;
+        f1[0].j = fn[0].j; f1[0].start = fn[0].start; f1[0].size = fn[0].size; f1[0].life = fn[0].life;
+        f1[0].own = fn[0].own; f1[0].mk = fn[0].mk;
+    } else {
+        const uint32_t k = wave * 64u + lane;
+        const bool act = k < pg.L;
+        f1[0].j = act ? pg.L - 1u - k : 0u; f1[0].life = 0x1Full; f1[0].own = 0; f1[0].mk = 0;
+        f1[0].start = act ? d.fstarts[pg.fbase + 8u * f1[0].j] : 0u;
+        f1[0].size = act ? d.fsizes[pg.fbase + 8u * f1[0].j] : 0u;
+        __syncthreads();
+    }
+    f1[0].pr = 0;
+    f1[0].ops.load(d.ops + f1[0].start, i, f1[0].size);
+    bool packed = true;  // (the pack at this step is done)
+    // a slot a wave: the step's results stay in registers over the barrier
+    for (; NW > 1u && i < steps; ++i) {
+        if (i % RA0_PACK == 0 && i && !packed) {
+            if (!pack(f1, i)) return;
+            if (NW == 1u) break;
+        }
+        packed = false;
+        WgFn<4> &f = f1[0];
+        const uint32_t k = wave * 64u + lane;
+        const uint32_t op = f.ops.next(d.ops + f.start, i, f.size);
+        const bool run = (int32_t)i < (int32_t)f.size;
+        WgMid m;
+        operands(run ? op : 0u, i, k, f.start, f.own, f.pr, m);
+        const uint32_t h1 = (m.x >> 16) & 0x3Fu, h2 = (m.x >> 22) & 0x3Fu;
+        // (an entry won in the step before is not in hold yet)
+        const uint32_t q1 = h1 == f.pr ? i - 1u : hold[h1], q2 = h2 == f.pr ? i - 1u : hold[h2];
+        const uint32_t mn1 = Wmn[i % RA0_WROWS][h1], mn2 = Wmn[i % RA0_WROWS][h2];
+        const uint32_t mx1 = Wmx[i % RA0_WROWS][h1], mx2 = Wmx[i % RA0_WROWS][h2];
+        const bool z1 = (m.x >> 6) & 1u, z2 = (m.x >> 14) & 1u;  // swapped already
+        uint32_t fl = 0, r1, r2, x;
+        wg_regs(m, 0u, r1, r2);
+        OpStep s = op_eval(m.op, r1, r2, f.life);
+        const uint64_t nb1 = q1 == m.p1 ? f.own & (1ull << h1) : 0ull, nb2 = q2 == m.p2 ? f.own & (1ull << h2) : 0ull;
+        const uint64_t nb = nb1 | nb2;
+        const uint64_t wl = (mn1 < f.j ? nb1 : 0ull) | (mn2 < f.j ? nb2 : 0ull);
+        // flips against the slot's own lookups, the walk's and `below`
+        auto settle_slot = [&](uint64_t below) {
+            uint64_t low = below | (uint64_t)suffix_or<4>((uint32_t)s.look, lane, x) |
+                           ((uint64_t)suffix_or<4>((uint32_t)(s.look >> 32), lane, x) << 32);
+            uint32_t nf = ((nb1 & low) && !z1 ? 1u : 0u) | ((nb2 & low) && !z2 ? 2u : 0u);
+            while (__ballot(nf != fl)) {
+                fl = nf;
+                wg_regs(m, fl, r1, r2);
+                s = op_eval(m.op, r1, r2, f.life);
+                low = below | (uint64_t)suffix_or<4>((uint32_t)s.look, lane, x) |
+                      ((uint64_t)suffix_or<4>((uint32_t)(s.look >> 32), lane, x) << 32);
+                nf = ((nb1 & low) && !z1 ? 1u : 0u) | ((nb2 & low) && !z2 ? 2u : 0u);
+            }
+        };
+        settle_slot(wl);
+        uint64_t tc = wg_touch(m.op, s);
+        uint32_t la = scan_or<4>((uint32_t)s.look), lb = scan_or<4>((uint32_t)(s.look >> 32));
+        uint32_t ta = scan_or<4>((uint32_t)tc), tb = scan_or<4>((uint32_t)(tc >> 32));
+        if (lane == 63u) tot[i & 1u][wave] = Ra0Tot{(uint64_t)la | ((uint64_t)lb << 32), (uint64_t)ta | ((uint64_t)tb << 32)};
+        const bool c1 = nb1 != 0 && !(fl & 1u) && !z1, c2 = nb2 != 0 && !(fl & 2u) && !z2;
+        if (c1 || c2) {
+            const uint32_t key = ((i & 0x3FFFFFFu) << 6) | wave;
+            if (c1) chk[i & 1u][h1] = key;
+            if (c2) chk[i & 1u][h2] = key;
+        }
+        lds_barrier();
+        hold[f.pr ? f.pr : 64u] = i - 1u;
+        Ra0Tot t = totals(tot[i & 1u]);
+        if (unsettled(t, i)) {
+            for (uint32_t r = 0;; ++r) {
+                const uint64_t below = lane64(suffix_or<4>((uint32_t)t.look, lane, x), suffix_or<4>((uint32_t)(t.look >> 32), lane, x), wave);
+                const uint64_t ol = lane64(la, lb, 63), ot = lane64(ta, tb, 63);
+                settle_slot(wl | below);
+                tc = wg_touch(m.op, s);
+                la = scan_or<4>((uint32_t)s.look); lb = scan_or<4>((uint32_t)(s.look >> 32));
+                ta = scan_or<4>((uint32_t)tc); tb = scan_or<4>((uint32_t)(tc >> 32));
+                const uint64_t nl = lane64(la, lb, 63), nt = lane64(ta, tb, 63);
+                if (lane == 0) settle[r & 1u][wave] = Ra0Tot{nl | (nl != ol || nt != ot ? 1ull : 0ull), nt};
                 lds_barrier();
                 t = totals(settle[r & 1u]);
                 if (!__ballot(t.look & 1ull)) break;
             }
         }
-        // the step's end: every slot's totals are final
-        uint64_t T = or64(t.look) | Wany[i % RA0_WROWS];
-        T &= ~1ull;
-        uint32_t al, ah, ul, uh;
-        ul = suffix_or<4>((uint32_t)t.touch, lane, al);
-        uh = suffix_or<4>((uint32_t)(t.touch >> 32), lane, ah);
-        const uint64_t lost = (uint64_t)al | ((uint64_t)ah << 32);
-#pragma unroll
-        for (int q = 0; q < PER; ++q) {
-            const uint32_t ws = wave + q * CW;
-            if (ws >= NW) continue;
-            Fn &f = fn[q];
-            const Mid &m = md[q];
-            const uint32_t k = ws * 64u + lane;
-            const uint32_t fl = (m.x >> 26) & 3u;
-            uint32_t r1, r2, x;
-            regs(m, fl, r1, r2);
-            const OpStep s = op_eval(m.op, r1, r2, f.life);
-            const uint64_t touch = touched(m, s);
-            uint64_t above = (uint64_t)suffix_or<4>((uint32_t)touch, lane, x) |
-                             ((uint64_t)suffix_or<4>((uint32_t)(touch >> 32), lane, x) << 32);
-            above |= (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)ul, (int)ws) |
-                     ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)uh, (int)ws) << 32);
-            const bool run = (int32_t)i < (int32_t)f.size, self = (m.op & OP_SELF) != 0;
-            const uint32_t h1 = (m.x >> 14) & 0x3Fu, h2 = (m.x >> 20) & 0x3Fu;
-            uint64_t mset = f.own & T;
-            if (has_nb[q]) {
-                uint32_t yl, yh;
-                uint64_t high = (uint64_t)suffix_or<4>((uint32_t)s.look, lane, x) |
-                                ((uint64_t)suffix_or<4>((uint32_t)(s.look >> 32), lane, x) << 32);
-                yl = suffix_or<4>((uint32_t)t.look, lane, x);
-                yh = suffix_or<4>((uint32_t)(t.look >> 32), lane, x);
-                high |= (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)yl, (int)ws) |
-                        ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)yh, (int)ws) << 32);
-                const uint64_t nb1 = ((m.x >> 28) & 1u) ? 1ull << h1 : 0ull, nb2 = ((m.x >> 29) & 1u) ? 1ull << h2 : 0ull;
-                if (Wmx[i % RA0_WROWS][h1] > f.j + 1u) high |= nb1;
-                if (Wmx[i % RA0_WROWS][h2] > f.j + 1u) high |= nb2;
-                const uint64_t nb = nb1 | nb2;
-                mset = f.own & ((T & ~nb) | (high & nb));
-                f.mk &= ~nb;
-            }
-            const bool s1 = ((m.x >> 6) & 1u) || (fl & 1u), s2 = ((m.x >> 13) & 1u) || (fl & 2u);
-            if (s1) {
-                if (i - m.p1 <= rm) wg_ring[(m.p1 & rm) * slots + k] = (uint8_t)(r1 | 0x80u);
-                d.sym[f.start + m.p1] = (uint16_t)(r1 | (h1 << 9));
-            }
-            if (s2) {
-                if (i - m.p2 <= rm) wg_ring[(m.p2 & rm) * slots + k] = (uint8_t)(r2 | 0x80u);
-                d.sym[f.start + m.p2] = (uint16_t)(r2 | (h2 << 9));
-            }
-            uint64_t nm = mset & ~f.mk;
-            f.mk |= mset;
-            while (nm) {
-                const uint32_t r = (uint32_t)__builtin_ctzll(nm);
-                nm &= nm - 1;
-                const uint32_t p = hold[r];
-                if (i - p <= rm) wg_ring[(p & rm) * slots + k] |= 0x40u;
-                reinterpret_cast<uint8_t *>(d.sym + f.start)[2u * p + 1u] = (uint8_t)(1u | (r << 1));
-            }
-            const uint64_t won = self ? s.dm & ~above : 0ull;
-            if (run) {
-                const uint32_t reg = self && !(m.op & OP_ZERO) ? s.rdr : 0u;
-                wg_ring[(i & rm) * slots + k] = (uint8_t)(reg | (self && reg != s.rdr ? 0x80u : 0u));
-                if (self) d.sym[f.start + i] = (uint16_t)(reg | (s.rdr << 9));
-            }
-            f.life = s.life;
-            f.own = (f.own & ~lost) | won;
-            f.mk &= ~lost;
-            f.pr = won ? s.rdr : 0u;
-            if ((i & 3u) == 3u) { f.cur = f.nxt; f.nxt = ops_at(f, i + 5u); }
-        }
+        // every slot's totals are final: of all, of the slots above (at most 16
+        // slots: one row of lanes)
+        const uint32_t sa = scan_or<1>((uint32_t)t.look), sb = scan_or<1>((uint32_t)(t.look >> 32));
+        const uint32_t ua = scan_or<1>((uint32_t)t.touch), ub = scan_or<1>((uint32_t)(t.touch >> 32));
+        const uint64_t T = (lane64(sa, sb, 15) | Wany[i % RA0_WROWS]) & ~1ull, lost = lane64(ua, ub, 15);
+        const uint32_t wp = wave ? wave - 1u : 31u;  // (lanes past the first row hold nothing)
+        uint64_t high = (uint64_t)from_below<4>(la) | ((uint64_t)from_below<4>(lb) << 32) | lane64(sa, sb, wp);
+        high |= (mx1 > f.j + 1u ? nb1 : 0ull) | (mx2 > f.j + 1u ? nb2 : 0ull);
+        const uint64_t above = (uint64_t)from_below<4>(ta) | ((uint64_t)from_below<4>(tb) << 32) | lane64(ua, ub, wp);
+        const uint64_t won = (m.op & OP_SELF) ? s.dm & ~above : 0ull;
+        f.mk &= ~nb;
+        const uint64_t nm = f.own & ~f.mk & ((T & ~nb) | (high & nb));
+        f.mk |= nm;
+        m.x |= fl << 28;
+        commit(m, s, r1, r2, i, k, f.start, run, nm);
+        f.life = s.life;
+        f.own = (f.own & ~lost) | won;
+        f.mk &= ~lost;
+        f.pr = won ? s.rdr : 0u;
+        next_row();
     }
     if (i >= steps) return;
     // one slot left: its steps need no exchange with other waves
-    RaL0 f{fn[0].start, fn[0].size, fn[0].life, fn[0].own, fn[0].mk};
+    RaL0 f{f1[0].start, f1[0].size, f1[0].life, f1[0].own, f1[0].mk};
     uint16_t *ring = reinterpret_cast<uint16_t *>(wg_ring);
     const uint32_t *ops = d.ops + f.start;
     OpBlock ob;
@@ -3487,7 +3666,7 @@ __global__ __launch_bounds__(1024) void k_ra_lane0_wg(Dev d, const Ra0Prog *prog
         for (uint32_t q = 0; q < 4; ++q) {
             const uint32_t r = (i + q) % RA0_WROWS;
             const uint32_t op = (int32_t)(i + q) < (int32_t)f.size ? ob.cur[0].o[q] : 0u;
-            ra_l0_step<5, 64, 1>(d, f, ring, hold, lane, 0u, lane, true, fn[0].j, i, i + q, op,
+            ra_l0_step<5, 64, 1>(d, f, ring, hold, lane, 0u, lane, true, f1[0].j, i, i + q, op,
                                  RaLooks{0ull, Wmn[r], Wmx[r], i + q < steps ? Wany[r] : 0ull});
         }
     }
