@@ -23,11 +23,10 @@
 //   regalloc     k_ra_walk (functions not in lane 0 of an 8-function group:
 //                independent), k_ra_lane0_wave / k_ra_lane0 (lane-0 functions in
 //                step lockstep: they share the first 64-entry region of the
-//                reference's register_state snapshot, :1290-1354), k_ra_group
-//                (programs of one group), k_ra_serial (exact in-order walk for
-//                programs where a function names another's register), then
-//                counts, scan, emit (:1422-1697), function table fix and frame
-//                words (:1714-1811).
+//                reference's register_state snapshot, :1290-1354), k_ra_serial (exact
+//                in-order walk for programs where a function names another's
+//                register), then counts, scan, emit (:1422-1697), function table
+//                fix and frame words (:1714-1811).
 //   fix_jumps    size + scan + fused move/encode/postprocess (:1853-1993, 1995-2011).
 //
 // Batches: P programs concatenated node-wise run through the same kernels.
@@ -1754,6 +1753,81 @@ struct OpQueue {
 };
 
 
+DEV uint32_t rdlane(uint32_t v, uint32_t l) { return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)l); }
+extern "C" __device__ int ptl_writelane(int x, int l, int v) __asm("llvm.amdgcn.writelane.i32");
+DEV uint32_t wrlane(uint32_t v, uint32_t l, uint32_t x) { return (uint32_t)ptl_writelane((int)x, (int)l, (int)v); }
+DEV uint32_t uniform(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
+
+// A walk of one function on a whole wave: the step is scalar code (a scalar
+// instruction takes about half a vector one's time in a dependent chain, has
+// 64-bit masks and cheap branches), and what it needs of the last words is a lane
+// of a vector register: `cur` has the ops of the block of 64 steps, `ringv` the
+// states of the last 64 words (word mod 64), written and read by lane.  States
+// go to HBM, and lookups to the tables, once a block, from all lanes.  Operands
+// 64 words back and more are in the LDS ring `old`.
+// Latency bound: 0.14 us a step against 0.30 as a lane (a function of 4115 words,
+// 1.24 -> 0.58 ms).
+constexpr uint32_t WALK_OLD = 16384;  // words of the LDS ring
+DEV void walk_one(const Dev &d, uint8_t *old, unsigned long long *mtab, const Ra0Prog &pg, uint32_t f, uint32_t grp,
+                  uint32_t lane, uint32_t *done) {
+    const uint32_t start = uniform(d.fstarts[f]), size = uniform(d.fsizes[f]);
+    const uint32_t L = pg.L, last = pg.rows - 1u;
+    unsigned long long *tab = mtab + pg.gbase + grp;
+    uint32_t ringv = 0, lo = 0, hi = 0;
+    uint64_t life = 0x1Full;
+    auto load = [&](uint32_t i) { return d.ops[start + min(i + lane, size)]; };
+    uint32_t nxt = load(0);
+    for (uint32_t b = 0; b < size; b += 64) {
+        uint32_t cur = nxt;
+        asm volatile("" : "+v"(cur) : : "memory");  // waited for before the next load is issued
+        nxt = load(b + 64u);
+        const uint32_t n = min(64u, size - b);
+        for (uint32_t k = 0; k < n; ++k) {
+            const uint32_t op = rdlane(cur, k);
+            const uint32_t d1 = op & 0xFFu, d2 = (op >> 8) & 0xFFu;
+            uint32_t r1 = d1 ? rdlane(ringv, (k - d1) & 63u) : 0u, r2 = d2 ? rdlane(ringv, (k - d2) & 63u) : 0u;
+            if (__builtin_expect((op & (0xC0C0u | OP_FAR1 | OP_FAR2)) != 0, 0)) {
+                const uint32_t i = b + k;
+                const uint4 w = d.w0_f4[start + i];
+                wait_loads();
+                const uint32_t p1 = (op & OP_FAR1) ? uniform(w.y) - 64u - start : i - d1;
+                const uint32_t p2 = (op & OP_FAR2) ? uniform(w.z) - 64u - start : i - d2;
+                // (a word 64 or more back is in a block that has ended)
+                auto state = [&](uint32_t p) {
+                    uint32_t v = i - p < WALK_OLD - 64u ? old[p % WALK_OLD] : d.sym[start + p];
+                    wait_loads();
+                    return uniform(v) & 0x3Fu;
+                };
+                if ((op & OP_FAR1) || d1 > 63u) r1 = state(p1);
+                if ((op & OP_FAR2) || d2 > 63u) r2 = state(p2);
+            }
+            const OpStep s = op_eval(op, r1, r2, life);
+            life = s.life;
+            ringv = wrlane(ringv, k, (op & (OP_SELF | OP_ZERO)) == OP_SELF ? s.rdr : 0u);
+            lo = wrlane(lo, k, (uint32_t)s.look);
+            hi = wrlane(hi, k, (uint32_t)(s.look >> 32));
+        }
+        if (lane < n) {
+            const uint32_t i = b + lane;
+            d.sym[start + i] = (uint16_t)ringv;
+            old[i % WALK_OLD] = (uint8_t)ringv;
+            const unsigned long long look = (unsigned long long)lo | ((unsigned long long)hi << 32);
+            if (look) atomicOr(tab + (uint64_t)min(i, last) * L, look);
+        }
+        if (done && pg.cbase != RA0_NOPUB) {
+            // the chunks of rows this block leaves (see k_ra_walk)
+            const uint32_t nch = last / WALK_PUB + 1u, e = b + 64u;
+            const uint32_t npub = min(nch, (size + WALK_PUB - 1u) / WALK_PUB);
+            const uint32_t from = min(b / WALK_PUB, nch - 1u), to = e >= size ? npub : min(e / WALK_PUB, nch - 1u);
+            if (from < to) {
+                __threadfence();
+                if (lane < to - from)
+                    __hip_atomic_fetch_add(&done[pg.cbase + from + lane], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
+    }
+}
+
 // One function per lane.  The states of a function's last OP_ROWS words are in
 // an LDS ring of bytes, row = word mod OP_ROWS (a state here is just the
 // register the word's rd was given; it never changes); operands further back
@@ -1765,12 +1839,25 @@ struct OpQueue {
 __global__ __launch_bounds__(64) void k_ra_walk(Dev d, uint32_t *gmin_all, uint32_t *gmax_all, uint64_t stride,
                                                 uint32_t copies, unsigned long long *mask_all, uint64_t mstride,
                                                 uint32_t mcopies, const Ra0Prog *progs, const uint32_t *permw,
-                                                uint32_t nw, uint32_t *done) {
-    __shared__ uint32_t smin[64], smax[64];
+                                                uint32_t nw, uint32_t nreg, uint32_t solo, uint32_t *done) {
+    __shared__ uint32_t smin[4][64], smax[4][64];
     __shared__ uint8_t ring[OP_ROWS * 64];
+    static_assert(sizeof(ring) >= WALK_OLD, "walk_one's LDS ring");
     const uint32_t lane = threadIdx.x;
-    const uint32_t t = blockIdx.x * 64u + lane;
-    const uint32_t f = t < nw ? permw[t] : d.F;
+    // 64 functions to a workgroup: those of programs with (step, register) tables
+    // (the first nreg, a workgroup's all of one program, padded), and the last
+    // ones; `solo` between them have one each
+    const uint32_t nb0 = (nreg + 63u) / 64u;
+    uint32_t t = blockIdx.x * 64u + lane, tend = nreg;
+    if (blockIdx.x >= nb0 + solo) { t = nreg + solo + (blockIdx.x - nb0 - solo) * 64u + lane; tend = nw; }
+    else if (blockIdx.x >= nb0) {
+        const uint32_t f = permw[nreg + blockIdx.x - nb0];
+        const uint32_t prg = prog_of(d.pf, d.P, f);
+        if (d.cflag[prg]) return;  // k_ra_serial's
+        walk_one(d, ring, mask_all + (blockIdx.x % mcopies) * mstride, progs[prg], f, (f - d.pf[prg]) >> 3, lane, done);
+        return;
+    }
+    const uint32_t f = t < tend ? permw[t] : d.F;
     const bool act = f < d.F;
     // group = function index within its program / 8; lookup table of the program
     const uint32_t prg = act ? prog_of(d.pf, d.P, f) : 0xFFFFFFFFu;
@@ -1779,19 +1866,14 @@ __global__ __launch_bounds__(64) void k_ra_walk(Dev d, uint32_t *gmin_all, uint3
     const uint32_t start = act ? d.fstarts[f] : 0u;
     const uint32_t size = act && !skip ? d.fsizes[f] : 0u;
     const uint32_t L = act ? progs[prg].L : 0u;
-    const bool masks = L <= RA0_WAVE_GROUPS;
-    uint32_t pmin = prg, pmax = act ? prg : 0u;
-    for (int s = 32; s > 0; s >>= 1) { pmin = min(pmin, (uint32_t)__shfl_xor((int)pmin, s, 64)); pmax = max(pmax, (uint32_t)__shfl_xor((int)pmax, s, 64)); }
-    // the workgroup's functions all belong to one program with (step, register) tables
-    const bool one = pmin == pmax && __ballot(act && !masks) != 0;
-    const bool any_reg = __ballot(act && !masks) != 0;
+    const bool reg = blockIdx.x < nb0;  // (step, register) tables
     uint32_t *gmin = gmin_all + (blockIdx.x % copies) * stride;
     uint32_t *gmax = gmax_all + (blockIdx.x % copies) * stride;
     unsigned long long *mtab = mask_all + (blockIdx.x % mcopies) * mstride;
-    const uint64_t tb = one ? progs[pmin].gbase : 0u;  // table base of that program
-    const uint32_t tlast = one ? progs[pmin].rows - 1u : 0u;
     const uint64_t mbase = act ? progs[prg].gbase : 0u;  // own program's table and its last row
     const uint32_t mlast = act ? progs[prg].rows - 1u : 0u;
+    const uint64_t tb = (uint64_t)uniform((uint32_t)mbase) | ((uint64_t)uniform((uint32_t)(mbase >> 32)) << 32);
+    const uint32_t tlast = uniform(mlast);  // (a workgroup's first lane has a function)
     // the lowest lane of each program in the workgroup publishes that program's
     // rows; pw = the size of the program's longest function here
     uint32_t pw = 0;
@@ -1814,7 +1896,7 @@ __global__ __launch_bounds__(64) void k_ra_walk(Dev d, uint32_t *gmin_all, uint3
     const uint32_t nch = mlast / WALK_PUB + 1u;
     const uint32_t npub = publishes ? min(nch, (pw + WALK_PUB - 1u) / WALK_PUB) : 0u;  // chunks it takes part in
     uint32_t pubd = 0;
-    smin[lane] = 0xFFFFFFFFu; smax[lane] = 0;
+    for (uint32_t q = 0; q < 4; ++q) { smin[q][lane] = 0xFFFFFFFFu; smax[q][lane] = 0; }
     uint32_t wmax = size;
     for (int s = 32; s > 0; s >>= 1) { uint32_t o = __shfl_xor(wmax, s, 64); wmax = wmax > o ? wmax : o; }
     uint64_t life = 0x1Full;
@@ -1846,32 +1928,30 @@ __global__ __launch_bounds__(64) void k_ra_walk(Dev d, uint32_t *gmin_all, uint3
             life = s.life;
             st[q] = (op & OP_SELF) && !(op & OP_ZERO) ? s.rdr : 0u;
             ring[(i & (OP_ROWS - 1u)) * 64u + lane] = (uint8_t)st[q];
-            if (run && masks && s.look) atomicOr(&mtab[mbase + (uint64_t)min(i, mlast) * L + grp], (unsigned long long)s.look);
-            if (any_reg) {
-                uint64_t lk = run && !masks ? s.look : 0ull;
-                if (!one) {  // functions of several programs: post straight to each program's table
-                    const uint64_t row = mbase + (uint64_t)min(i, mlast) * 64u;
-                    while (lk) {
-                        const uint32_t r = (uint32_t)__builtin_ctzll(lk);
-                        lk &= lk - 1;
-                        atomicMin(&gmin[row + r], grp); atomicMax(&gmax[row + r], grp + 1u);
-                    }
-                } else {
-                    while (lk) {
-                        const uint32_t r = (uint32_t)__builtin_ctzll(lk);
-                        lk &= lk - 1;
-                        atomicMin(&smin[r], grp); atomicMax(&smax[r], grp + 1u);
-                    }
-                    lds_barrier();
-                    const uint32_t mx = smax[lane];
-                    if (mx) {
-                        atomicMin(&gmin[tb + (uint64_t)min(i, tlast) * 64u + lane], smin[lane]);
-                        atomicMax(&gmax[tb + (uint64_t)min(i, tlast) * 64u + lane], mx);
-                        smin[lane] = 0xFFFFFFFFu; smax[lane] = 0;
-                    }
-                    lds_barrier();
+            if (!reg) {
+                if (run && s.look) atomicOr(&mtab[mbase + (uint64_t)min(i, mlast) * L + grp], (unsigned long long)s.look);
+            } else {
+                uint64_t lk = run ? s.look : 0ull;
+                while (lk) {
+                    const uint32_t r = (uint32_t)__builtin_ctzll(lk);
+                    lk &= lk - 1;
+                    atomicMin(&smin[q][r], grp); atomicMax(&smax[q][r], grp + 1u);
                 }
             }
+        }
+        if (reg) {  // the four steps' lookups, folded over the workgroup
+            lds_barrier();
+#pragma unroll
+            for (uint32_t q = 0; q < 4; ++q) {
+                const uint32_t mn = smin[q][lane], mx = smax[q][lane];
+                if (mx) {
+                    const uint64_t e = tb + (uint64_t)min(i0 + q, tlast) * 64u + lane;
+                    atomicMin(&gmin[e], mn);
+                    atomicMax(&gmax[e], mx);
+                    smin[q][lane] = 0xFFFFFFFFu; smax[q][lane] = 0;
+                }
+            }
+            lds_barrier();
         }
         // (sym starts cleared: only words past the last whole four need care)
         if ((int32_t)(i0 + 3u) < (int32_t)size) {
@@ -1927,10 +2007,13 @@ DEV void ra0_wait(const Dev &d, const uint32_t *done, const uint32_t *need, uint
     if (!ok) return;
     const uint32_t want = need[c];
     const uint64_t t0 = wall_clock64();
-    while (__hip_atomic_load(&done[c], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT) < want) {
+    // (the polls are relaxed: an acquire invalidates the compute unit's caches,
+    // which the waves beside use; one at the end orders the rows' loads)
+    while (__hip_atomic_load(&done[c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < want) {
         if (wall_clock64() - t0 > RA0_WAIT_TICKS) { ok = false; atomicOr(d.flags, EF_WAIT); return; }
-        __builtin_amdgcn_s_sleep(2);
+        __builtin_amdgcn_s_sleep(8);
     }
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
 }
 
 // ---------------------------------------------- lane-0 functions in one wave
@@ -2016,14 +2099,13 @@ DEV void ra_flush(const Dev &d, const RaL0 &f, const uint16_t *ring, uint32_t rc
 }
 
 // One step i (of the block of four from b) of this lane's function on its word's
-// op (0 where it has ended).  MODE 0: programs of one group, 8 to a wave, lane
-// 8s + k walking function k of program slot s (l0: k is 0); the group's lookups
-// of the step mark, except an entry whose register the word names (its reset
-// lands after a same-group mark).  MODE 1, 4, 5: the wave's lanes walk the lane-0
-// functions of one program, the highest group in lane 0 (j: the lane's group), in
-// the first row of 16 lanes (1) or all four, the walk's lookups given by lane (1,
-// 4) or by register (5).
-// There a lookup by a lower group is seen by the owner's operand read of the same
+// op (0 where it has ended).  The wave's lanes walk the lane-0 functions of one
+// program, the highest group in lane 0 (j: the lane's group), in the first row of
+// 16 lanes (MODE 1) or all four (4, 5), the walk's lookups given by lane (1, 4) or
+// by register (5).
+// A lookup marks the virtual register its entry holds, except one the word names
+// (its reset lands after a mark by its own or a lower group).  A lookup by a lower
+// group is seen by the owner's operand read of the same
 // step (a flip), settled by re-evaluation until the flips are stable: a group's
 // depend on the groups below it alone, so this reaches the in-order result.  A
 // lookup by a higher group lands after the owner's own reset, and the last group
@@ -2032,10 +2114,10 @@ DEV void ra_flush(const Dev &d, const RaL0 &f, const uint16_t *ring, uint32_t rc
 // whether it is taken or not: everything but the rare cases (a state read from
 // HBM, a second mark, a flip) is straight-line, its writes going to a spare row or
 // entry where there is nothing to write.
-// hold has an entry per register (and one spare) and, MODE 0, program slot (HC).
-template <int MODE, int RC, int HC>
-DEV void ra_l0_step(const Dev &d, RaL0 &f, uint16_t *ring, uint32_t *hold, uint32_t rc, uint32_t hc, uint32_t lane,
-                    bool l0, uint32_t j, uint32_t b, uint32_t i, uint32_t op, const RaLooks &lk) {
+// hold has an entry per register and one spare.
+template <int MODE, int RC>
+DEV void ra_l0_step(const Dev &d, RaL0 &f, uint16_t *ring, uint32_t *hold, uint32_t rc, uint32_t lane, uint32_t j,
+                    uint32_t b, uint32_t i, uint32_t op, const RaLooks &lk) {
     constexpr int ROWS = MODE > 1 ? 4 : 1;
     constexpr int LAST = ROWS == 1 ? 15 : 63;
     const uint32_t d1 = op & 0xFFu, d2 = (op >> 8) & 0xFFu;
@@ -2063,7 +2145,7 @@ DEV void ra_l0_step(const Dev &d, RaL0 &f, uint16_t *ring, uint32_t *hold, uint3
     // whether the entry of an operand's home holds it (no operand: home x0, which
     // is never held)
     const uint32_t h1 = e1 >> 9, h2 = e2 >> 9;
-    const uint32_t q1 = hold[h1 * HC + hc], q2 = hold[h2 * HC + hc];
+    const uint32_t q1 = hold[h1], q2 = hold[h2];
     uint32_t mn1 = 0, mn2 = 0, mx1 = 0, mx2 = 0;
     if (MODE == 5) { mn1 = lk.mn[h1]; mn2 = lk.mn[h2]; mx1 = lk.mx[h1]; mx2 = lk.mx[h2]; }
     const uint32_t sr1 = (op & OP_FP) ? 37u : 5u, sr2 = (op & OP_FP) ? 38u : 6u;
@@ -2073,56 +2155,45 @@ DEV void ra_l0_step(const Dev &d, RaL0 &f, uint16_t *ring, uint32_t *hold, uint3
     const uint64_t nb1 = q1 == p1 ? f.own & (1ull << h1) : 0ull, nb2 = q2 == p2 ? f.own & (1ull << h2) : 0ull;
     const uint64_t nb = nb1 | nb2;
     const bool self = (op & OP_SELF) != 0;
-    uint64_t T, high = 0;
-    if (MODE == 0) {
-        T = sm_or8_64(s.look);
-    } else {
-        uint32_t tl = (uint32_t)s.look | (uint32_t)lk.W, th = (uint32_t)(s.look >> 32) | (uint32_t)(lk.W >> 32);
-        // looked up by a lower group (the lanes above); the walk's by register
-        const uint64_t wl = MODE == 5 ? (mn1 < j ? nb1 : 0ull) | (mn2 < j ? nb2 : 0ull) : 0ull;
-        uint32_t x;
-        uint64_t low = wl | (uint64_t)suffix_or<ROWS>(tl, lane, x) | ((uint64_t)suffix_or<ROWS>(th, lane, x) << 32);
-        bool n1 = (nb1 & low) != 0, n2 = (nb2 & low) != 0;
-        const bool z1 = s1, z2 = s2;  // swapped already
-        if (__ballot((n1 && !z1) || (n2 && !z2))) {
-            bool ch;
-            do {
-                const bool f1 = n1, f2 = n2;
-                s1 = z1 || f1; s2 = z2 || f2;
-                r1 = s1 ? sr1 : e1 & 0x3Fu; r2 = s2 ? sr2 : e2 & 0x3Fu;
-                s = op_eval(op, r1, r2, f.life);
-                tl = (uint32_t)s.look | (uint32_t)lk.W; th = (uint32_t)(s.look >> 32) | (uint32_t)(lk.W >> 32);
-                low = wl | (uint64_t)suffix_or<ROWS>(tl, lane, x) | ((uint64_t)suffix_or<ROWS>(th, lane, x) << 32);
-                n1 = (nb1 & low) != 0; n2 = (nb2 & low) != 0;
-                ch = (n1 != f1 && !z1) || (n2 != f2 && !z2);
-            } while (__ballot(ch));
-        }
-        const uint32_t il = scan_or<ROWS>(tl), ih = scan_or<ROWS>(th);
-        high = (uint64_t)from_below<ROWS>(il) | ((uint64_t)from_below<ROWS>(ih) << 32);
-        if (MODE == 5) high |= (mx1 > j + 1u ? nb1 : 0ull) | (mx2 > j + 1u ? nb2 : 0ull);
-        T = (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)il, LAST) |
-            ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)ih, LAST) << 32);
-        if (MODE == 5) T |= lk.any;
+    uint32_t tl = (uint32_t)s.look | (uint32_t)lk.W, th = (uint32_t)(s.look >> 32) | (uint32_t)(lk.W >> 32);
+    // looked up by a lower group (the lanes above); the walk's by register
+    const uint64_t wl = MODE == 5 ? (mn1 < j ? nb1 : 0ull) | (mn2 < j ? nb2 : 0ull) : 0ull;
+    uint32_t x;
+    uint64_t low = wl | (uint64_t)suffix_or<ROWS>(tl, lane, x) | ((uint64_t)suffix_or<ROWS>(th, lane, x) << 32);
+    bool n1 = (nb1 & low) != 0, n2 = (nb2 & low) != 0;
+    const bool z1 = s1, z2 = s2;  // swapped already
+    if (__ballot((n1 && !z1) || (n2 && !z2))) {
+        bool ch;
+        do {
+            const bool f1 = n1, f2 = n2;
+            s1 = z1 || f1; s2 = z2 || f2;
+            r1 = s1 ? sr1 : e1 & 0x3Fu; r2 = s2 ? sr2 : e2 & 0x3Fu;
+            s = op_eval(op, r1, r2, f.life);
+            tl = (uint32_t)s.look | (uint32_t)lk.W; th = (uint32_t)(s.look >> 32) | (uint32_t)(lk.W >> 32);
+            low = wl | (uint64_t)suffix_or<ROWS>(tl, lane, x) | ((uint64_t)suffix_or<ROWS>(th, lane, x) << 32);
+            n1 = (nb1 & low) != 0; n2 = (nb2 & low) != 0;
+            ch = (n1 != f1 && !z1) || (n2 != f2 && !z2);
+        } while (__ballot(ch));
     }
+    const uint32_t il = scan_or<ROWS>(tl), ih = scan_or<ROWS>(th);
+    uint64_t high = (uint64_t)from_below<ROWS>(il) | ((uint64_t)from_below<ROWS>(ih) << 32);
+    if (MODE == 5) high |= (mx1 > j + 1u ? nb1 : 0ull) | (mx2 > j + 1u ? nb2 : 0ull);
+    uint64_t T = (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)il, LAST) |
+        ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)ih, LAST) << 32);
+    if (MODE == 5) T |= lk.any;
     // new marks: owned entries looked up whose mark does not stand yet
     f.mk &= ~nb;
     const uint64_t nm = f.own & ~f.mk & ((T & ~nb) | (high & nb));
     f.mk |= nm;
     const uint32_t mr = (uint32_t)__builtin_ctzll(nm | (1ull << 63));
-    const uint32_t mp = hold[mr * HC + hc];
+    const uint32_t mp = hold[mr];
     // the registers written or freed: by any lane, by a higher group
     const uint64_t touch = s.m | ((op & (OP_SELF | (63u << OP_CONST))) ? s.dm : 0ull);
-    uint64_t lost, won;
-    if (MODE == 0) {
-        lost = touch;
-        won = self && l0 ? s.dm : 0ull;
-    } else {
-        const uint32_t il = scan_or<ROWS>((uint32_t)touch), ih = scan_or<ROWS>((uint32_t)(touch >> 32));
-        const uint64_t above = (uint64_t)from_below<ROWS>(il) | ((uint64_t)from_below<ROWS>(ih) << 32);
-        lost = (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)il, LAST) |
-               ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)ih, LAST) << 32);
-        won = self ? s.dm & ~above : 0ull;
-    }
+    const uint32_t wl2 = scan_or<ROWS>((uint32_t)touch), wh2 = scan_or<ROWS>((uint32_t)(touch >> 32));
+    const uint64_t above = (uint64_t)from_below<ROWS>(wl2) | ((uint64_t)from_below<ROWS>(wh2) << 32);
+    const uint64_t lost = (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)wl2, LAST) |
+           ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)wh2, LAST) << 32);
+    const uint64_t won = self ? s.dm & ~above : 0ull;
     // the step's commit: swapped operands take the register they were read
     // through, and their flags are cleared (an operand not swapped keeps its
     // entry; without one, this word's row takes the write and its own after it)
@@ -2139,59 +2210,141 @@ DEV void ra_l0_step(const Dev &d, RaL0 &f, uint16_t *ring, uint32_t *hold, uint3
     rb[2u * ((inr ? mp & (OP_ROWS - 1u) : OP_ROWS) * RC + rc) + 1u] = (uint8_t)(1u | (mr << 1));
     if (__builtin_expect(__ballot((nm & (nm - 1)) != 0 || (nm != 0 && !inr)) != 0, 0)) {
         for (uint64_t m = nm; m; m &= m - 1) {
-            const uint32_t r = (uint32_t)__builtin_ctzll(m), p = hold[r * HC + hc];
+            const uint32_t r = (uint32_t)__builtin_ctzll(m), p = hold[r];
             const uint8_t fl = (uint8_t)(1u | (r << 1));
             if (p >= rl) rb[2u * ((p & (OP_ROWS - 1u)) * RC + rc) + 1u] = fl;
             else reinterpret_cast<uint8_t *>(d.sym + f.start)[2u * p + 1u] = fl;
         }
     }
     ring[ws * RC + rc] = (uint16_t)(self ? ((op & OP_ZERO) ? 0u : s.rdr) | (s.rdr << 9) : 0u);
-    hold[(won ? s.rdr : 64u) * HC + hc] = i;
+    hold[won ? s.rdr : 64u] = i;
     f.life = s.life;
     f.own = (f.own & ~lost) | won;
     f.mk &= ~lost;
 }
 
-// Programs of at most 8 functions (one group): the reference's vector loop runs
-// them as one 8-lane vector, and only its lane 0 writes region 0 of
-// register_state.  One wave holds 8 such programs.  The first `solo` programs
-// of the list (the longest) have a wave each, in slot 0, so that no other
-// program's rarer paths (a mark, a state read from HBM) hold up their steps.
-// Latency bound: 1.5 -> 0.59 us a step alone in a wave (a function of 35k words,
-// 52 -> 21 ms).
-__global__ __launch_bounds__(64) void k_ra_group(Dev d, const uint32_t *plist, uint32_t np, uint32_t solo) {
-    __shared__ uint16_t ring[(OP_ROWS + 1) * 64];
-    __shared__ uint32_t hold[65 * 8];
-    const uint32_t lane = threadIdx.x, slot = lane >> 3, k = lane & 7u;
-    const uint32_t pi = blockIdx.x < solo ? (slot == 0 ? blockIdx.x : np) : solo + (blockIdx.x - solo) * 8u + slot;
-    const uint32_t prg = pi < np ? plist[pi] : 0xFFFFFFFFu;
-    const uint32_t fb = prg != 0xFFFFFFFFu ? d.pf[prg] : 0u;
-    const uint32_t nf = prg != 0xFFFFFFFFu ? d.pf[prg + 1] - fb : 0u;
-    if (nf > 8u) atomicOr(d.flags, EF_OOB);
-    const bool act = k < nf && nf <= 8u && d.cflag[prg] == 0;  // (flagged programs: k_ra_serial's)
-    RaL0 f{act ? d.fstarts[fb + k] : 0u, act ? d.fsizes[fb + k] : 0u, 0x1Full, 0, 0};
-    uint32_t wmax = f.size;
-    for (int s = 32; s > 0; s >>= 1) { uint32_t o = __shfl_xor(wmax, s, 64); wmax = wmax > o ? wmax : o; }
-    const uint32_t *ops = d.ops + f.start;
-    const RaLooks none{0, nullptr, nullptr, 0};
-    OpBlock ob;
-    ob.load(ops, 0, f.size);
-    __syncthreads();
-    for (uint32_t i = 0; i < wmax; i += 4) {
-        ob.step4(ops, i, f.size);
-        ra_evict<64>(d, f, ring, lane, i);
-#pragma unroll
-        for (uint32_t q = 0; q < 4; ++q) {
-            const uint32_t op = (int32_t)(i + q) < (int32_t)f.size ? ob.cur[0].o[q] : 0u;
-            ra_l0_step<0, 64, 8>(d, f, ring, hold, lane, slot, lane, k == 0, 0u, i, i + q, op, none);
+// The lane-0 function of a program of one group, on a whole wave as walk_one
+// (`own`, `mk` and the state as in ra_l0_step): every entry of region 0 is this
+// function's, so a step needs of the others only their lookups, a mask a step
+// (`wlo`, `whi`: those of the block's steps, by lane).  hold is a vector register,
+// lane = entry.  A change to a state of an earlier block goes to HBM, to the LDS
+// ring and, within the last 64 words, to ringv.
+// Latency bound: 1.5 -> 0.32 us a step (0.59 as a lane of eight programs' wave):
+// 64 stress programs, whose longest functions these are mostly, 42 -> 32 ms.
+constexpr uint32_t ONE_OLD = 4096;    // words of the LDS ring
+constexpr uint32_t ONE_BLOCK = 32;    // steps of a block: a chunk of the walk's rows
+__global__ __launch_bounds__(64) void k_ra_lane0_one(Dev d, const Ra0Prog *progs, const unsigned long long *mask_all,
+                                                     uint64_t mstride, uint32_t mcopies, const uint32_t *done,
+                                                     const uint32_t *need) {
+    __shared__ uint16_t old[ONE_OLD];
+    const uint32_t lane = threadIdx.x;
+    const Ra0Prog pg = progs[blockIdx.x];
+    if (d.cflag[pg.prg]) return;  // k_ra_serial's
+    if (pg.L > 1u) { if (lane == 0) atomicOr(d.flags, EF_OOB); return; }
+    const uint32_t start = uniform(d.fstarts[pg.fbase]), size = uniform(d.fsizes[pg.fbase]), rows = pg.rows;
+    const uint32_t *pdone = done && pg.cbase != RA0_NOPUB ? done + pg.cbase : nullptr;
+    const uint32_t *pneed = pdone ? need + pg.cbase : nullptr;
+    const unsigned long long *tab = mask_all + pg.gbase;
+    const uint64_t m1 = mcopies > 1 ? mstride : 0u;
+    bool wok = true;
+    uint8_t *symb = reinterpret_cast<uint8_t *>(d.sym + start);
+    uint32_t ringv = 0, holdv = 0;
+    uint64_t life = 0x1Full, own = 0, mk = 0;
+    // ops and lookups of the steps i + lane, lane < ONE_BLOCK (rows past the last: none)
+    struct Block { uint32_t op; unsigned long long a, b; };
+    auto load = [&](uint32_t i) {
+        if (pdone && i < rows) ra0_wait(d, pdone, pneed, i / WALK_PUB, wok);
+        const uint32_t x = i + lane, e = min(x, rows - 1u);
+        Block r{0, 0, 0};
+        if (lane < ONE_BLOCK) {
+            r.op = d.ops[start + min(x, size)];
+            if (x < rows) { r.a = tab[e]; r.b = tab[m1 + e]; }
+        }
+        return r;
+    };
+    // sets a state of word p at step i of the block from b
+    auto put = [&](uint32_t p, uint32_t i, uint32_t b, uint32_t st) {
+        if (i - p < 64u) ringv = wrlane(ringv, p & 63u, st);
+        if (p < b) {
+            if (i - p < ONE_OLD) old[p % ONE_OLD] = (uint16_t)st;
+            d.sym[start + p] = (uint16_t)st;
+        }
+    };
+    Block nx = load(0);
+    for (uint32_t b = 0; b < size; b += ONE_BLOCK) {
+        uint32_t cur = nx.op, wlo = (uint32_t)(nx.a | nx.b), whi = (uint32_t)((nx.a | nx.b) >> 32);
+        asm volatile("" : "+v"(cur), "+v"(wlo), "+v"(whi) : : "memory");  // waited for before the next loads are issued
+        nx = load(b + ONE_BLOCK);
+        const uint32_t n = min(ONE_BLOCK, size - b);
+        for (uint32_t k = 0; k < n; ++k) {
+            const uint32_t i = b + k;
+            const uint32_t op = rdlane(cur, k);
+            const uint64_t W = (uint64_t)rdlane(wlo, k) | ((uint64_t)rdlane(whi, k) << 32);
+            const uint32_t d1 = op & 0xFFu, d2 = (op >> 8) & 0xFFu;
+            uint32_t p1 = i - d1, p2 = i - d2;
+            uint32_t e1 = d1 ? rdlane(ringv, p1 & 63u) : 0u, e2 = d2 ? rdlane(ringv, p2 & 63u) : 0u;
+            if (__builtin_expect((op & (0xC0C0u | OP_FAR1 | OP_FAR2)) != 0, 0)) {
+                const uint4 w = d.w0_f4[start + i];
+                wait_loads();
+                if (op & OP_FAR1) p1 = uniform(w.y) - 64u - start;
+                if (op & OP_FAR2) p2 = uniform(w.z) - 64u - start;
+                // (a word 64 or more back is in a block that has ended)
+                auto state = [&](uint32_t p) {
+                    uint32_t v = i - p < ONE_OLD - 64u ? old[p % ONE_OLD] : d.sym[start + p];
+                    wait_loads();
+                    return uniform(v);
+                };
+                if ((op & OP_FAR1) || d1 > 63u) e1 = state(p1);
+                if ((op & OP_FAR2) || d2 > 63u) e2 = state(p2);
+            }
+            const uint32_t h1 = e1 >> 9, h2 = e2 >> 9;
+            const uint64_t nb = (rdlane(holdv, h1) == p1 ? own & (1ull << h1) : 0ull) |
+                                (rdlane(holdv, h2) == p2 ? own & (1ull << h2) : 0ull);
+            const bool s1 = (e1 & 0x100u) != 0, s2 = (e2 & 0x100u) != 0;
+            const uint32_t r1 = s1 ? ((op & OP_FP) ? 37u : 5u) : e1 & 0x3Fu;
+            const uint32_t r2 = s2 ? ((op & OP_FP) ? 38u : 6u) : e2 & 0x3Fu;
+            const OpStep s = op_eval(op, r1, r2, life);
+            const bool self = (op & OP_SELF) != 0;
+            mk &= ~nb;
+            uint64_t nm = own & ~mk & (s.look | W) & ~nb;
+            mk |= nm;
+            if (s1) put(p1, i, b, r1 | (h1 << 9));
+            if (s2) put(p2, i, b, r2 | (h2 << 9));
+            while (nm) {  // new marks
+                const uint32_t r = (uint32_t)__builtin_ctzll(nm);
+                nm &= nm - 1;
+                const uint32_t p = rdlane(holdv, r);
+                if (i - p < 64u) ringv = wrlane(ringv, p & 63u, rdlane(ringv, p & 63u) | 0x100u);
+                if (p < b) {
+                    if (i - p < ONE_OLD) reinterpret_cast<uint8_t *>(old)[2u * (p % ONE_OLD) + 1u] = (uint8_t)(1u | (r << 1));
+                    symb[2u * (uint64_t)p + 1u] = (uint8_t)(1u | (r << 1));
+                }
+            }
+            ringv = wrlane(ringv, i & 63u, self ? ((op & OP_ZERO) ? 0u : s.rdr) | (s.rdr << 9) : 0u);
+            holdv = wrlane(holdv, s.rdr, i);  // (of an entry not won: not owned, never read)
+            const uint64_t lost = s.m | ((op & (OP_SELF | (63u << OP_CONST))) ? s.dm : 0ull);
+            own = (own & ~lost) | (self ? s.dm : 0ull);
+            mk &= ~lost;
+            life = s.life;
+        }
+        // the block's states (lane x of ringv: word x mod 64)
+        const uint32_t x = (lane - b) & 63u;
+        if (x < n) {
+            d.sym[start + b + x] = (uint16_t)ringv;
+            old[(b + x) % ONE_OLD] = (uint16_t)ringv;
         }
     }
-    ra_flush<64>(d, f, ring, lane);
+    if (rows > size) {  // the row that gathers the steps past the last
+        if (pdone) ra0_wait(d, pdone, pneed, (rows - 1u) / WALK_PUB, wok);
+        const unsigned long long W = tab[rows - 1u] | tab[m1 + rows - 1u];
+        const uint64_t nm = own & ~mk & ((uint64_t)uniform((uint32_t)W) | ((uint64_t)uniform((uint32_t)(W >> 32)) << 32));
+        if ((nm >> lane) & 1u) symb[2u * (uint64_t)holdv + 1u] = (uint8_t)(1u | (lane << 1));
+    }
 }
 
-// The lane-0 functions of a program of 2 to 16 (ROWS 1) or 64 (ROWS 4) groups,
-// in step lockstep on one wave: what the groups exchange in a step goes through
-// ballots and DPP scans of 64-bit register masks, so a step has no barrier.  A
+// The lane-0 functions of a program of 2 to 16 (ROWS 1) or 64 (4) groups, in
+// step lockstep on one wave: what the groups exchange in a step goes
+// through DPP scans of 64-bit register masks, so a step has no barrier.  A
 // second wave fetches the ops and the walk's lookups (one mask per group and
 // step) into LDS, RA0_FETCH steps ahead: the stepping wave then waits for no
 // load, and so for none of its own stores either (they share a counter).
@@ -2264,15 +2417,15 @@ __global__ __launch_bounds__(128) void k_ra_lane0_wave(Dev d, const Ra0Prog *pro
                 const uint32_t kn = (k + q + 1u) % RA0_FETCH;
                 const uint32_t opn = fop[b][kn][col];
                 const unsigned long long Wn = fw[b][kn][col];
-                ra_l0_step<ROWS, NL, 1>(d, f, ring, hold, col, 0u, lane, true, j, i0 + k, i0 + k + q,
-                                        lane < (uint32_t)NL ? op : 0u,
-                                        RaLooks{lane < (uint32_t)NL ? W : 0ull, nullptr, nullptr, 0});
+                ra_l0_step<ROWS, NL>(d, f, ring, hold, col, lane, j, i0 + k, i0 + k + q,
+                                     lane < (uint32_t)NL ? op : 0u,
+                                     RaLooks{lane < (uint32_t)NL ? W : 0ull, nullptr, nullptr, 0});
                 op = opn; W = Wn;
             }
         }
         lds_barrier();  // the next steps are in
     }
-    ra_flush<NL>(d, f, ring, col);
+    if (lane < (uint32_t)NL) ra_flush<NL>(d, f, ring, col);
 }
 
 // ============================================================ small programs
@@ -2308,7 +2461,7 @@ constexpr uint32_t SM_STATE_OFF = 40960; // LDS bytes before the register states
 constexpr uint32_t SM_STATE_MAX = 40960;   // LDS bytes of register states per wave at most (80 KB of
                                            // LDS in all: two waves per compute unit)
 constexpr uint32_t SM_STATE_SMALL = 40960;
-constexpr uint32_t SM_MIN_FUNCS = 9;       // programs of one group keep k_ra_group
+constexpr uint32_t SM_MIN_FUNCS = 9;       // programs of one group keep k_ra_lane0_one
 
 struct SmWave { uint32_t np, state_bytes, prog[SM_PROGS], seg[SM_PROGS]; };
 
@@ -3666,7 +3819,7 @@ __global__ __launch_bounds__(1024) void k_ra_lane0_wg(Dev d, const Ra0Prog *prog
         for (uint32_t q = 0; q < 4; ++q) {
             const uint32_t r = (i + q) % RA0_WROWS;
             const uint32_t op = (int32_t)(i + q) < (int32_t)f.size ? ob.cur[0].o[q] : 0u;
-            ra_l0_step<5, 64, 1>(d, f, ring, hold, lane, 0u, lane, true, f1[0].j, i, i + q, op,
+            ra_l0_step<5, 64>(d, f, ring, hold, lane, lane, f1[0].j, i, i + q, op,
                                  RaLooks{0ull, Wmn[r], Wmx[r], i + q < steps ? Wany[r] : 0ull});
         }
     }

@@ -1,5 +1,5 @@
 """Register allocation's walks at the sizes where their launch changes: programs
-around one group of 8 functions (k_ra_group), around 16 and 64 groups (the
+around one group of 8 functions (k_ra_lane0_one), around 16 and 64 groups (the
 lockstep in one wave, one row of lanes or four) and 256, 960 and 2880 groups (a
 workgroup of one slot of 64 groups a wave or three), alone with walk and lockstep
 overlapped and not, and together in one batch; and operands defined more words
