@@ -2016,6 +2016,23 @@ DEV void ra0_wait(const Dev &d, const uint32_t *done, const uint32_t *need, uint
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
 }
 
+// The same for the wave's 64 chunks from c on: waits until c is published and
+// returns the first chunk not known to be (a lockstep behind the walk then polls
+// once in 64 chunks).
+DEV uint32_t ra0_wait_run(const Dev &d, const uint32_t *done, const uint32_t *need, uint32_t c, uint32_t n, bool &ok) {
+    if (!ok) return n;
+    const uint32_t x = min(c + (threadIdx.x & 63u), n - 1u);
+    const uint32_t want = need[x];
+    const uint64_t t0 = wall_clock64();
+    uint64_t got;
+    while (got = __ballot(__hip_atomic_load(&done[x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= want), (got & 1u) == 0) {
+        if (wall_clock64() - t0 > RA0_WAIT_TICKS) { ok = false; atomicOr(d.flags, EF_WAIT); return n; }
+        __builtin_amdgcn_s_sleep(8);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    return c + (got == ~0ull ? 64u : (uint32_t)__builtin_ctzll(~got));
+}
+
 // ---------------------------------------------- lane-0 functions in one wave
 // Region 0 of the reference's register_state holds the last lane-0 write per
 // physical register; every lookup of any function at step i reads its
@@ -2227,12 +2244,20 @@ DEV void ra_l0_step(const Dev &d, RaL0 &f, uint16_t *ring, uint32_t *hold, uint3
 // (`own`, `mk` and the state as in ra_l0_step): every entry of region 0 is this
 // function's, so a step needs of the others only their lookups, a mask a step
 // (`wlo`, `whi`: those of the block's steps, by lane).  hold is a vector register,
-// lane = entry.  A change to a state of an earlier block goes to HBM, to the LDS
-// ring and, within the last 64 words, to ringv.
-// Latency bound: 1.5 -> 0.32 us a step (0.59 as a lane of eight programs' wave):
-// 64 stress programs, whose longest functions these are mostly, 42 -> 32 ms.
+// lane = entry, and ringv the states of this block's words and the last one's: those
+// before are in HBM and an LDS ring, and a change to one goes to both.
+// Latency bound, ~7 cycles for each of a step's ~90 scalar instructions; the rare
+// cases (an operand ONE_BLOCK or more back, a marked operand, a mark of an old
+// word or a second one) are out of line.  1.5 -> 0.24 us a step (0.59 as a lane of
+// eight programs' wave; 0.32 with every mark a loop and the walk's progress
+// polled each block): a stress program of 91k steps, 32 -> 26.6 ms.
 constexpr uint32_t ONE_OLD = 4096;    // words of the LDS ring
 constexpr uint32_t ONE_BLOCK = 32;    // steps of a block: a chunk of the walk's rows
+constexpr uint32_t ONE_SELF = 23, ONE_WRITES = 28;  // bits of an op here: OP_SELF, and one set a block
+static_assert(OP_SELF == 1u << ONE_SELF, "");
+// first bit that is 1 (0), ~0 if there is none
+DEV uint32_t ff1(uint64_t x) { uint32_t r; asm("s_ff1_i32_b64 %0, %1" : "=s"(r) : "s"(x)); return r; }
+DEV uint32_t ff0(uint32_t x) { uint32_t r; asm("s_ff0_i32_b32 %0, %1" : "=s"(r) : "s"(x)); return r; }
 __global__ __launch_bounds__(64) void k_ra_lane0_one(Dev d, const Ra0Prog *progs, const unsigned long long *mask_all,
                                                      uint64_t mstride, uint32_t mcopies, const uint32_t *done,
                                                      const uint32_t *need) {
@@ -2252,8 +2277,10 @@ __global__ __launch_bounds__(64) void k_ra_lane0_one(Dev d, const Ra0Prog *progs
     uint64_t life = 0x1Full, own = 0, mk = 0;
     // ops and lookups of the steps i + lane, lane < ONE_BLOCK (rows past the last: none)
     struct Block { uint32_t op; unsigned long long a, b; };
+    uint32_t ready = 0;  // chunks known to be published
     auto load = [&](uint32_t i) {
-        if (pdone && i < rows) ra0_wait(d, pdone, pneed, i / WALK_PUB, wok);
+        if (pdone && i < rows && i / WALK_PUB >= ready)
+            ready = uniform(ra0_wait_run(d, pdone, pneed, i / WALK_PUB, (rows - 1u) / WALK_PUB + 1u, wok));
         const uint32_t x = i + lane, e = min(x, rows - 1u);
         Block r{0, 0, 0};
         if (lane < ONE_BLOCK) {
@@ -2262,12 +2289,12 @@ __global__ __launch_bounds__(64) void k_ra_lane0_one(Dev d, const Ra0Prog *progs
         }
         return r;
     };
-    // sets a state of word p at step i of the block from b
-    auto put = [&](uint32_t p, uint32_t i, uint32_t b, uint32_t st) {
-        if (i - p < 64u) ringv = wrlane(ringv, p & 63u, st);
-        if (p < b) {
-            if (i - p < ONE_OLD) old[p % ONE_OLD] = (uint16_t)st;
-            d.sym[start + p] = (uint16_t)st;
+    // the states of the words [lo, hi), hi - lo <= 64, leave the ring
+    auto flush = [&](uint32_t lo, uint32_t hi) {
+        const uint32_t w = lo + ((lane - lo) & 63u);
+        if (w < hi) {
+            d.sym[start + w] = (uint16_t)ringv;
+            old[w % ONE_OLD] = (uint16_t)ringv;
         }
     };
     Block nx = load(0);
@@ -2275,64 +2302,88 @@ __global__ __launch_bounds__(64) void k_ra_lane0_one(Dev d, const Ra0Prog *progs
         uint32_t cur = nx.op, wlo = (uint32_t)(nx.a | nx.b), whi = (uint32_t)((nx.a | nx.b) >> 32);
         asm volatile("" : "+v"(cur), "+v"(wlo), "+v"(whi) : : "memory");  // waited for before the next loads are issued
         nx = load(b + ONE_BLOCK);
-        const uint32_t n = min(ONE_BLOCK, size - b);
+        // the ring holds the words from kept on; the lanes of this block's are 0
+        // until they are written, which is also the state of no operand
+        const uint32_t kept = b >= ONE_BLOCK ? b - ONE_BLOCK : 0u;
+        if (b >= 2u * ONE_BLOCK) flush(b - 2u * ONE_BLOCK, kept);
+        if (((lane - b) & 63u) < ONE_BLOCK) ringv = 0;
+        const uint64_t oldown = __ballot(holdv < kept);  // entries whose word may have left the ring
+        // state of a word from its register, as a factor; whether it ends its entry's holding
+        const uint32_t fac = (cur & OP_SELF) ? ((cur & OP_ZERO) ? 0x200u : 0x201u) : 0u;
+        cur |= (cur & (OP_SELF | (63u << OP_CONST))) ? 1u << ONE_WRITES : 0u;
+        const uint32_t n = uniform(min(ONE_BLOCK, size - b));
         for (uint32_t k = 0; k < n; ++k) {
             const uint32_t i = b + k;
             const uint32_t op = rdlane(cur, k);
             const uint64_t W = (uint64_t)rdlane(wlo, k) | ((uint64_t)rdlane(whi, k) << 32);
-            const uint32_t d1 = op & 0xFFu, d2 = (op >> 8) & 0xFFu;
-            uint32_t p1 = i - d1, p2 = i - d2;
-            uint32_t e1 = d1 ? rdlane(ringv, p1 & 63u) : 0u, e2 = d2 ? rdlane(ringv, p2 & 63u) : 0u;
-            if (__builtin_expect((op & (0xC0C0u | OP_FAR1 | OP_FAR2)) != 0, 0)) {
-                const uint4 w = d.w0_f4[start + i];
-                wait_loads();
-                if (op & OP_FAR1) p1 = uniform(w.y) - 64u - start;
-                if (op & OP_FAR2) p2 = uniform(w.z) - 64u - start;
-                // (a word 64 or more back is in a block that has ended)
-                auto state = [&](uint32_t p) {
-                    uint32_t v = i - p < ONE_OLD - 64u ? old[p % ONE_OLD] : d.sym[start + p];
+            uint32_t p1 = i - (op & 0xFFu), p2 = i - ((op >> 8) & 0xFFu);
+            uint32_t e1 = rdlane(ringv, p1 & 63u), e2 = rdlane(ringv, p2 & 63u);
+            if (__builtin_expect((op & (0xE0E0u | OP_FAR1 | OP_FAR2)) != 0, 0)) {
+                if (op & (OP_FAR1 | OP_FAR2)) {
+                    const uint4 w = d.w0_f4[start + i];
                     wait_loads();
+                    if (op & OP_FAR1) p1 = uniform(w.y) - 64u - start;
+                    if (op & OP_FAR2) p2 = uniform(w.z) - 64u - start;
+                }
+                // states of words that may have left the ring, then those a mark is
+                // flipped back in (rs1's and rs2's word may be the same)
+                auto look = [&](uint32_t p, uint32_t e) {
+                    if (p >= kept) return e;
+                    uint32_t v;
+                    if (i - p < ONE_OLD - 64u) v = old[p % ONE_OLD];
+                    else { v = d.sym[start + p]; wait_loads(); }
                     return uniform(v);
                 };
-                if ((op & OP_FAR1) || d1 > 63u) e1 = state(p1);
-                if ((op & OP_FAR2) || d2 > 63u) e2 = state(p2);
+                auto flip = [&](uint32_t p, uint32_t e, uint32_t r) {
+                    if (p >= kept || !(e & 0x100u)) return e;
+                    const uint32_t v = (e & ~0x1FFu) | r | ((op & OP_FP) ? 32u : 0u);
+                    if (i - p < ONE_OLD) old[p % ONE_OLD] = (uint16_t)v;
+                    d.sym[start + p] = (uint16_t)v;
+                    return v;
+                };
+                e1 = look(p1, e1);
+                e2 = look(p2, e2);
+                e1 = flip(p1, e1, 5u);
+                e2 = flip(p2, e2, 6u);
+            }
+            if (__builtin_expect(((e1 | e2) & 0x100u) != 0, 0)) {  // marked operands: flipped back
+                const uint32_t fp = (op & OP_FP) ? 32u : 0u;
+                if (e1 & 0x100u) { e1 = (e1 & ~0x1FFu) | fp | 5u; ringv = wrlane(ringv, p1 & 63u, e1); }
+                if (e2 & 0x100u) { e2 = (e2 & ~0x1FFu) | fp | 6u; ringv = wrlane(ringv, p2 & 63u, e2); }
             }
             const uint32_t h1 = e1 >> 9, h2 = e2 >> 9;
-            const uint64_t nb = (rdlane(holdv, h1) == p1 ? own & (1ull << h1) : 0ull) |
-                                (rdlane(holdv, h2) == p2 ? own & (1ull << h2) : 0ull);
-            const bool s1 = (e1 & 0x100u) != 0, s2 = (e2 & 0x100u) != 0;
-            const uint32_t r1 = s1 ? ((op & OP_FP) ? 37u : 5u) : e1 & 0x3Fu;
-            const uint32_t r2 = s2 ? ((op & OP_FP) ? 38u : 6u) : e2 & 0x3Fu;
-            const OpStep s = op_eval(op, r1, r2, life);
-            const bool self = (op & OP_SELF) != 0;
+            const uint64_t nb = own & ((rdlane(holdv, h1) == p1 ? 1ull << h1 : 0ull) | (rdlane(holdv, h2) == p2 ? 1ull << h2 : 0ull));
+            // the step's lookups, as op_eval
+            const uint64_t m = ((1ull << (e1 & 63u)) | (1ull << (e2 & 63u))) & ~1ull, cl = life & ~m;
+            const uint32_t fr = ff0((uint32_t)cl), al = fr != ~0u ? fr : 5u;
+            const uint32_t rdr = (op & OP_ALLOC) ? al : (op >> OP_CONST) & 63u;
+            const uint64_t dm = 1ull << rdr;
             mk &= ~nb;
-            uint64_t nm = own & ~mk & (s.look | W) & ~nb;
+            uint64_t nm = own & ~(mk | nb) & ((((m & life) | (dm & cl)) & ~1ull) | W);
             mk |= nm;
-            if (s1) put(p1, i, b, r1 | (h1 << 9));
-            if (s2) put(p2, i, b, r2 | (h2 << 9));
-            while (nm) {  // new marks
-                const uint32_t r = (uint32_t)__builtin_ctzll(nm);
-                nm &= nm - 1;
-                const uint32_t p = rdlane(holdv, r);
-                if (i - p < 64u) ringv = wrlane(ringv, p & 63u, rdlane(ringv, p & 63u) | 0x100u);
-                if (p < b) {
+            // new marks: mostly none or one, of a word in the ring
+            const uint64_t more = (nm & (nm - 1)) | (nm & oldown);
+            const uint32_t q = rdlane(holdv, ff1(nm) & 63u) & 63u, fl = nm ? 0x100u : 0u;
+            ringv = wrlane(ringv, q, rdlane(ringv, q) | (more ? 0u : fl));
+            if (__builtin_expect(more != 0, 0)) {
+                for (; nm; nm &= nm - 1) {
+                    const uint32_t r = (uint32_t)__builtin_ctzll(nm), p = rdlane(holdv, r);
+                    if (p >= kept) { ringv = wrlane(ringv, p & 63u, rdlane(ringv, p & 63u) | 0x100u); continue; }
                     if (i - p < ONE_OLD) reinterpret_cast<uint8_t *>(old)[2u * (p % ONE_OLD) + 1u] = (uint8_t)(1u | (r << 1));
                     symb[2u * (uint64_t)p + 1u] = (uint8_t)(1u | (r << 1));
                 }
             }
-            ringv = wrlane(ringv, i & 63u, self ? ((op & OP_ZERO) ? 0u : s.rdr) | (s.rdr << 9) : 0u);
-            holdv = wrlane(holdv, s.rdr, i);  // (of an entry not won: not owned, never read)
-            const uint64_t lost = s.m | ((op & (OP_SELF | (63u << OP_CONST))) ? s.dm : 0ull);
-            own = (own & ~lost) | (self ? s.dm : 0ull);
+            ringv = wrlane(ringv, i & 63u, rdr * rdlane(fac, k));
+            holdv = wrlane(holdv, rdr, i);  // (of an entry not won: not owned, never read)
+            const uint64_t lost = m | ((uint64_t)((op >> ONE_WRITES) & 1u) << rdr);
+            own = (own & ~lost) | ((uint64_t)((op >> ONE_SELF) & 1u) << rdr);
             mk &= ~lost;
-            life = s.life;
+            life = cl | dm;
         }
-        // the block's states (lane x of ringv: word x mod 64)
-        const uint32_t x = (lane - b) & 63u;
-        if (x < n) {
-            d.sym[start + b + x] = (uint16_t)ringv;
-            old[(b + x) % ONE_OLD] = (uint16_t)ringv;
-        }
+    }
+    if (size) {
+        const uint32_t last = (size - 1u) / ONE_BLOCK * ONE_BLOCK;  // the last block's first word
+        flush(last >= ONE_BLOCK ? last - ONE_BLOCK : 0u, size);
     }
     if (rows > size) {  // the row that gathers the steps past the last
         if (pdone) ra0_wait(d, pdone, pneed, (rows - 1u) / WALK_PUB, wok);
