@@ -836,84 +836,31 @@ DEV uint32_t stop_bits(const Seg &g, int32_t p, const int32_t *skey, uint32_t i)
     return (!(k < p) ? 1u : 0u) | (!(p < k) ? 2u : 0u);
 }
 
-// Per-tile counts of left and right stops over the active list.
+// Compaction of the stops: Lpos[k] / Rpos[k] = position of the k-th left / right
+// stop of the level; base[s] = counts before range s, *total those of the level.
+// One pass over the active list: tiles in ticket order, both counts carried by
+// decoupled look-back as in k_scan_dlb, a status word each (the ticket counter is
+// word 2 * cap), all zero before the launch.
+// (Three launches, a reduction before and its scan between, took 17 us a level on
+// 50k nodes and read the keys twice: 61 us a level of 16M.)
 // The level kernels read the level's counts from the device (lv[0] active
 // elements, lv[1] ranges) and are launched on grids sized for an upper bound
 // of them; workgroups past the counts exit.
-__global__ __launch_bounds__(SCAN_BLOCK) void k_sortlvl_reduce(const Seg *segs, const uint32_t *lv,
-                                                               const int32_t *pivot, const int32_t *skey,
-                                                               uint2 *tile_sums) {
-    __shared__ uint32_t sL[SCAN_BLOCK / 64], sR[SCAN_BLOCK / 64];
-    const uint32_t A = lv[0], m = lv[1];
-    if (blockIdx.x * (uint32_t)SCAN_TILE >= A) return;
-    const SegWindow wd = seg_window(segs, m, A, blockIdx.x * (uint32_t)SCAN_TILE, (uint32_t)SCAN_TILE);
-    const uint32_t a0 = blockIdx.x * (uint32_t)SCAN_TILE + threadIdx.x * SCAN_ITEMS;
-    uint32_t cl = 0, cr = 0;
-    if (a0 < A) {
-        SegWalk w(segs, m, wd, a0);
-        int32_t p = pivot[w.s];
-        for (int k = 0; k < SCAN_ITEMS; ++k) {
-            const uint32_t a = a0 + k;
-            if (a >= A) break;
-            const uint32_t s0 = w.s;
-            w.to(a);
-            if (w.s != s0) p = pivot[w.s];
-            const uint32_t b = stop_bits(w.g, p, skey, w.pos(a));
-            cl += b & 1u; cr += b >> 1;
-        }
-    }
-    cl = wave_sum(cl); cr = wave_sum(cr);
-    if ((threadIdx.x & 63) == 0) { sL[threadIdx.x >> 6] = cl; sR[threadIdx.x >> 6] = cr; }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint32_t tl = 0, tr = 0;
-#pragma unroll
-        for (int w = 0; w < SCAN_BLOCK / 64; ++w) { tl += sL[w]; tr += sR[w]; }
-        tile_sums[blockIdx.x] = make_uint2(tl, tr);
-    }
-}
-
-// One workgroup: exclusive scan of (left, right) tile sums in place; totals to *total.
-__global__ __launch_bounds__(1024) void k_scan_tiles2(uint2 *sums, const uint32_t *lv, uint2 *total) {
-    __shared__ uint32_t wl[16], wr[16];
-    __shared__ uint32_t cl, cr;
-    const uint32_t ntiles = (uint32_t)((lv[0] + SCAN_TILE - 1) / SCAN_TILE);
-    const uint32_t lane = threadIdx.x & 63u, wid = threadIdx.x >> 6;
-    if (threadIdx.x == 0) { cl = 0; cr = 0; }
-    __syncthreads();
-    for (uint32_t b = 0; b < ntiles; b += 1024) {
-        const uint32_t i = b + threadIdx.x;
-        const uint2 v = i < ntiles ? sums[i] : make_uint2(0, 0);
-        const uint32_t xl = wave_incl_scan(v.x, lane), xr = wave_incl_scan(v.y, lane);
-        if (lane == 63) { wl[wid] = xl; wr[wid] = xr; }
-        __syncthreads();
-        uint32_t pl = cl, pr = cr, al = 0, ar = 0;
-        for (uint32_t w = 0; w < 16; ++w) {
-            if (w < wid) { pl += wl[w]; pr += wr[w]; }
-            al += wl[w]; ar += wr[w];
-        }
-        if (i < ntiles) sums[i] = make_uint2(pl + xl - v.x, pr + xr - v.y);
-        __syncthreads();
-        if (threadIdx.x == 0) { cl += al; cr += ar; }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) *total = make_uint2(cl, cr);
-}
-
-// Compaction of the stops: Lpos[k] / Rpos[k] = position of the k-th left / right
-// stop of the level; base[s] = counts before range s.
-__global__ __launch_bounds__(SCAN_BLOCK) void k_sortlvl_down(const Seg *segs, const uint32_t *lv,
+__global__ __launch_bounds__(SCAN_BLOCK) void k_sortlvl_scan(const Seg *segs, const uint32_t *lv,
                                                              const int32_t *pivot, const int32_t *skey,
-                                                             const uint2 *tile_pre, uint32_t *Lpos, uint32_t *Rpos,
-                                                             uint2 *base) {
-    __shared__ uint32_t sL[SCAN_BLOCK / 64], sR[SCAN_BLOCK / 64];
+                                                             unsigned long long *status, uint32_t cap, uint2 *total,
+                                                             uint32_t *Lpos, uint32_t *Rpos, uint2 *base) {
+    __shared__ uint32_t sL[SCAN_BLOCK / 64], sR[SCAN_BLOCK / 64], s_tile, pL, pR;
     const uint32_t A = lv[0], m = lv[1];
     if (blockIdx.x * (uint32_t)SCAN_TILE >= A) return;
     // the tile's stops, staged: its left and right stops are each one
     // contiguous range of Lpos / Rpos, written out coalesced at the end
     __shared__ uint32_t stL[SCAN_TILE], stR[SCAN_TILE];
-    const SegWindow wd = seg_window(segs, m, A, blockIdx.x * (uint32_t)SCAN_TILE, (uint32_t)SCAN_TILE);
-    const uint32_t a0 = blockIdx.x * (uint32_t)SCAN_TILE + threadIdx.x * SCAN_ITEMS;
+    if (threadIdx.x == 0) s_tile = atomicAdd(reinterpret_cast<uint32_t *>(status + 2 * (uint64_t)cap), 1u);
+    __syncthreads();
+    const uint32_t tile = s_tile;
+    const SegWindow wd = seg_window(segs, m, A, tile * (uint32_t)SCAN_TILE, (uint32_t)SCAN_TILE);
+    const uint32_t a0 = tile * (uint32_t)SCAN_TILE + threadIdx.x * SCAN_ITEMS;
     uint32_t bits = 0, cl = 0, cr = 0;  // 2 bits per item
     if (a0 < A) {
         SegWalk w(segs, m, wd, a0);
@@ -933,10 +880,48 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_sortlvl_down(const Seg *segs, co
     const uint32_t xl = wave_incl_scan(cl, lane), xr = wave_incl_scan(cr, lane);
     if (lane == 63) { sL[wid] = xl; sR[wid] = xr; }
     __syncthreads();
-    const uint32_t tL = tile_pre[blockIdx.x].x, tR = tile_pre[blockIdx.x].y;
+    uint32_t nL = 0, nR = 0;
     uint32_t rl = xl - cl, rr = xr - cr;  // offsets within the tile's ranges
 #pragma unroll
-    for (int w = 0; w < SCAN_BLOCK / 64; ++w) if ((uint32_t)w < wid) { rl += sL[w]; rr += sR[w]; }
+    for (int w = 0; w < SCAN_BLOCK / 64; ++w) {
+        if ((uint32_t)w < wid) { rl += sL[w]; rr += sR[w]; }
+        nL += sL[w]; nR += sR[w];
+    }
+    if (wid == 0) {
+        auto put = [&](uint32_t l, uint32_t r, uint64_t flag) {
+            __hip_atomic_store(status + 2u * tile, (unsigned long long)l | flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(status + 2u * tile + 1u, (unsigned long long)r | flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        };
+        if (lane == 0) put(nL, nR, tile == 0 ? SCAN_INCL : SCAN_AGG);
+        uint32_t l = 0, r = 0;
+        for (int64_t j = (int64_t)tile - 1; j >= 0;) {  // nearest predecessor not yet summed (lane 0 reads it)
+            const int64_t idx = j - (int64_t)lane;
+            unsigned long long sl = SCAN_INCL, sr = SCAN_INCL;
+            if (idx >= 0) {
+                sl = __hip_atomic_load(status + 2 * idx, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                sr = __hip_atomic_load(status + 2 * idx + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            // (a tile of which only one word is there, or is inclusive, is read again)
+            const uint32_t fl = sl >> 32 == sr >> 32 ? (uint32_t)(sl >> 32) : 0u;
+            const uint64_t incl = __ballot(fl == 2u), none = __ballot(fl == 0u);
+            const uint32_t stop = incl ? (uint32_t)__builtin_ctzll(incl) : 64u;
+            if (none && (uint32_t)__builtin_ctzll(none) < stop) {
+                __builtin_amdgcn_s_sleep(1);
+                continue;
+            }
+            l += wave_sum(lane <= stop ? (uint32_t)sl : 0u);
+            r += wave_sum(lane <= stop ? (uint32_t)sr : 0u);
+            if (incl) break;
+            j -= 64;
+        }
+        if (lane == 0) {
+            if (tile > 0) put(l + nL, r + nR, SCAN_INCL);
+            pL = l; pR = r;
+            if ((tile + 1u) * (uint64_t)SCAN_TILE >= A) *total = make_uint2(l + nL, r + nR);
+        }
+    }
+    __syncthreads();
+    const uint32_t tL = pL, tR = pR;
     if (a0 < A) {
         SegWalk w(segs, m, wd, a0);
         for (int k = 0; k < SCAN_ITEMS; ++k) {
@@ -950,9 +935,6 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_sortlvl_down(const Seg *segs, co
             if (b & 2u) stR[rr++] = i;
         }
     }
-    uint32_t nL = 0, nR = 0;
-#pragma unroll
-    for (int w = 0; w < SCAN_BLOCK / 64; ++w) { nL += sL[w]; nR += sR[w]; }
     __syncthreads();
     for (uint32_t k = threadIdx.x; k < nL; k += SCAN_BLOCK) Lpos[tL + k] = stL[k];
     for (uint32_t k = threadIdx.x; k < nR; k += SCAN_BLOCK) Rpos[tR + k] = stR[k];
@@ -991,9 +973,11 @@ DEV uint32_t uniform_final(uint32_t a, uint32_t b, uint32_t pos) {
 }
 
 __global__ void k_sort_search(const Seg *segs, const uint32_t *lv, const uint2 *base, const uint2 *total,
-                              const uint32_t *Lpos, const uint32_t *Rpos, SegCut *cuts) {
+                              const uint32_t *Lpos, const uint32_t *Rpos, SegCut *cuts,
+                              unsigned long long *qa_next) {
     const uint32_t m = lv[1];
     uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s == 0) *qa_next = 0ull;  // the counts that k_sort_plan adds to
     if (s >= m) return;
     uint32_t first = segs[s].first, last = segs[s].last;
     const uint2 b0 = base[s], b1 = s + 1 < m ? base[s + 1] : *total;
@@ -1024,8 +1008,14 @@ __global__ void k_sort_search(const Seg *segs, const uint32_t *lv, const uint2 *
 // consecutive pairs (coalesced stop lists).
 __global__ __launch_bounds__(256) void k_sort_swap(const Seg *segs, const uint32_t *lv, const SegCut *cuts,
                                                    const uint32_t *Lpos, const uint32_t *Rpos, uint32_t *sidx,
-                                                   int32_t *skey) {
+                                                   int32_t *skey, unsigned long long *status_next, uint32_t cap) {
     const uint32_t A = lv[0], m = lv[1];
+    static_assert(256 * SCAN_ITEMS == SCAN_TILE, "a tile a workgroup");
+    if (threadIdx.x == 0) {  // cleared for the next level's scan, of no more tiles
+        status_next[2 * (uint64_t)blockIdx.x] = 0ull;
+        status_next[2 * (uint64_t)blockIdx.x + 1] = 0ull;
+        if (blockIdx.x == 0) status_next[2 * (uint64_t)cap] = 0ull;
+    }
     if (blockIdx.x * 256u * SCAN_ITEMS >= A) return;
     const SegWindow wd = seg_window(segs, m, A, blockIdx.x * 256u * SCAN_ITEMS, 256u * SCAN_ITEMS);
     const uint32_t a0 = blockIdx.x * 256u * SCAN_ITEMS + threadIdx.x;
@@ -1051,10 +1041,10 @@ __global__ __launch_bounds__(256) void k_sort_swap(const Seg *segs, const uint32
 // not take (never, by construction; the host reports it as an internal error).
 struct SortCnt { unsigned long long qa[2], ue; uint32_t nheap, nloc, bad, pad; };
 
-// Ranges of at most SORT_LOCAL elements finish in one workgroup's LDS
+// Ranges of at most SORT_LOCAL (or SORT_LOCAL_FEW) elements finish in one workgroup's LDS
 // (k_sort_local): k_sort_plan lists them (median already moved to first)
 // instead of the next level.
-constexpr uint32_t SORT_LOCAL = 2048;
+constexpr uint32_t SORT_LOCAL = 2048, SORT_LOCAL_FEW = 8192;
 
 DEV uint32_t block_excl_scan(uint32_t v, uint32_t *tmp /* 16 */, uint32_t &total) {
     const uint32_t lane = threadIdx.x & 63u, wid = threadIdx.x >> 6;
@@ -1079,7 +1069,7 @@ __global__ __launch_bounds__(1024) void k_sort_plan(const Seg *segs, const SegCu
                                                     Seg *next, int32_t *next_pivot, Seg *heap, Seg *uni,
                                                     Seg *loc, int32_t *loc_pivot,
                                                     unsigned long long *qa_next, SortCnt *cnt, uint8_t *bound,
-                                                    uint32_t *sidx, int32_t *skey) {
+                                                    uint32_t *sidx, int32_t *skey, uint32_t lcap) {
     __shared__ uint32_t tmp[16];
     __shared__ uint32_t base[6];
     const uint32_t m = lv[1];
@@ -1092,8 +1082,8 @@ __global__ __launch_bounds__(1024) void k_sort_plan(const Seg *segs, const SegCu
     const uint32_t lim = g.limit - 1;
     const uint32_t c0 = ct.cut - g.first, c1 = g.last - ct.cut;
     const bool r0 = v && !un && c0 > 16 && lim > 0, r1 = v && !un && c1 > 16 && lim > 0;
-    const bool n0 = r0 && c0 > SORT_LOCAL, n1 = r1 && c1 > SORT_LOCAL;    // next level
-    const bool l0 = r0 && c0 <= SORT_LOCAL, l1 = r1 && c1 <= SORT_LOCAL;  // finished in LDS
+    const bool n0 = r0 && c0 > lcap, n1 = r1 && c1 > lcap;    // next level
+    const bool l0 = r0 && c0 <= lcap, l1 = r1 && c1 <= lcap;  // finished in LDS
     const bool h0b = v && !un && c0 > 16 && lim == 0, h1b = v && !un && c1 > 16 && lim == 0;
     uint32_t tq, ta, th, tu, te, tl;
     const uint32_t xl = block_excl_scan((l0 ? 1u : 0u) + (l1 ? 1u : 0u), tmp, tl);
@@ -1132,32 +1122,38 @@ __global__ __launch_bounds__(1024) void k_sort_plan(const Seg *segs, const SegCu
 // partitions as the level kernels above (stops, pairs, cut, all-equal ranges
 // in closed form when their recursion fits the limit), the same outputs
 // (boundaries in `bound`, entries of the heap and all-equal lists), its
-// subranges kept in position order.  Thread t holds positions [8t, 8t + 8).
-constexpr uint32_t SORT_LOCAL_SUBS = SORT_LOCAL / 17 + 2;
-__global__ __launch_bounds__(256) void k_sort_local(const Seg *loc, const int32_t *loc_pivot, const SortCnt *cntr,
-                                                    uint32_t *sidx, int32_t *skey, uint8_t *bound, Seg *heap,
-                                                    Seg *uni, SortCnt *cnt) {
-    static_assert(SORT_LOCAL == 256 * 8, "8 positions per thread");
-    __shared__ int32_t K[SORT_LOCAL];
-    __shared__ uint32_t X[SORT_LOCAL];
-    __shared__ uint16_t LP[SORT_LOCAL], RP[SORT_LOCAL];
-    __shared__ uint16_t sf[2][SORT_LOCAL_SUBS], sl[2][SORT_LOCAL_SUBS];
-    __shared__ uint8_t slim[2][SORT_LOCAL_SUBS];
-    __shared__ int32_t spiv[2][SORT_LOCAL_SUBS];
-    __shared__ uint16_t bL[SORT_LOCAL_SUBS], bR[SORT_LOCAL_SUBS], cLs[SORT_LOCAL_SUBS], cRs[SORT_LOCAL_SUBS];
-    __shared__ uint16_t mms[SORT_LOCAL_SUBS], cts[SORT_LOCAL_SUBS];
-    __shared__ uint8_t unis[SORT_LOCAL_SUBS];
-    __shared__ uint32_t tmp[16];
+// subranges kept in position order.  Each thread holds ppt consecutive positions.
+template <uint32_t CAP, uint32_t NT>
+__global__ __launch_bounds__(NT) void k_sort_local(const Seg *loc, const int32_t *loc_pivot, const SortCnt *cntr,
+                                                   uint32_t *sidx, int32_t *skey, uint8_t *bound, Seg *heap,
+                                                   Seg *uni, SortCnt *cnt) {
+    constexpr uint32_t SUBS = CAP / 17 + 2;
+    static_assert(CAP % NT == 0 && CAP / NT <= 16 && SUBS <= NT, "two bits of `bits` a position, a thread a subrange");
+    __shared__ int32_t K[CAP];
+    __shared__ uint32_t X[CAP];
+    __shared__ uint16_t LP[CAP], RP[CAP];
+    __shared__ uint16_t sf[2][SUBS], sl[2][SUBS];
+    __shared__ uint8_t slim[2][SUBS];
+    __shared__ int32_t spiv[2][SUBS];
+    __shared__ uint16_t bL[SUBS + 1], bR[SUBS + 1], cts[SUBS];  // stops before a subrange; its cut
+    __shared__ uint8_t unis[SUBS];
+    __shared__ uint16_t uf[SUBS], ul[SUBS];  // all-equal ranges found
+    __shared__ uint8_t ulim[SUBS];
+    __shared__ uint32_t tmp[16], nnext, nuni;
+    __shared__ unsigned long long ubase;
     if (blockIdx.x >= cntr->nloc) return;
     const uint32_t tid = threadIdx.x;
     const Seg g = loc[blockIdx.x];
     const uint32_t base = g.first, len = g.last - g.first;
-    if (len > SORT_LOCAL || len < 17) { if (tid == 0) atomicOr(&cnt->bad, 1u); return; }
-    for (uint32_t p = tid; p < len; p += 256) { K[p] = skey[base + p]; X[p] = sidx[base + p]; }
-    if (tid == 0) { sf[0][0] = 0; sl[0][0] = (uint16_t)len; slim[0][0] = (uint8_t)g.limit; spiv[0][0] = loc_pivot[blockIdx.x]; }
+    if (len > CAP || len < 17) { if (tid == 0) atomicOr(&cnt->bad, 1u); return; }
+    for (uint32_t p = tid; p < len; p += NT) { K[p] = skey[base + p]; X[p] = sidx[base + p]; }
+    if (tid == 0) {
+        sf[0][0] = 0; sl[0][0] = (uint16_t)len; slim[0][0] = (uint8_t)g.limit; spiv[0][0] = loc_pivot[blockIdx.x];
+        nuni = 0;
+    }
     uint32_t cur = 0, nsub = 1;
     __syncthreads();
-    const uint32_t p0 = tid * 8u;
+    const uint32_t ppt = (len + NT - 1) / NT, p0 = min(tid * ppt, len), pe = min(p0 + ppt, len);
     while (nsub > 0) {
         // stops of this thread's positions: subrange walk from the last one starting at or before p0
         uint32_t s0 = 0;
@@ -1169,105 +1165,113 @@ __global__ __launch_bounds__(256) void k_sort_local(const Seg *loc, const int32_
         uint32_t bits = 0, cl = 0, cr = 0;
         {
             uint32_t s = s0;
-            for (uint32_t k = 0; k < 8; ++k) {
-                const uint32_t p = p0 + k;
-                if (p >= len) break;
+            for (uint32_t p = p0, k = 0; p < pe; ++p, k += 2) {
                 while (s + 1 < nsub && sf[cur][s + 1] <= p) ++s;
                 if (p < sf[cur][s] || p >= sl[cur][s] || p == sf[cur][s]) continue;
                 const int32_t kk = K[p], pv = spiv[cur][s];
                 const uint32_t b = (!(kk < pv) ? 1u : 0u) | (!(pv < kk) ? 2u : 0u);
-                bits |= b << (2 * k);
+                bits |= b << k;
                 cl += b & 1u; cr += b >> 1;
             }
         }
-        // both counts in one scan (each at most SORT_LOCAL, so 16 bits apiece)
+        // both counts in one scan (each at most CAP, so 16 bits apiece)
         uint32_t tot2;
         const uint32_t x2 = block_excl_scan(cl | (cr << 16), tmp, tot2);
-        const uint32_t totL = tot2 & 0xFFFFu, totR = tot2 >> 16;
         uint32_t rl = x2 & 0xFFFFu, rr = x2 >> 16;
         const uint32_t rl0 = rl;
         {
             uint32_t s = s0;
-            for (uint32_t k = 0; k < 8; ++k) {
-                const uint32_t p = p0 + k;
-                if (p >= len) break;
+            for (uint32_t p = p0, k = 0; p < pe; ++p, k += 2) {
                 while (s + 1 < nsub && sf[cur][s + 1] <= p) ++s;
-                if (p == sf[cur][s]) { bL[s] = (uint16_t)rl; bR[s] = (uint16_t)rr; }
-                const uint32_t b = (bits >> (2 * k)) & 3u;
+                if (p == sf[cur][s]) { bL[s] = (uint16_t)rl; bR[s] = (uint16_t)rr; cts[s] = (uint16_t)(p + 1); unis[s] = 0; }
+                const uint32_t b = (bits >> k) & 3u;
                 if (b & 1u) LP[rl++] = (uint16_t)p;
                 if (b & 2u) RP[rr++] = (uint16_t)p;
             }
         }
+        if (tid == 0) { bL[nsub] = (uint16_t)(tot2 & 0xFFFFu); bR[nsub] = (uint16_t)(tot2 >> 16); }
         __syncthreads();
-        // per subrange: stop counts, pairs, cut (k_sort_search)
-        if (tid < nsub) {
-            const uint32_t s = tid, f = sf[cur][s], l = sl[cur][s];
-            const uint32_t eL = s + 1 < nsub ? bL[s + 1] : totL, eR = s + 1 < nsub ? bR[s + 1] : totR;
-            const uint32_t b0 = bL[s], b1 = bR[s], cL = eL - b0, cR = eR - b1;
-            uint32_t lo = 0, hi = cL < cR ? cL : cR;
-            while (lo < hi) {
-                const uint32_t mid = (lo + hi + 1) / 2;
-                if (LP[b0 + mid - 1] < RP[b1 + cR - mid]) lo = mid; else hi = mid - 1;
-            }
-            uint32_t cut = 0xFFFFFFFFu;
-            if (lo + 1 <= cL) cut = LP[b0 + lo];
-            if (lo >= 1) { const uint32_t r = RP[b1 + cR - lo]; if (r < cut) cut = r; }
-            if (cut <= f || cut >= l) cut = f + 1;
-            const uint32_t n = l - f;
-            const bool un = cL == n - 1 && cR == n - 1 && uniform_depth(n) <= slim[cur][s];
-            cLs[s] = (uint16_t)cL; cRs[s] = (uint16_t)cR;
-            mms[s] = (uint16_t)(un ? 0u : lo); cts[s] = (uint16_t)(un ? l : cut); unis[s] = un ? 1 : 0;
-        }
-        __syncthreads();
-        // the pairs' swaps, each by the thread holding its left stop
+        // Each pair's swap, by the thread holding its left stop.  The pairs with
+        // L_k < R_k are the first ones, so each thread tells its own from the two
+        // stops; the one at the first pair that is not (or the last left stop)
+        // sets the cut, as k_sort_search.
         {
             uint32_t s = s0, r = rl0;
-            for (uint32_t k = 0; k < 8; ++k) {
-                const uint32_t p = p0 + k;
-                if (p >= len) break;
+            for (uint32_t p = p0, k = 0; p < pe; ++p, k += 2) {
                 while (s + 1 < nsub && sf[cur][s + 1] <= p) ++s;
-                if (!((bits >> (2 * k)) & 1u)) continue;
-                const uint32_t kk = r++ - bL[s];
-                if (kk < mms[s]) {
-                    const uint32_t q = RP[bR[s] + cRs[s] - 1u - kk];
+                if (!((bits >> k) & 1u)) continue;
+                const uint32_t f = sf[cur][s], l = sl[cur][s], b0 = bL[s], b1 = bR[s];
+                const uint32_t cL = bL[s + 1] - b0, cR = bR[s + 1] - b1, kk = r++ - b0, n = l - f;
+                if (cL == n - 1 && cR == n - 1 && uniform_depth(n) <= slim[cur][s]) {
+                    if (kk == 0) { cts[s] = (uint16_t)l; unis[s] = 1; }
+                    continue;
+                }
+                const uint32_t q = kk < cR ? RP[b1 + cR - 1u - kk] : 0u;          // right stop kk
+                const uint32_t qp = kk - 1u < cR ? RP[b1 + cR - kk] : 0u;         // and kk - 1
+                const bool pair = p < q;
+                uint32_t cut = 0xFFFFFFFFu;
+                if (pair) {
                     const int32_t tk = K[p]; K[p] = K[q]; K[q] = tk;
                     const uint32_t tx = X[p]; X[p] = X[q]; X[q] = tx;
+                    if (kk == cL - 1u) cut = q;
+                } else if (kk == 0u) {
+                    cut = p;
+                } else if (LP[b0 + kk - 1u] < qp) {
+                    cut = min(p, qp);
+                }
+                if (cut > f && cut < l) cts[s] = (uint16_t)cut;  // (first + 1: unreachable after a median-of-three pivot)
+            }
+        }
+        __syncthreads();
+        // children (k_sort_plan): the next subranges in position order, each with
+        // its median moved to first; up to 64 subranges by one wave
+        const uint32_t nx = cur ^ 1u;
+        const bool one = nsub <= 64u;
+        if (!one || tid < 64u) {
+            uint32_t nc = 0, f = 0, l = 0, cut = 0, lim = 0;
+            bool c0n = false, c1n = false;
+            if (tid < nsub) {
+                f = sf[cur][tid]; l = sl[cur][tid]; cut = cts[tid];
+                const uint32_t limit = slim[cur][tid];
+                lim = limit - 1u;
+                if (unis[tid]) {
+                    const uint32_t u = atomicAdd(&nuni, 1u);
+                    uf[u] = (uint16_t)f; ul[u] = (uint16_t)l; ulim[u] = (uint8_t)limit;
+                    bound[base + f] = 2;
+                } else {
+                    bound[base + cut] = 1;
+                    const uint32_t c0 = cut - f, c1 = l - cut;
+                    c0n = c0 > 16 && lim > 0; c1n = c1 > 16 && lim > 0;
+                    if (c0 > 16 && lim == 0) heap[atomicAdd(&cnt->nheap, 1u)] = Seg{base + f, base + cut, 0, 0};
+                    if (c1 > 16 && lim == 0) heap[atomicAdd(&cnt->nheap, 1u)] = Seg{base + cut, base + l, 0, 0};
+                    nc = (c0n ? 1u : 0u) + (c1n ? 1u : 0u);
                 }
             }
-        }
-        __syncthreads();
-        // children (k_sort_plan): the next subranges in position order
-        const uint32_t nx = cur ^ 1u;
-        uint32_t nc = 0, f = 0, l = 0, cut = 0, lim = 0;
-        bool c0n = false, c1n = false;
-        if (tid < nsub) {
-            f = sf[cur][tid]; l = sl[cur][tid]; cut = cts[tid];
-            const uint32_t limit = slim[cur][tid];
-            lim = limit - 1u;
-            if (unis[tid]) {
-                const unsigned long long ue = atomicAdd(&cnt->ue, (1ull << 32) | (unsigned long long)(l - f));
-                uni[(uint32_t)(ue >> 32)] = Seg{base + f, base + l, limit, (uint32_t)ue};
-                bound[base + f] = 2;
+            uint32_t tot, q;
+            if (one) {
+                const uint32_t x = wave_incl_scan(nc, tid);
+                q = x - nc;
+                tot = (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
             } else {
-                bound[base + cut] = 1;
-                const uint32_t c0 = cut - f, c1 = l - cut;
-                c0n = c0 > 16 && lim > 0; c1n = c1 > 16 && lim > 0;
-                if (c0 > 16 && lim == 0) heap[atomicAdd(&cnt->nheap, 1u)] = Seg{base + f, base + cut, 0, 0};
-                if (c1 > 16 && lim == 0) heap[atomicAdd(&cnt->nheap, 1u)] = Seg{base + cut, base + l, 0, 0};
-                nc = (c0n ? 1u : 0u) + (c1n ? 1u : 0u);
+                q = block_excl_scan(nc, tmp, tot);
             }
+            if (c0n) { sf[nx][q] = (uint16_t)f; sl[nx][q] = (uint16_t)cut; slim[nx][q] = (uint8_t)lim; spiv[nx][q] = median_to_first(f, cut, X, K); ++q; }
+            if (c1n) { sf[nx][q] = (uint16_t)cut; sl[nx][q] = (uint16_t)l; slim[nx][q] = (uint8_t)lim; spiv[nx][q] = median_to_first(cut, l, X, K); }
+            if (tid == 0) nnext = tot;
         }
-        uint32_t tot;
-        uint32_t q = block_excl_scan(nc, tmp, tot);
-        if (c0n) { sf[nx][q] = (uint16_t)f; sl[nx][q] = (uint16_t)cut; slim[nx][q] = (uint8_t)lim; ++q; }
-        if (c1n) { sf[nx][q] = (uint16_t)cut; sl[nx][q] = (uint16_t)l; slim[nx][q] = (uint8_t)lim; }
-        __syncthreads();
-        if (tid < tot) spiv[nx][tid] = median_to_first(sf[nx][tid], sl[nx][tid], X, K);
         __syncthreads();
         cur = nx;
-        nsub = tot;
+        nsub = nnext;
     }
-    for (uint32_t p = tid; p < len; p += 256) { skey[base + p] = K[p]; sidx[base + p] = X[p]; }
+    for (uint32_t p = tid; p < len; p += NT) { skey[base + p] = K[p]; sidx[base + p] = X[p]; }
+    const uint32_t nu = nuni;
+    if (nu > 0) {  // the all-equal ranges to their list (ranges << 32 | elements)
+        uint32_t tot;
+        const uint32_t o = block_excl_scan(tid < nu ? (uint32_t)(ul[tid] - uf[tid]) : 0u, tmp, tot);
+        if (tid == 0) ubase = atomicAdd(&cnt->ue, ((unsigned long long)nu << 32) | tot);
+        __syncthreads();
+        if (tid < nu) uni[(uint32_t)(ubase >> 32) + tid] = Seg{base + uf[tid], base + ul[tid], ulim[tid], (uint32_t)ubase + o};
+    }
 }
 
 DEV bool KLESS(const int32_t *skey, uint32_t a, uint32_t b) { return skey[a] < skey[b]; }
@@ -1297,10 +1301,11 @@ DEV void heap_adjust(uint32_t *si, int32_t *sk, uint32_t base, int64_t hole, int
     si[base + hole] = vi; sk[base + hole] = vk;
 }
 
-__global__ void k_sort_heap(const Seg *heap, const uint32_t *heap_cnt, uint32_t *si, int32_t *sk) {
+__global__ void k_sort_heap(const Seg *heap, const uint32_t *heap_cnt, uint32_t *si, int32_t *sk, uint8_t *bound) {
     uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= *heap_cnt) return;
     uint32_t base = heap[s].first;
+    bound[base] = 2;
     int64_t len = heap[s].last - heap[s].first;
     if (len >= 2) {
         for (int64_t parent = (len - 2) / 2;; --parent) {
@@ -1316,27 +1321,40 @@ __global__ void k_sort_heap(const Seg *heap, const uint32_t *heap_cnt, uint32_t 
     }
 }
 
-// Leaves are the ranges between consecutive boundaries; boundaries are marked in
-// `bound` (1 at each range start).  Each boundary thread insertion-sorts its range.
-__global__ void k_sort_insertion(const uint8_t *bound, uint64_t n, uint32_t *si, int32_t *sk) {
-    uint64_t b = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
-    if (b >= n || bound[b] != 1) return;  // 2: an all-equal range, nothing moves
-    uint64_t e = b + 1;
-    while (e < n && !bound[e]) ++e;
-    for (uint64_t i = b + 1; i < e; ++i) {
-        uint32_t vi = si[i]; int32_t vk = sk[i];
-        uint64_t j = i;
-        while (j > b && vk < sk[j - 1]) { si[j] = si[j - 1]; sk[j] = sk[j - 1]; --j; }
-        si[j] = vi; sk[j] = vk;
+// Leaves are the ranges between consecutive boundaries, marked in `bound` (1 at
+// each range start, at most 16 elements, insertion-sorted; 2: an all-equal or a
+// heapsorted range, in which nothing moves).  Insertion sort keeps equal keys in
+// order, so an element's final place is the count of the leaf's elements before
+// it in that order: a thread an element, the tile with 16 more on either side in
+// LDS.  (A thread a leaf sorting it in memory, and a pass for the ranks: 25 + 6 us
+// on 4k nodes.)
+constexpr uint32_t LEAF = 16;
+__global__ __launch_bounds__(256) void k_sort_leaves(const uint8_t *bound, uint64_t n, const uint32_t *si,
+                                                     const int32_t *sk, uint32_t *rank, uint32_t *rinv) {
+    __shared__ int32_t K[256 + 2 * LEAF];
+    __shared__ uint8_t B[256 + 2 * LEAF];
+    const uint64_t t0 = blockIdx.x * (uint64_t)256;
+    for (uint32_t x = threadIdx.x; x < 256u + 2u * LEAF; x += 256u) {
+        const uint64_t i = t0 + x;  // element i - LEAF
+        const bool in = i >= LEAF && i - LEAF < n;
+        K[x] = in ? sk[i - LEAF] : 0;
+        B[x] = in ? bound[i - LEAF] : 1;
     }
-}
-
-__global__ void k_sort_rank(const uint32_t *si, uint64_t n, uint32_t *rank, uint32_t *rinv) {
-    uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
+    __syncthreads();
+    const uint64_t i = t0 + threadIdx.x;
     if (i >= n) return;
-    const uint32_t v = si[i];
-    rank[v] = (uint32_t)i;
-    rinv[i] = v;
+    const uint32_t v = si[i], x = threadIdx.x + LEAF;
+    uint32_t b = x, pos = x;
+    while (!B[b] && x - b < LEAF - 1u) --b;
+    if (B[b] == 1) {
+        const int32_t k = K[x];
+        pos = b;
+        for (uint32_t y = b; y < x; ++y) pos += K[y] <= k ? 1u : 0u;
+        for (uint32_t y = x + 1u; y < b + LEAF && !B[y]; ++y) pos += K[y] < k ? 1u : 0u;
+    }
+    const uint64_t q = t0 + pos - LEAF;
+    rank[v] = (uint32_t)q;
+    rinv[q] = v;
 }
 
 // Elements of all-equal ranges go to their closed-form places (after the
