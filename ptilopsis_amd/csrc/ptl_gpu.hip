@@ -112,6 +112,35 @@ __global__ void k_fill(T *p, uint64_t n, T v) {
     for (; i < n; i += stride) p[i] = v;
 }
 
+// Several fills in one launch (a launch takes longer than most of them): words of
+// 256-byte aligned ranges, four a thread and step.
+struct ClearRange { uint32_t *p; uint64_t n; uint32_t v; };
+struct ClearList { ClearRange r[8]; uint32_t count; };
+__global__ __launch_bounds__(256) void k_clear(ClearList L, uint64_t quads) {
+    const uint64_t stride = (uint64_t)gridDim.x * 256u;
+    for (uint64_t i = blockIdx.x * (uint64_t)256 + threadIdx.x; i < quads; i += stride) {
+        uint64_t q = i;
+        for (uint32_t k = 0; k < L.count; ++k) {
+            const uint64_t nq = (L.r[k].n + 3u) / 4u;
+            if (q >= nq) { q -= nq; continue; }
+            uint32_t *p = L.r[k].p + 4u * q;
+            const uint32_t v = L.r[k].v, m = (uint32_t)min((uint64_t)4, L.r[k].n - 4u * q);
+            if (m == 4u && (reinterpret_cast<uint64_t>(p) & 15u) == 0u) *reinterpret_cast<uint4 *>(p) = make_uint4(v, v, v, v);
+            else for (uint32_t y = 0; y < m; ++y) p[y] = v;
+            break;
+        }
+    }
+}
+
+// Words from different places, or two arrays of n, to consecutive (pinned host) words.
+struct GatherList { const uint32_t *p[8]; uint32_t count; };
+__global__ void k_gather(GatherList g, uint32_t *dst) {
+    if (threadIdx.x < g.count) dst[threadIdx.x] = *g.p[threadIdx.x];
+}
+__global__ void k_gather2(const uint32_t *a, const uint32_t *b, uint32_t n, uint32_t *dst) {
+    for (uint32_t i = threadIdx.x; i < 2u * n; i += blockDim.x) dst[i] = i < n ? a[i] : b[i - n];
+}
+
 __global__ void k_set_u8(uint8_t *p, uint8_t v) { *p = v; }
 
 // A plain streaming copy (16 B per thread and step, grid-stride), for the
@@ -777,9 +806,13 @@ DEV int32_t median_to_first(uint32_t first, uint32_t last, uint32_t *sidx, int32
 }
 
 // The first level: one range per program of more than 16 nodes.
-__global__ void k_sort_root(const Seg *segs, uint32_t m, uint32_t *sidx, int32_t *skey, int32_t *pivot) {
+// (A single one comes by value and is stored here.)
+__global__ void k_sort_root(Seg *segs, uint32_t m, uint32_t *sidx, int32_t *skey, int32_t *pivot, Seg one) {
     const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s < m) pivot[s] = median_to_first(segs[s].first, segs[s].last, sidx, skey);
+    if (s >= m) return;
+    const Seg g = m == 1 ? one : segs[s];
+    if (m == 1) segs[0] = one;
+    pivot[s] = median_to_first(g.first, g.last, sidx, skey);
 }
 
 // Last range whose active offset is <= a.
