@@ -132,13 +132,25 @@ __global__ __launch_bounds__(256) void k_clear(ClearList L, uint64_t quads) {
     }
 }
 
-// Words from different places, or two arrays of n, to consecutive (pinned host) words.
+// Words from different places, then two arrays of n, to consecutive (pinned host) words.
 struct GatherList { const uint32_t *p[8]; uint32_t count; };
-__global__ void k_gather(GatherList g, uint32_t *dst) {
+__global__ void k_gather(GatherList g, const uint32_t *a, const uint32_t *b, uint32_t n, uint32_t *dst) {
     if (threadIdx.x < g.count) dst[threadIdx.x] = *g.p[threadIdx.x];
+    for (uint32_t i = threadIdx.x; i < 2u * n; i += blockDim.x) dst[g.count + i] = i < n ? a[i] : b[i - n];
 }
-__global__ void k_gather2(const uint32_t *a, const uint32_t *b, uint32_t n, uint32_t *dst) {
-    for (uint32_t i = threadIdx.x; i < 2u * n; i += blockDim.x) dst[i] = i < n ? a[i] : b[i - n];
+// The words and the four function arrays of a small result, likewise.
+__global__ __launch_bounds__(256) void k_gather_result(const uint32_t *words, uint32_t nw, const uint32_t *f0,
+                                                       const uint32_t *f1, const uint32_t *f2, const uint32_t *f3,
+                                                       uint32_t nf, uint32_t *dst) {
+    for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < nw + 4u * nf; i += gridDim.x * 256u) {
+        uint32_t k = i, v;
+        if (k < nw) v = words[k];
+        else {
+            k -= nw;
+            v = k < nf ? f0[k] : k < 2u * nf ? f1[k - nf] : k < 3u * nf ? f2[k - 2u * nf] : f3[k - 3u * nf];
+        }
+        dst[i] = v;
+    }
 }
 
 __global__ void k_set_u8(uint8_t *p, uint8_t v) { *p = v; }
@@ -549,11 +561,11 @@ __global__ void k_prog_words(Dev d, const uint32_t *total) {
 
 // Function base of every program: functions (decl nodes, in node order) before
 // its first node.
-__global__ void k_prog_funcs(Dev d) {
+__global__ void k_prog_funcs(Dev d, const uint32_t *F) {
     const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p > d.P) return;
     const uint32_t b = p < d.P ? d.pn[p] : (uint32_t)d.n;
-    uint32_t lo = 0, hi = d.F;  // first decl index >= b
+    uint32_t lo = 0, hi = *F;  // first decl index >= b
     while (lo < hi) { const uint32_t m = (lo + hi) >> 1; if (d.decl[m] < b) lo = m + 1; else hi = m; }
     d.pf[p] = lo;
 }
