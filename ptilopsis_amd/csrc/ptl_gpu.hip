@@ -2194,7 +2194,8 @@ DEV void ra_flush(const Dev &d, const RaL0 &f, const uint16_t *ring, uint32_t rc
 // A wave runs alone on its SIMD, so a branch costs what ten instructions do
 // whether it is taken or not: everything but the rare cases (a state read from
 // HBM, a second mark, a flip) is straight-line, its writes going to a spare row or
-// entry where there is nothing to write.
+// entry where there is nothing to write, and the rare cases are out of line (in
+// line, jumped over: 0.55 us a step of 8 groups against 0.53).
 // hold has an entry per register and one spare.
 template <int MODE, int RC>
 DEV void ra_l0_step(const Dev &d, RaL0 &f, uint16_t *ring, uint32_t *hold, uint32_t rc, uint32_t lane, uint32_t j,
@@ -2208,8 +2209,8 @@ DEV void ra_l0_step(const Dev &d, RaL0 &f, uint16_t *ring, uint32_t *hold, uint3
     uint32_t e1 = ring[w1 * RC + rc], e2 = ring[w2 * RC + rc];
     e1 = d1 ? e1 : 0u; e2 = d2 ? e2 : 0u;
     const uint32_t rl = ring_low(b, f.size);
-    const bool far = __builtin_expect(__ballot((op & (OP_FAR1 | OP_FAR2)) != 0) != 0, 0);
-    if (far) {
+    const bool far = __ballot((op & (OP_FAR1 | OP_FAR2)) != 0) != 0;
+    if (__builtin_expect(far, 0)) {
         if (op & (OP_FAR1 | OP_FAR2)) {
             const uint4 w = d.w0_f4[f.start + i];
             if (op & OP_FAR1) {
@@ -2243,7 +2244,7 @@ DEV void ra_l0_step(const Dev &d, RaL0 &f, uint16_t *ring, uint32_t *hold, uint3
     uint64_t low = wl | (uint64_t)suffix_or<ROWS>(tl, lane, x) | ((uint64_t)suffix_or<ROWS>(th, lane, x) << 32);
     bool n1 = (nb1 & low) != 0, n2 = (nb2 & low) != 0;
     const bool z1 = s1, z2 = s2;  // swapped already
-    if (__ballot((n1 && !z1) || (n2 && !z2))) {
+    if (__builtin_expect(__ballot((n1 && !z1) || (n2 && !z2)) != 0, 0)) {
         bool ch;
         do {
             const bool f1 = n1, f2 = n2;
@@ -2281,7 +2282,7 @@ DEV void ra_l0_step(const Dev &d, RaL0 &f, uint16_t *ring, uint32_t *hold, uint3
     const uint32_t st1 = s1 ? r1 | (h1 << 9) : e1, st2 = s2 ? r2 | (h2 << 9) : e2;
     ring[w1 * RC + rc] = (uint16_t)st1;
     ring[w2 * RC + rc] = (uint16_t)st2;
-    if (far) {
+    if (__builtin_expect(far, 0)) {
         if ((op & OP_FAR1) && s1 && p1 < rl) d.sym[f.start + p1] = (uint16_t)st1;
         if ((op & OP_FAR2) && s2 && p2 < rl) d.sym[f.start + p2] = (uint16_t)st2;
     }
