@@ -73,8 +73,8 @@ def kernel_alg_bytes(name: str, n: int, w0: int, w1: int, w2: int, f: int) -> fl
         "k_opt_init": 16 * w0 + 2 * w0,
         "k_opt_iter": 12 * w0 + 1 * w0,
         "k_opt_final": 4 * w0 + 2 * w0,
-        "k_ra_walk": 16 * w0 * 7 // 8 + 2 * w0 * 7 // 8,
-        "k_ra_lane0": 16 * w0 // 8 + 2 * w0 // 8,
+        "k_ra_walk": 4 * w0 * 7 // 8 + 2 * w0 * 7 // 8,  # a word's op; its state
+        "k_ra_lane0": 4 * w0 // 8 + 2 * w0 // 8,
         "k_scan_ra_count": 13 * w0 + 4 * w0,
         "k_ra_emit": 24 * w0 + 2 * w0 + 20 * w1,
         "k_scan_fj_size": 4 * w1 + 4 * w1,
@@ -176,7 +176,8 @@ def measured_traffic(kernel: str, workload: str) -> float | None:
         return None
     for line in open(path):
         cells = [c.strip() for c in line.strip().strip("|").split("|")]
-        if len(cells) == 5 and cells[0].split("<")[0] == kernel:
+        # (the lockstep's kernels are profiled under one name, k_ra_lane0)
+        if len(cells) == 5 and (cells[0].split("<")[0] == kernel or cells[0].startswith(kernel + "_")):
             try:
                 return float(cells[4].replace(",", ""))
             except ValueError:
