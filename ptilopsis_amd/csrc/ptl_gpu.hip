@@ -2323,6 +2323,134 @@ static_assert(OP_SELF == 1u << ONE_SELF, "");
 // first bit that is 1 (0), ~0 if there is none
 DEV uint32_t ff1(uint64_t x) { uint32_t r; asm("s_ff1_i32_b64 %0, %1" : "=s"(r) : "s"(x)); return r; }
 DEV uint32_t ff0(uint32_t x) { uint32_t r; asm("s_ff0_i32_b32 %0, %1" : "=s"(r) : "s"(x)); return r; }
+// The state of such a function and its steps, B at a time.  old: an LDS ring of OLD
+// words, STRIDE entries apart.  MULTI: the one function left of a program of more
+// groups (k_ra_lane0_wave): the other groups' walked functions still look registers
+// up, those of a lower group in time for the step's own reads (a flip, ra_l0_step),
+// and entries that ended functions hold (oth, defined at word holdv of the function
+// that starts at obase) are still marked.
+struct SoloLooks { uint64_t W, low, high; };  // of every group; of those below and above the function's
+template <uint32_t B, uint32_t OLD, uint32_t STRIDE, bool MULTI>
+struct Solo {
+    const Dev &d;
+    uint32_t start, lane;
+    uint16_t *old;
+    uint32_t ringv, holdv, obase;
+    uint64_t life, own, mk, oth;
+    DEV uint16_t &at(uint32_t p) { return old[(p % OLD) * STRIDE]; }
+    DEV uint8_t *flag(uint32_t p) { return reinterpret_cast<uint8_t *>(&at(p)) + 1; }
+    // the states of the words [lo, hi), hi - lo <= 64, leave the ring
+    DEV void flush(uint32_t lo, uint32_t hi) {
+        const uint32_t w = lo + ((lane - lo) & 63u);
+        if (w < hi) {
+            d.sym[start + w] = (uint16_t)ringv;
+            at(w) = (uint16_t)ringv;
+        }
+    }
+    // the first word the ring holds in the block from b
+    static DEV uint32_t kept_at(uint32_t b) { return b > 64u - B ? b - (64u - B) : 0u; }
+    // before the block from b; first: the first block's
+    DEV void begin(uint32_t b, uint32_t first) {
+        if (b >= 64u && b >= first + B) flush(b - 64u, b - 64u + B);
+        if (((lane - b) & 63u) < B) ringv = 0;
+    }
+    // steps b .. b + n - 1 on the ops `cur` (by lane); looks(k): the walk's lookups of step b + k
+    template <class Looks>
+    DEV void steps(uint32_t b, uint32_t n, uint32_t cur, Looks looks) {
+        // the ring holds the words from kept on; the lanes of this block's are 0
+        // until they are written, which is also the state of no operand
+        const uint32_t kept = kept_at(b);
+        const uint64_t oldown = __ballot(holdv < kept);  // entries whose word may have left the ring
+        // state of a word from its register, as a factor; whether it ends its entry's holding
+        const uint32_t fac = (cur & OP_SELF) ? ((cur & OP_ZERO) ? 0x200u : 0x201u) : 0u;
+        cur |= (cur & (OP_SELF | (63u << OP_CONST))) ? 1u << ONE_WRITES : 0u;
+        for (uint32_t k = 0; k < n; ++k) {
+            const uint32_t i = b + k;
+            const uint32_t op = rdlane(cur, k);
+            const SoloLooks lk = looks(k);
+            uint32_t p1 = i - (op & 0xFFu), p2 = i - ((op >> 8) & 0xFFu);
+            uint32_t e1 = rdlane(ringv, p1 & 63u), e2 = rdlane(ringv, p2 & 63u);
+            // a word's state after a read through register r that finds it marked
+            auto flipped = [&](uint32_t e, uint32_t r) { return (e & ~0x1FFu) | r | ((op & OP_FP) ? 32u : 0u); };
+            auto put = [&](uint32_t p, uint32_t v) {  // of a word that may have left the ring
+                if (p >= kept) { ringv = wrlane(ringv, p & 63u, v); return; }
+                if (i - p < OLD) at(p) = (uint16_t)v;
+                d.sym[start + p] = (uint16_t)v;
+            };
+            if (__builtin_expect((op & (0xE0E0u | OP_FAR1 | OP_FAR2)) != 0, 0)) {
+                if (op & (OP_FAR1 | OP_FAR2)) {
+                    const uint4 w = d.w0_f4[start + i];
+                    wait_loads();
+                    if (op & OP_FAR1) p1 = uniform(w.y) - 64u - start;
+                    if (op & OP_FAR2) p2 = uniform(w.z) - 64u - start;
+                }
+                auto look = [&](uint32_t p, uint32_t e) {
+                    if (p >= kept) return p == i ? 0u : rdlane(ringv, p & 63u);
+                    uint32_t v;
+                    if (i - p < OLD - 64u) v = at(p);
+                    else { v = d.sym[start + p]; wait_loads(); }
+                    return uniform(v);
+                };
+                e1 = look(p1, e1);
+                e2 = look(p2, e2);
+            }
+            if (__builtin_expect(((e1 | e2) & 0x100u) != 0, 0)) {  // marked operands: flipped back
+                // (both read before either is written: they may be the same word)
+                if (e1 & 0x100u) { e1 = flipped(e1, 5u); put(p1, e1); }
+                if (e2 & 0x100u) { e2 = flipped(e2, 6u); put(p2, e2); }
+            }
+            const uint32_t h1 = e1 >> 9, h2 = e2 >> 9;
+            const uint64_t nb1 = rdlane(holdv, h1) == p1 ? 1ull << h1 : 0ull, nb2 = rdlane(holdv, h2) == p2 ? 1ull << h2 : 0ull;
+            const uint64_t nb = own & (nb1 | nb2);
+            if (MULTI && __builtin_expect((nb & lk.low) != 0, 0)) {
+                if (nb1 & own & lk.low) { e1 = flipped(e1, 5u); put(p1, e1); }
+                if (nb2 & own & lk.low) { e2 = flipped(e2, 6u); put(p2, e2); }
+            }
+            // the step's lookups, as op_eval
+            const uint64_t m = ((1ull << (e1 & 63u)) | (1ull << (e2 & 63u))) & ~1ull, cl = life & ~m;
+            const uint32_t fr = ff0((uint32_t)cl), al = fr != ~0u ? fr : 5u;
+            const uint32_t rdr = (op & OP_ALLOC) ? al : (op >> OP_CONST) & 63u;
+            const uint64_t dm = 1ull << rdr;
+            const uint64_t T = (((m & life) | (dm & cl)) & ~1ull) | lk.W;
+            mk &= ~nb;
+            uint64_t nm = MULTI ? own & ~mk & ((T & ~nb) | (lk.high & nb)) : own & ~(mk | nb) & T;
+            mk |= nm;
+            // new marks: mostly none or one, of a word in the ring
+            const uint64_t more = (nm & (nm - 1)) | (nm & oldown);
+            const uint32_t q = rdlane(holdv, ff1(nm) & 63u) & 63u, fl = nm ? 0x100u : 0u;
+            ringv = wrlane(ringv, q, rdlane(ringv, q) | (more ? 0u : fl));
+            if (__builtin_expect(more != 0, 0)) {
+                for (; nm; nm &= nm - 1) {
+                    const uint32_t r = (uint32_t)__builtin_ctzll(nm), p = rdlane(holdv, r);
+                    if (p >= kept) { ringv = wrlane(ringv, p & 63u, rdlane(ringv, p & 63u) | 0x100u); continue; }
+                    if (i - p < OLD) *flag(p) = (uint8_t)(1u | (r << 1));
+                    reinterpret_cast<uint8_t *>(d.sym + start + p)[1] = (uint8_t)(1u | (r << 1));
+                }
+            }
+            const uint64_t lost = m | ((uint64_t)((op >> ONE_WRITES) & 1u) << rdr);
+            if (MULTI) {
+                if (__builtin_expect((oth & T) != 0, 0)) mark_others(T);
+                oth &= ~lost;
+            }
+            ringv = wrlane(ringv, i & 63u, rdr * rdlane(fac, k));
+            holdv = wrlane(holdv, rdr, i);  // (of an entry not won: not owned, never read)
+            own = (own & ~lost) | ((uint64_t)((op >> ONE_SELF) & 1u) << rdr);
+            mk &= ~lost;
+            life = cl | dm;
+        }
+    }
+    DEV void mark_others(uint64_t T) {
+        if (((oth & T) >> lane) & 1u) reinterpret_cast<uint8_t *>(d.sym + obase + holdv)[1] = (uint8_t)(1u | (lane << 1));
+        oth &= ~T;
+    }
+    // the row that gathers the steps past the last, after the last flush
+    DEV void finish(uint64_t W) {
+        const uint64_t nm = own & ~mk & W;
+        if ((nm >> lane) & 1u) reinterpret_cast<uint8_t *>(d.sym + start + holdv)[1] = (uint8_t)(1u | (lane << 1));
+        if (MULTI) mark_others(W);
+    }
+};
+
 __global__ __launch_bounds__(64) void k_ra_lane0_one(Dev d, const Ra0Prog *progs, const unsigned long long *mask_all,
                                                      uint64_t mstride, uint32_t mcopies, const uint32_t *done,
                                                      const uint32_t *need) {
@@ -2337,9 +2465,6 @@ __global__ __launch_bounds__(64) void k_ra_lane0_one(Dev d, const Ra0Prog *progs
     const unsigned long long *tab = mask_all + pg.gbase;
     const uint64_t m1 = mcopies > 1 ? mstride : 0u;
     bool wok = true;
-    uint8_t *symb = reinterpret_cast<uint8_t *>(d.sym + start);
-    uint32_t ringv = 0, holdv = 0;
-    uint64_t life = 0x1Full, own = 0, mk = 0;
     // ops and lookups of the steps i + lane, lane < ONE_BLOCK (rows past the last: none)
     struct Block { uint32_t op; unsigned long long a, b; };
     uint32_t ready = 0;  // chunks known to be published
@@ -2354,107 +2479,22 @@ __global__ __launch_bounds__(64) void k_ra_lane0_one(Dev d, const Ra0Prog *progs
         }
         return r;
     };
-    // the states of the words [lo, hi), hi - lo <= 64, leave the ring
-    auto flush = [&](uint32_t lo, uint32_t hi) {
-        const uint32_t w = lo + ((lane - lo) & 63u);
-        if (w < hi) {
-            d.sym[start + w] = (uint16_t)ringv;
-            old[w % ONE_OLD] = (uint16_t)ringv;
-        }
-    };
+    Solo<ONE_BLOCK, ONE_OLD, 1, false> f{d, start, lane, old, 0u, 0u, 0u, 0x1Full, 0ull, 0ull, 0ull};
     Block nx = load(0);
     for (uint32_t b = 0; b < size; b += ONE_BLOCK) {
         uint32_t cur = nx.op, wlo = (uint32_t)(nx.a | nx.b), whi = (uint32_t)((nx.a | nx.b) >> 32);
         asm volatile("" : "+v"(cur), "+v"(wlo), "+v"(whi) : : "memory");  // waited for before the next loads are issued
         nx = load(b + ONE_BLOCK);
-        // the ring holds the words from kept on; the lanes of this block's are 0
-        // until they are written, which is also the state of no operand
-        const uint32_t kept = b >= ONE_BLOCK ? b - ONE_BLOCK : 0u;
-        if (b >= 2u * ONE_BLOCK) flush(b - 2u * ONE_BLOCK, kept);
-        if (((lane - b) & 63u) < ONE_BLOCK) ringv = 0;
-        const uint64_t oldown = __ballot(holdv < kept);  // entries whose word may have left the ring
-        // state of a word from its register, as a factor; whether it ends its entry's holding
-        const uint32_t fac = (cur & OP_SELF) ? ((cur & OP_ZERO) ? 0x200u : 0x201u) : 0u;
-        cur |= (cur & (OP_SELF | (63u << OP_CONST))) ? 1u << ONE_WRITES : 0u;
-        const uint32_t n = uniform(min(ONE_BLOCK, size - b));
-        for (uint32_t k = 0; k < n; ++k) {
-            const uint32_t i = b + k;
-            const uint32_t op = rdlane(cur, k);
-            const uint64_t W = (uint64_t)rdlane(wlo, k) | ((uint64_t)rdlane(whi, k) << 32);
-            uint32_t p1 = i - (op & 0xFFu), p2 = i - ((op >> 8) & 0xFFu);
-            uint32_t e1 = rdlane(ringv, p1 & 63u), e2 = rdlane(ringv, p2 & 63u);
-            if (__builtin_expect((op & (0xE0E0u | OP_FAR1 | OP_FAR2)) != 0, 0)) {
-                if (op & (OP_FAR1 | OP_FAR2)) {
-                    const uint4 w = d.w0_f4[start + i];
-                    wait_loads();
-                    if (op & OP_FAR1) p1 = uniform(w.y) - 64u - start;
-                    if (op & OP_FAR2) p2 = uniform(w.z) - 64u - start;
-                }
-                // states of words that may have left the ring, then those a mark is
-                // flipped back in (rs1's and rs2's word may be the same)
-                auto look = [&](uint32_t p, uint32_t e) {
-                    if (p >= kept) return e;
-                    uint32_t v;
-                    if (i - p < ONE_OLD - 64u) v = old[p % ONE_OLD];
-                    else { v = d.sym[start + p]; wait_loads(); }
-                    return uniform(v);
-                };
-                auto flip = [&](uint32_t p, uint32_t e, uint32_t r) {
-                    if (p >= kept || !(e & 0x100u)) return e;
-                    const uint32_t v = (e & ~0x1FFu) | r | ((op & OP_FP) ? 32u : 0u);
-                    if (i - p < ONE_OLD) old[p % ONE_OLD] = (uint16_t)v;
-                    d.sym[start + p] = (uint16_t)v;
-                    return v;
-                };
-                e1 = look(p1, e1);
-                e2 = look(p2, e2);
-                e1 = flip(p1, e1, 5u);
-                e2 = flip(p2, e2, 6u);
-            }
-            if (__builtin_expect(((e1 | e2) & 0x100u) != 0, 0)) {  // marked operands: flipped back
-                const uint32_t fp = (op & OP_FP) ? 32u : 0u;
-                if (e1 & 0x100u) { e1 = (e1 & ~0x1FFu) | fp | 5u; ringv = wrlane(ringv, p1 & 63u, e1); }
-                if (e2 & 0x100u) { e2 = (e2 & ~0x1FFu) | fp | 6u; ringv = wrlane(ringv, p2 & 63u, e2); }
-            }
-            const uint32_t h1 = e1 >> 9, h2 = e2 >> 9;
-            const uint64_t nb = own & ((rdlane(holdv, h1) == p1 ? 1ull << h1 : 0ull) | (rdlane(holdv, h2) == p2 ? 1ull << h2 : 0ull));
-            // the step's lookups, as op_eval
-            const uint64_t m = ((1ull << (e1 & 63u)) | (1ull << (e2 & 63u))) & ~1ull, cl = life & ~m;
-            const uint32_t fr = ff0((uint32_t)cl), al = fr != ~0u ? fr : 5u;
-            const uint32_t rdr = (op & OP_ALLOC) ? al : (op >> OP_CONST) & 63u;
-            const uint64_t dm = 1ull << rdr;
-            mk &= ~nb;
-            uint64_t nm = own & ~(mk | nb) & ((((m & life) | (dm & cl)) & ~1ull) | W);
-            mk |= nm;
-            // new marks: mostly none or one, of a word in the ring
-            const uint64_t more = (nm & (nm - 1)) | (nm & oldown);
-            const uint32_t q = rdlane(holdv, ff1(nm) & 63u) & 63u, fl = nm ? 0x100u : 0u;
-            ringv = wrlane(ringv, q, rdlane(ringv, q) | (more ? 0u : fl));
-            if (__builtin_expect(more != 0, 0)) {
-                for (; nm; nm &= nm - 1) {
-                    const uint32_t r = (uint32_t)__builtin_ctzll(nm), p = rdlane(holdv, r);
-                    if (p >= kept) { ringv = wrlane(ringv, p & 63u, rdlane(ringv, p & 63u) | 0x100u); continue; }
-                    if (i - p < ONE_OLD) reinterpret_cast<uint8_t *>(old)[2u * (p % ONE_OLD) + 1u] = (uint8_t)(1u | (r << 1));
-                    symb[2u * (uint64_t)p + 1u] = (uint8_t)(1u | (r << 1));
-                }
-            }
-            ringv = wrlane(ringv, i & 63u, rdr * rdlane(fac, k));
-            holdv = wrlane(holdv, rdr, i);  // (of an entry not won: not owned, never read)
-            const uint64_t lost = m | ((uint64_t)((op >> ONE_WRITES) & 1u) << rdr);
-            own = (own & ~lost) | ((uint64_t)((op >> ONE_SELF) & 1u) << rdr);
-            mk &= ~lost;
-            life = cl | dm;
-        }
+        f.begin(b, 0u);
+        f.steps(b, uniform(min(ONE_BLOCK, size - b)), cur, [&](uint32_t k) {
+            return SoloLooks{(uint64_t)rdlane(wlo, k) | ((uint64_t)rdlane(whi, k) << 32), 0ull, 0ull};
+        });
     }
-    if (size) {
-        const uint32_t last = (size - 1u) / ONE_BLOCK * ONE_BLOCK;  // the last block's first word
-        flush(last >= ONE_BLOCK ? last - ONE_BLOCK : 0u, size);
-    }
-    if (rows > size) {  // the row that gathers the steps past the last
+    if (size) f.flush(f.kept_at((size - 1u) / ONE_BLOCK * ONE_BLOCK), size);
+    if (rows > size) {
         if (pdone) ra0_wait(d, pdone, pneed, (rows - 1u) / WALK_PUB, wok);
         const unsigned long long W = tab[rows - 1u] | tab[m1 + rows - 1u];
-        const uint64_t nm = own & ~mk & ((uint64_t)uniform((uint32_t)W) | ((uint64_t)uniform((uint32_t)(W >> 32)) << 32));
-        if ((nm >> lane) & 1u) symb[2u * (uint64_t)holdv + 1u] = (uint8_t)(1u | (lane << 1));
+        f.finish((uint64_t)uniform((uint32_t)W) | ((uint64_t)uniform((uint32_t)(W >> 32)) << 32));
     }
 }
 
@@ -2467,6 +2507,10 @@ __global__ __launch_bounds__(64) void k_ra_lane0_one(Dev d, const Ra0Prog *progs
 // Bound by the chain of a step's instructions (latency): 5.4 -> 0.53 us a step
 // for 8 groups, against a workgroup exchanging lookups through LDS atomics and
 // barriers with its states in HBM; 0.8 us with the loads in the stepping wave.
+// From the block on in which one function is left, its steps are a one-group
+// program's (Solo; a step as above has three LDS reads in a chain, and leaving out
+// its scans alone gained nothing): 62 functions, a quarter of 3740 steps, 2.10 ->
+// 1.94 ms; 60 programs 6.5 -> 6.25 ms summed.
 constexpr uint32_t RA0_FETCH = 16;
 template <int ROWS>
 __global__ __launch_bounds__(128) void k_ra_lane0_wave(Dev d, const Ra0Prog *progs, const unsigned long long *mask_all,
@@ -2486,6 +2530,13 @@ __global__ __launch_bounds__(128) void k_ra_lane0_wave(Dev d, const Ra0Prog *pro
     const uint32_t j = act ? pg.L - 1u - lane : 0u;  // the lane's group
     RaL0 f{act ? d.fstarts[pg.fbase + 8u * j] : 0u, act ? d.fsizes[pg.fbase + 8u * j] : 0u, 0x1Full, 0, 0};
     const uint32_t rows = pg.rows;
+    // the longest function's lane, and the first block of steps it is alone in
+    uint32_t top = f.size;
+    for (uint32_t o = 32; o > 0; o >>= 1) top = max(top, (uint32_t)__shfl_xor((int)top, (int)o, 64));
+    const uint32_t al = uniform((uint32_t)__builtin_ctzll(__ballot(f.size == top)));
+    uint32_t second = lane == al ? 0u : f.size;
+    for (uint32_t o = 32; o > 0; o >>= 1) second = max(second, (uint32_t)__shfl_xor((int)second, (int)o, 64));
+    const uint32_t alone = uniform((second + RA0_FETCH - 1u) / RA0_FETCH * RA0_FETCH);
     if (fetch) {
         const uint32_t *pdone = done && pg.cbase != RA0_NOPUB ? done + pg.cbase : nullptr;
         const uint32_t *pneed = pdone ? need + pg.cbase : nullptr;
@@ -2511,7 +2562,21 @@ __global__ __launch_bounds__(128) void k_ra_lane0_wave(Dev d, const Ra0Prog *pro
 #pragma unroll
                     for (uint32_t k = 0; k < RA0_FETCH; ++k) {
                         fop[b][k][col] = (int32_t)(i + k) < (int32_t)f.size ? o[k / 4].o[k % 4] : 0u;
-                        fw[b][k][col] = act && i + k < rows ? w0[k] | w1[k] : 0ull;
+                        if (i < alone) fw[b][k][col] = act && i + k < rows ? w0[k] | w1[k] : 0ull;
+                    }
+                }
+                if (i >= alone) {  // the masks of RaLooks for one function
+#pragma unroll
+                    for (uint32_t k = 0; k < RA0_FETCH; ++k) {
+                        const uint64_t w = act && i + k < rows ? w0[k] | w1[k] : 0ull;
+                        const uint64_t wo = lane > al ? w : 0ull, wh = lane < al ? w : 0ull;
+                        constexpr uint32_t LAST = NL - 1;
+                        const uint32_t a = scan_or<ROWS>((uint32_t)wo), c = scan_or<ROWS>((uint32_t)(wo >> 32));
+                        const uint32_t g = scan_or<ROWS>((uint32_t)wh), h = scan_or<ROWS>((uint32_t)(wh >> 32));
+                        const uint64_t low = (uint64_t)rdlane(a, LAST) | ((uint64_t)rdlane(c, LAST) << 32);
+                        const uint64_t high = (uint64_t)rdlane(g, LAST) | ((uint64_t)rdlane(h, LAST) << 32);
+                        const uint64_t own = (uint64_t)rdlane((uint32_t)w, al) | ((uint64_t)rdlane((uint32_t)(w >> 32), al) << 32);
+                        if (lane < 3u) fw[b][k][lane] = lane == 0 ? low : lane == 1 ? high : low | high | own;
                     }
                 }
             }
@@ -2521,7 +2586,8 @@ __global__ __launch_bounds__(128) void k_ra_lane0_wave(Dev d, const Ra0Prog *pro
         return;
     }
     lds_barrier();  // the first steps are in
-    for (uint32_t i0 = 0; i0 < rows; i0 += RA0_FETCH) {
+    uint32_t i0 = 0;
+    for (; i0 < min(alone, rows); i0 += RA0_FETCH) {
         const uint32_t b = (i0 / RA0_FETCH) & 1u;
         uint32_t op = fop[b][0][col];
         unsigned long long W = fw[b][0][col];
@@ -2541,7 +2607,43 @@ __global__ __launch_bounds__(128) void k_ra_lane0_wave(Dev d, const Ra0Prog *pro
         }
         lds_barrier();  // the next steps are in
     }
-    if (lane < (uint32_t)NL) ra_flush<NL>(d, f, ring, col);
+    if (i0 >= rows) {
+        if (lane < (uint32_t)NL) ra_flush<NL>(d, f, ring, col);
+        return;
+    }
+    // One function left, the one of lane al: stepped as a one-group program's.  The
+    // states of the others go to HBM, and those of its last words: the LDS ring
+    // keeps these, the last of them go to the register ring.
+    const uint32_t start = rdlane(f.start, al), size = rdlane(f.size, al);
+    if (lane < (uint32_t)NL && (lane != al || size <= i0)) ra_flush<NL>(d, f, ring, col);
+    if (size > i0)
+        for (uint32_t p = (i0 > OP_ROWS ? i0 - OP_ROWS : 0u) + lane; p < i0; p += 64u)
+            d.sym[start + p] = ring[(p & (OP_ROWS - 1u)) * NL + al];
+    auto of = [&](uint64_t v, uint32_t l) { return (uint64_t)rdlane((uint32_t)v, l) | ((uint64_t)rdlane((uint32_t)(v >> 32), l) << 32); };
+    Solo<RA0_FETCH, OP_ROWS, NL, true> g{d, start, lane, ring + al, 0u, hold[lane], 0u, of(f.life, al), of(f.own, al), of(f.mk, al), 0ull};
+    for (uint32_t l = 0; l < pg.L; ++l) {
+        const uint64_t o = l == al ? 0ull : of(f.own & ~f.mk, l);
+        g.oth |= o;
+        if ((o >> lane) & 1u) g.obase = rdlane(f.start, l);
+    }
+    {
+        const uint32_t lo = i0 > 64u - RA0_FETCH ? i0 - (64u - RA0_FETCH) : 0u, w = lo + ((lane - lo) & 63u);
+        if (w < i0) g.ringv = ring[(w & (OP_ROWS - 1u)) * NL + al];
+    }
+    wait_loads();  // (the others' states are written before a mark of one of them)
+    const uint32_t first = i0;
+    for (; i0 < rows; i0 += RA0_FETCH) {
+        const uint32_t b = (i0 / RA0_FETCH) & 1u, kl = lane % RA0_FETCH;
+        const uint32_t cur = fop[b][kl][al];
+        const uint64_t lo = fw[b][kl][0], hi = fw[b][kl][1], W = fw[b][kl][2];
+        if (i0 < size) {
+            g.begin(i0, first);
+            g.steps(i0, uniform(min(RA0_FETCH, size - i0)), cur, [&](uint32_t k) { return SoloLooks{of(W, k), of(lo, k), of(hi, k)}; });
+            if (size - i0 <= RA0_FETCH) g.flush(g.kept_at(i0), size);  // the last block
+        }
+        if (rows > size && size / RA0_FETCH == i0 / RA0_FETCH) g.finish(of(W, size % RA0_FETCH));
+        lds_barrier();
+    }
 }
 
 // ============================================================ small programs

@@ -85,3 +85,20 @@ def test_gpu_alloc_far_operands(gpu_ctx, nf):
     assert far > 0
     say("allocation, far operands", far, "in", t.n, "nodes")
     assert_same(gpu_ctx.compile(t), oracle.compile_tree(t), nf)
+
+
+@pytest.mark.parametrize("where", ["first", "middle", "last"])
+@pytest.mark.parametrize("nf", [9, 24, 130, 512])
+def test_gpu_alloc_one_function_left(gpu_ctx, nf, where):
+    # one lane-0 function far longer than the others, in the first, a middle or
+    # the last group: the lockstep in one wave ends on it alone, from steps on
+    # both sides of a block
+    groups = (nf + 7) // 8
+    g = {"first": 0, "middle": groups // 2, "last": groups - 1}[where]
+    for k in range(3):
+        rng = np.random.default_rng(97 * nf + k)
+        targets = rng.integers(20, 300, nf).astype(np.uint32)
+        targets[8 * g] = 2500
+        t = parse_source(W.program_source(0xA1100 + 8 * nf + k, nf, targets)[0])
+        say("allocation, one long function,", nf, where, k)
+        assert_same(gpu_ctx.compile(t), oracle.compile_tree(t), (nf, where, k))
