@@ -24,8 +24,8 @@
 //                independent), k_ra_lane0_wave / k_ra_lane0 (lane-0 functions in
 //                step lockstep: they share the first 64-entry region of the
 //                reference's register_state snapshot, :1290-1354), k_ra_serial (exact
-//                in-order walk for programs where a function names another's
-//                register), then counts, scan, emit (:1422-1697), function table
+//                in-order walk for programs where a function names a register that
+//                another defines), then counts, scan, emit (:1422-1697), function table
 //                fix and frame words (:1714-1811).
 //   fix_jumps    size + scan + fused move/encode/postprocess (:1853-1993, 1995-2011).
 //
@@ -1564,16 +1564,29 @@ constexpr uint32_t OP_CONST = 16;     // shift of the constant register
 constexpr uint32_t OP_ALLOC = 1u << 22, OP_SELF = 1u << 23, OP_FP = 1u << 24, OP_FAR1 = 1u << 25, OP_FAR2 = 1u << 26,
                    OP_ZERO = 1u << 27;
 
-// The op of word i of the function [s, s + size).  `odd` turns true for a word
-// of another form: an operand or destination naming a word of another function
-// (isn_gen ORs a word's own virtual register into physical argument registers,
-// rv_generator_avx.cpp:676-697, :842, which for calls with many arguments can
-// name one), a later word, or a destination other than the word's own
-// register.  The walks keep a register's state with the one thread that walks
-// its function, in the order of that function's words; a program with an odd
-// word is allocated by k_ra_serial in the reference's step and group order.
-DEV uint32_t ra_op(const Dev &d, uint32_t i, uint32_t s, uint32_t rd, uint32_t rs1, uint32_t rs2, uint32_t ins,
-                   bool &odd) {
+// Whether an operand of function f's word i that names word v, of another function
+// or after i, reads the cleared state whatever the order of the walks: v is a word
+// of f's program that does not define its register (a word that defines another
+// one's is odd itself), or a later word of f itself (v > i), not yet defined.
+DEV bool ra_never_set(const Dev &d, uint32_t f, uint32_t s, uint32_t i, uint32_t v) {
+    const uint32_t p = prog_of(d.pf, d.P, f);
+    if (v < d.pw[p] || v >= d.pw[p + 1]) return false;
+    return d.w0_rd[v] != v + 64u || (v > i && v - s < d.fsizes[f]);
+}
+
+// The op of word i of function f, the words [s, s + size).  `odd` turns true for a
+// word of another form: an operand naming a word of another function that defines
+// its register (isn_gen ORs a word's own virtual register into physical argument
+// registers, rv_generator_avx.cpp:676-697, :842, which for calls with many
+// arguments can name one), or a destination other than the word's own register.
+// The walks keep a register's state with the one thread that walks its function,
+// in the order of that function's words; a program with an odd word is allocated by
+// k_ra_serial in the reference's step and group order.  A register that nothing has
+// defined yet reads as x0 in any order and its state stays cleared: no operand (a
+// program of 20 functions and 7.2k words with one such read: walk and lockstep 0.45
+// ms, k_ra_serial 2.54).
+DEV uint32_t ra_op(const Dev &d, uint32_t f, uint32_t i, uint32_t s, uint32_t rd, uint32_t rs1, uint32_t rs2,
+                   uint32_t ins, bool &odd) {
     const bool fp = (ins & 0x7Fu) == 0x53u;
     uint32_t op = fp ? OP_FP : 0u;
     const uint32_t rs[2] = {rs1, rs2};
@@ -1582,7 +1595,7 @@ DEV uint32_t ra_op(const Dev &d, uint32_t i, uint32_t s, uint32_t rd, uint32_t r
         if ((int32_t)rs[k] <= 63) continue;
         const uint32_t v = rs[k] - 64u;
         if (v >= d.W0) { atomicOr(d.flags, EF_OOB); odd = true; continue; }
-        if (v < s || v > i) { odd = true; continue; }
+        if (v < s || v > i) { odd = odd || !ra_never_set(d, f, s, i, v); continue; }
         const uint32_t dist = i - v;
         if (dist == 0) op |= OP_ZERO;
         else if (dist <= OP_WINDOW) op |= dist << (8 * k);
@@ -1617,7 +1630,7 @@ __global__ __launch_bounds__(256) void k_opt_final(Dev d) {
     const uint32_t s = d.fstarts[f];
     // (a word outside every function is walked by none)
     const bool in = (uint32_t)i - s < d.fsizes[f];
-    const uint32_t op = in ? ra_op(d, (uint32_t)i, s, rd, rs1, rs2, ins, odd) : 0u;
+    const uint32_t op = in ? ra_op(d, f, (uint32_t)i, s, rd, rs1, rs2, ins, odd) : 0u;
     d.ops[i] = op;
     if (odd) { atomicOr(d.flags, EF_XCONFLICT); d.cflag[prog_of(d.pf, d.P, f)] = 1; }
 }
@@ -4053,8 +4066,8 @@ __global__ __launch_bounds__(1024) void k_ra_lane0_wg(Dev d, const Ra0Prog *prog
     ra_flush<64>(d, f, ring, lane);
 }
 
-// Exact fallback for programs in which two functions name the same virtual
-// register (ra_op): the reference's allocation walk as written
+// Exact fallback for programs in which a function names a register that another
+// one defines (ra_op): the reference's allocation walk as written
 // (rv_generator_avx.cpp:1041-1418 at one thread), one wave: steps in order,
 // groups of 8 functions in order within a step, the 8 functions of a group on
 // lanes 0-7.  Each group body reads its operands' states before any of its
