@@ -210,7 +210,8 @@ int ptl_result_listing(ptl_ctx *ctx, uint32_t program, const char **text, uint64
  * "func_ids", "func_starts", "func_ends", "func_sizes", "instr", "rd", "rs1",
  * "rs2", "jt", "used", "sym_reg", "sym_sw", "sorted", and per program
  * "ra_rows" (steps of the allocation lockstep) and "ra_maxsize" (its longest
- * function, in words).  Copies up to cap elements (u32) into dst and returns
+ * function, in words); or "pinned", the context's pinned staging buffers for the
+ * function sizes and the allocation plan, in KiB.  Copies up to cap elements (u32) into dst and returns
  * the element count, or a negative status. */
 int64_t ptl_debug_dump(ptl_ctx *ctx, const char *name, uint32_t *dst, uint64_t cap);
 
