@@ -181,6 +181,10 @@ int ptl_server_wait(ptl_server *s, uint64_t ticket, ptl_result *out, ptl_serve_t
 int ptl_server_release(ptl_server *s, uint64_t ticket);
 int ptl_server_stats(ptl_server *s, uint64_t *batches, uint64_t *requests_done, uint64_t *nodes_done,
                      uint64_t *largest_batch);
+/* Allocations that the workers' batches did twice because a lockstep gave up
+ * waiting for its walk (see ptl_debug_overlap): 0 unless something else keeps the
+ * device's compute units from the walks. */
+int ptl_server_redos(ptl_server *s, uint64_t *redos);
 
 /* Text output: replaces rv_generator::to_asm (src/codegen/rv_generator.cpp:114-120),
  * which prints every word as rvdisasm::instruction(word) (src/disassembler.cpp:453-462)
@@ -210,7 +214,8 @@ int ptl_result_listing(ptl_ctx *ctx, uint32_t program, const char **text, uint64
  * "func_ids", "func_starts", "func_ends", "func_sizes", "instr", "rd", "rs1",
  * "rs2", "jt", "used", "sym_reg", "sym_sw", "sorted", and per program
  * "ra_rows" (steps of the allocation lockstep) and "ra_maxsize" (its longest
- * function, in words); or "pinned", the context's pinned staging buffers for the
+ * function, in words); or "ra_redos", the context's allocations redone (one after
+ * the other, see ptl_debug_overlap) so far, or "pinned", the context's pinned staging buffers for the
  * function sizes and the allocation plan, in KiB.  Copies up to cap elements (u32) into dst and returns
  * the element count, or a negative status. */
 int64_t ptl_debug_dump(ptl_ctx *ctx, const char *name, uint32_t *dst, uint64_t cap);
@@ -241,6 +246,13 @@ int ptl_tune_get(ptl_ctx *ctx, const char *knob, uint32_t bucket, uint32_t *valu
  * other, as it does when the device serializes the kernels.  PTL_ERR_ARG for
  * other values. */
 int ptl_debug_overlap(ptl_ctx *ctx, int on);
+/* Host only: plans the allocation of one batch (words of every function, first
+ * function of every program, n_programs + 1) for n_contexts contexts that compile
+ * it at the same time on a device of n_cus compute units; room[k] is the compute
+ * units' worth of lockstep workgroups that context k lets wait for its walk.
+ * Together they leave the walks at least one. */
+int ptl_debug_ra_room(const uint32_t *func_sizes, const uint32_t *prog_funcs, uint32_t n_programs, uint32_t n_contexts,
+                      uint32_t n_cus, double *room);
 
 /* Per-kernel timing: with profiling on, every kernel launch of the following
  * calls is bracketed by HIP events on the context's stream.  ptl_profile_get

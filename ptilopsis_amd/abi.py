@@ -20,7 +20,8 @@ EXPORTS = ("ptl_create", "ptl_destroy", "ptl_strerror", "ptl_compile", "ptl_uplo
            "ptl_debug_dump", "ptl_debug_stop_after", "ptl_debug_overlap",
            "ptl_debug_exclusive_scan", "ptl_debug_depth_sort", "ptl_profile_enable", "ptl_profile_get",
            "ptl_compile_noalloc", "ptl_tree_build", "ptl_upload_arena", "ptl_compile_arena",
-           "ptl_server_submit_arena", "ptl_result_listing", "ptl_debug_copy_bandwidth")
+           "ptl_server_submit_arena", "ptl_result_listing", "ptl_debug_copy_bandwidth", "ptl_server_redos",
+           "ptl_debug_ra_room")
 
 
 class PtlAst(C.Structure):
@@ -89,6 +90,10 @@ def bind(lib):
     lib.ptl_server_release.restype = C.c_int
     lib.ptl_server_stats.argtypes = [C.c_void_p] + [C.POINTER(C.c_uint64)] * 4
     lib.ptl_server_stats.restype = C.c_int
+    lib.ptl_server_redos.argtypes = [C.c_void_p, C.POINTER(C.c_uint64)]
+    lib.ptl_server_redos.restype = C.c_int
+    lib.ptl_debug_ra_room.argtypes = [C.c_void_p, C.c_void_p, C.c_uint32, C.c_uint32, C.c_uint32, C.c_void_p]
+    lib.ptl_debug_ra_room.restype = C.c_int
     lib.ptl_debug_dump.argtypes = [C.c_void_p, C.c_char_p, C.c_void_p, C.c_uint64]
     lib.ptl_debug_dump.restype = C.c_int64
     lib.ptl_debug_stop_after.argtypes = [C.c_void_p, C.c_int]

@@ -310,6 +310,12 @@ class Server:
         self.lib.ptl_server_stats(self.h, *[C.byref(x) for x in v])
         return dict(zip(("batches", "requests_done", "nodes_done", "largest_batch"), (int(x.value) for x in v)))
 
+    def redos(self) -> int:
+        """Allocations the batches did twice after a lockstep gave up waiting."""
+        v = C.c_uint64()
+        self.lib.ptl_server_redos(self.h, C.byref(v))
+        return int(v.value)
+
     def close(self):
         if getattr(self, "h", None):
             self.lib.ptl_server_destroy(self.h)
