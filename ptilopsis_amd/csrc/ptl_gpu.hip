@@ -153,8 +153,6 @@ __global__ __launch_bounds__(256) void k_gather_result(const uint32_t *words, ui
     }
 }
 
-__global__ void k_set_u8(uint8_t *p, uint8_t v) { *p = v; }
-
 // A plain streaming copy (16 B per thread and step, grid-stride), for the
 // measured HBM bandwidth the stages are reported against.
 __global__ __launch_bounds__(256) void k_copy16(const uint4 *a, uint4 *b, uint64_t n) {
@@ -1318,8 +1316,6 @@ __global__ __launch_bounds__(NT) void k_sort_local(const Seg *loc, const int32_t
         if (tid < nu) uni[(uint32_t)(ubase >> 32) + tid] = Seg{base + uf[tid], base + ul[tid], ulim[tid], (uint32_t)ubase + o};
     }
 }
-
-DEV bool KLESS(const int32_t *skey, uint32_t a, uint32_t b) { return skey[a] < skey[b]; }
 
 // libstdc++ heap routines on one range, one thread (std::__make_heap,
 // std::__adjust_heap, std::__push_heap, std::__sort_heap).
@@ -3046,7 +3042,7 @@ struct Ra0Fn {
     uint32_t j, start, size;              // group, first word, word count
     uint64_t life;
     uint64_t own;                         // snapshot registers this function may own
-    uint32_t ord, rs1, rs2;               // step i (kept, or reloaded from LDS in every phase)
+    uint32_t ord, rs1, rs2;               // step i (reloaded from LDS in every phase)
     uint4 nw;                             // step i+1: rd, rs1, rs2, instruction (zeros past the end)
     uint32_t rr;                          // step i's result: r1r | r2r << 8 | rdr << 16
     uint32_t pk;                          // step i: raw1 | raw2 << 8 | s1 << 16 | s2 << 17 | flips << 18 |
@@ -3108,11 +3104,9 @@ DEV uint32_t ra0_owned_flips(uint64_t own, const int32_t *Sv, const int32_t *So,
 
 constexpr uint32_t RA0_LDS_FNS = 8192;  // lane-0 functions whose current fields fit in LDS
 
-// A function's fields of step i, from LDS where its thread does not keep them
-// in registers across the step (KEEP: at most three functions per thread).
-template <bool KEEP>
+// A function's fields of step i, from LDS.
 DEV void ra0_cur(Ra0Fn &f, const uint32_t *crd, const uint32_t *crs1, const uint32_t *crs2, uint32_t j) {
-    if (!KEEP) { f.ord = crd[j]; f.rs1 = crs1[j]; f.rs2 = crs2[j]; }
+    f.ord = crd[j]; f.rs1 = crs1[j]; f.rs2 = crs2[j];
 }
 
 DEV void ra0_lookups(uint32_t *mn, uint32_t *mx, const RaStep &r, uint32_t j) {
@@ -3183,7 +3177,6 @@ __global__ __launch_bounds__(1024) void k_ra_lane0(Dev d, const Ra0Prog *progs, 
     __shared__ int changed;
     const uint32_t tid = threadIdx.x, nth = blockDim.x;
     const uint32_t wid = tid >> 6, nwv = nth >> 6, lane = tid & 63u;
-    constexpr bool KEEP = PER <= 3;  // a function's fields of step i stay in registers
     // with one table copy per loading wave, a loading wave holds its copy's
     // row of step i+2 in registers, loaded a step before it is staged
     const uint32_t k0 = nwv - 1u - wid;
@@ -3254,7 +3247,7 @@ __global__ __launch_bounds__(1024) void k_ra_lane0(Dev d, const Ra0Prog *progs, 
             Ra0Fn &f = fn[q];
             const uint32_t j = f.j;
             if ((int32_t)i < (int32_t)f.size) {
-                ra0_cur<KEEP>(f, cur_rd, cur_rs1, cur_rs2, j);
+                ra0_cur(f, cur_rd, cur_rs1, cur_rs2, j);
                 const RaStep r = ra0_step(f);
                 if (f.own) {
                     ra0_lookups(Omin[c], Omax[c], r, j);
@@ -3303,7 +3296,7 @@ __global__ __launch_bounds__(1024) void k_ra_lane0(Dev d, const Ra0Prog *progs, 
                     if (fn[q].own && (int32_t)i < (int32_t)fn[q].size) {
                         fn[q].pk = (fn[q].pk & ~(3u << 18)) |
                                    (ra0_owned_flips(fn[q].own & fm, Sv[c], So[c], flip, j) << 18);
-                        ra0_cur<KEEP>(fn[q], cur_rd, cur_rs1, cur_rs2, j);
+                        ra0_cur(fn[q], cur_rd, cur_rs1, cur_rs2, j);
                         const RaStep r = ra0_step(fn[q]);
                         ra0_lookups(Omin[c], Omax[c], r, j);
                         fn[q].rr = r.r1r | (r.r2r << 8) | (r.rdr << 16);
@@ -3340,7 +3333,7 @@ __global__ __launch_bounds__(1024) void k_ra_lane0(Dev d, const Ra0Prog *progs, 
             if (fn[q].own && (int32_t)i < (int32_t)fn[q].size) {
                 const uint32_t rr = fn[q].rr;
                 RaStep r;
-                r.ord = KEEP ? fn[q].ord : cur_rd[j];
+                r.ord = cur_rd[j];
                 r.r1r = rr & 0xFFu; r.r2r = (rr >> 8) & 0xFFu; r.rdr = (rr >> 16) & 0xFFu;
                 const uint64_t clr = ((1ull << r.r1r) | (1ull << r.r2r)) & ~1ull;
                 fn[q].life = (fn[q].life & ~clr) | (1ull << r.rdr);
@@ -3392,7 +3385,7 @@ __global__ __launch_bounds__(1024) void k_ra_lane0(Dev d, const Ra0Prog *progs, 
             if (t >= L) continue;
             uint64_t won = 0;
             if ((int32_t)i < (int32_t)f.size) {
-                ra0_cur<KEEP>(f, cur_rd, cur_rs1, cur_rs2, j);
+                ra0_cur(f, cur_rd, cur_rs1, cur_rs2, j);
                 const uint32_t rr = f.rr;
                 RaStep r;
                 r.ord = f.ord; r.rs1 = f.rs1; r.rs2 = f.rs2;
@@ -3411,7 +3404,6 @@ __global__ __launch_bounds__(1024) void k_ra_lane0(Dev d, const Ra0Prog *progs, 
                 ra0_commit(d, r, (f.pk & 0xFFu) | (((f.pk >> 16) & 1u) << 8), ((f.pk >> 8) & 0xFFu) | (((f.pk >> 17) & 1u) << 8));
                 const bool nx = (int32_t)(i + 1) < (int32_t)f.size;
                 cur_rd[j] = nx ? f.nw.x : 0u; cur_rs1[j] = nx ? f.nw.y : 0u; cur_rs2[j] = nx ? f.nw.z : 0u;
-                if (KEEP) { f.ord = nx ? f.nw.x : 0u; f.rs1 = nx ? f.nw.y : 0u; f.rs2 = nx ? f.nw.z : 0u; }
             }
             if ((int32_t)(i + 1) < (int32_t)f.size) {
                 ra0_gather(d, f.nw.y, f.nw.z, g1[q], g2[q]);

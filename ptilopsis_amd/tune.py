@@ -3,8 +3,8 @@
     python -m ptilopsis_amd.tune [--out PATH]   (on the GPU; default ptilopsis_amd/tuning.json)
 
 Knobs (include/ptl.h, ptl_tune_set): the block size of each stage's per-node
-and per-word kernels (64, 128 or 256 threads), the walk_ring knob (without
-effect) and small_programs.  Buckets: a compile's node count below 64Ki, 1Mi,
+and per-word kernels (64, 128 or 256 threads), small_programs, and walk_ring, which
+has no effect and is not measured.  Buckets: a compile's node count below 64Ki, 1Mi,
 8Mi, or larger.  For each bucket a representative workload is compiled with
 each value of each knob in turn (the others at their current choice), and the
 value with the smallest device time of the stage the knob affects is kept
@@ -34,7 +34,7 @@ KNOBS = {
     "block.optimize": ((64, 128, 256), 256, 3),
     "block.emit": ((64, 128, 256), 256, 4),
     "block.fix_jumps": ((64, 128, 256), 256, 5),
-    "walk_ring": ((4, 8), 4, 4),  # without effect: the allocation walks keep their states in LDS
+    "walk_ring": ((4, 8), 4, None),  # without effect: the allocation walks keep their states in LDS
     # programs of at most 64 functions allocated by one wave each (1) or by the
     # walk and the lockstep (0)
     "small_programs": ((0, 1), 0, 4),
@@ -91,7 +91,6 @@ def main() -> int:
         2: ("program_4m", [W.sized_program(0x5EED0011, 4_000_000, 5000)]),
         3: ("large_16m", [W.large_16m()]),
     }
-    ring_work_3 = ("stress_1024", W.stress_1024())  # the walks bound this batch; in the one 17M-node program they hide behind the lockstep
     print(f"workloads generated in {time.time() - t0:.1f}s", file=sys.stderr, flush=True)
     ctx = Context(0)
     values = {k: [v[1]] * len(BUCKETS) for k, v in KNOBS.items()}
@@ -101,23 +100,19 @@ def main() -> int:
         ctx.upload_batch(1, trees)
         measured[BUCKETS[b]] = {}
         for knob, (allowed, default, stage) in KNOBS.items():
-            slot = 1
-            if knob == "walk_ring" and b == 3:
-                ctx.upload_batch(2, ring_work_3[1])
-                slot, wname = 2, ring_work_3[0]
-            else:
-                wname = name
+            if stage is None:
+                continue
             times = {}
             for v in allowed:
                 ctx.lib.ptl_tune_set(ctx.h, knob.encode(), b, v)
-                times[v] = _measure(ctx, slot, stage)
+                times[v] = _measure(ctx, 1, stage)
             best = min(times, key=times.get)
             choice = best if times[best] < 0.98 * times[default] else default
             values[knob][b] = choice
             ctx.lib.ptl_tune_set(ctx.h, knob.encode(), b, choice)
-            measured[BUCKETS[b]][knob] = {"workload": wname, "stage_ms": {str(k): round(v, 4) for k, v in times.items()},
+            measured[BUCKETS[b]][knob] = {"workload": name, "stage_ms": {str(k): round(v, 4) for k, v in times.items()},
                                           "choice": choice}
-            print(f"bucket {b} {knob:18s} {wname:12s} " +
+            print(f"bucket {b} {knob:18s} {name:12s} " +
                   " ".join(f"{k}:{v:.3f}ms" for k, v in times.items()) + f" -> {choice}", file=sys.stderr, flush=True)
     ctx.close()
     import torch
