@@ -360,7 +360,7 @@ def measure_serving(rates, seconds: float, pool_n: int, against_oracle: bool = F
                     time.sleep(0.00005)
                 tickets[i] = srv.submit_records(pool_rec[i % pool_n]) if records else srv.submit(pool[i % pool_n])
 
-        st0 = srv.stats()
+        st0, redos0 = srv.stats(), srv.redos()
         th = threading.Thread(target=submitter)
         tb = time.perf_counter()
         th.start()
@@ -384,7 +384,7 @@ def measure_serving(rates, seconds: float, pool_n: int, against_oracle: bool = F
             nodes += pool[i % pool_n].n
         th.join()
         el = time.perf_counter() - tb
-        st1 = srv.stats()
+        st1, redos = srv.stats(), srv.redos() - redos0
         nb = st1["batches"] - st0["batches"]
         for d in mism:
             d["batch_members"] = members.get(d["batch_id"], [])
@@ -392,13 +392,13 @@ def measure_serving(rates, seconds: float, pool_n: int, against_oracle: bool = F
         rec = {"rate_offered": rate, "input": "records" if records else "arrays", "requests": len(arr),
                "seconds": el, "rate_achieved": len(arr) / max(1e-9, float(arr[-1]) if len(arr) else 1.0),
                "p50_ms": pct(lat, 50), "p99_ms": pct(lat, 99), "nodes_per_s": nodes / el,
-               "batches": nb, "mean_batch": len(arr) / max(1, nb),
+               "batches": nb, "mean_batch": len(arr) / max(1, nb), "allocation_redos": redos,
                "breakdown_ms": {k[:-3]: {"p50": pct(v, 50), "p99": pct(v, 99)} for k, v in phases.items()},
                "same_as_alone": not mism, "mismatches": mism}
         b = rec["breakdown_ms"]
         log(f"serving {rate} req/s ({rec['input']}): p50 {rec['p50_ms']:.2f} ms, p99 {rec['p99_ms']:.2f} ms, "
             f"{rec['nodes_per_s'] / 1e6:.1f} M nodes/s, {nb} batches (mean {rec['mean_batch']:.1f}), "
-            f"mismatches: {len(mism)}; p50 queue {b['queue']['p50']:.2f} pack {b['pack']['p50']:.2f} "
+            f"mismatches: {len(mism)}, allocations redone: {redos}; p50 queue {b['queue']['p50']:.2f} pack {b['pack']['p50']:.2f} "
             f"run {b['run']['p50']:.2f} (device {b['device']['p50']:.2f}) copyout {b['copyout']['p50']:.2f} ms")
         return rec
 

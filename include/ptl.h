@@ -147,9 +147,9 @@ int ptl_compile_arena(ptl_ctx *ctx, const ptl_arena *in, ptl_result *out);
  * batches are on the device at once.  A request's device footprint is
  * estimated as 1 MiB + 384 B per node; one larger than the whole budget is
  * refused (PTL_ERR_ADMISSION).  hbm_budget_bytes 0 means 64 GiB.  Requests of
- * 256k nodes or more queue apart from smaller ones (even workers take small
- * requests first, odd workers large ones), so small requests do not wait
- * behind a large one's batch.
+ * 32k nodes or more queue apart from smaller ones, and a worker takes from the
+ * queue whose head has waited longer, so small requests do not wait behind a
+ * large one's batch.
  * ptl_server_submit copies the arrays and returns at once; ptl_server_wait
  * blocks until the request is done and fills out (valid until
  * ptl_server_release of that ticket) and, if given, its times.  Each result is
